@@ -10,7 +10,9 @@
 // the head entering K as ⌊h/rep⌋) with scalar factors and additive mask terms around it; the
 // value leaf an affine bf16 view.
 //
-// Kernel shape (one workgroup = one head × 128 query rows, 4 waves × 32 rows):
+// Any number of rows and keys with row-major V; whole tiles (rows % 128 = 0, keys % 64 = 0) with
+// V^T. Kernel shape (one workgroup = one head × 128 query rows, 4 waves × 32 rows; 64 rows, 4
+// waves × 16, for lengths off those tiles):
 //   S^T = K·Q^T per 64-key tile (so a lane owns one query column: the running max, the sum and
 //   the O rescale are lane-local, with one 4-lane shuffle per tile for the max);
 //   O^T += V^T·P^T with P packed to bf16 in registers (the MFMA k-order is chosen to match the
@@ -47,6 +49,7 @@ struct FlashPlan {
     // view: rendered per element once per workgroup, at coordinates qcoords over the vars
     // {0: head, 1: key, 2: d, 3: query row}
     bool qexpr = false;
+    bool ragged = false;      // rows not a multiple of 128 or keys not a multiple of 64
     int qnode = -1;
     std::vector<Sym> qcoords;
 };
@@ -148,6 +151,41 @@ bool find_flash_dot(const sanic_program_desc* d, int node, const std::vector<Sym
     return true;
 }
 
+// A window edge read off the first and last row of a block must not decrease with the query row
+// in between: values that do not move with the row, coordinates, sums of such edges, differences
+// from a row-free value and products with a constant that is not negative.
+std::vector<int> kid_bind(const sanic_program_desc* d, int node, int k, const std::vector<int>& b) {
+    const sanic_node& n = d->nodes[node];
+    const sanic_node& m = d->nodes[n.in[k]];
+    std::vector<int> cb(m.rank);
+    for (int j = 0; j < m.rank; j++) cb[j] = m.shape[j] == 1 ? SANIC_BIND_BCAST : b[n.rank - m.rank + j];
+    return cb;
+}
+
+bool row_free(const sanic_program_desc* d, int node, const std::vector<int>& b, int qdim) {
+    const sanic_node& n = d->nodes[node];
+    if (n.kind == SANIC_NODE_COORDINATE) return b[n.dim] != qdim;
+    if (n.kind == SANIC_NODE_MAP) {
+        for (int k = 0; k < n.n_in; k++) if (!row_free(d, n.in[k], kid_bind(d, node, k, b), qdim)) return false;
+        return true;
+    }
+    for (int j = 0; j < n.rank; j++) if (n.shape[j] != 1 && b[j] == qdim) return false;
+    return true;
+}
+
+bool rising_edge(const sanic_program_desc* d, int node, const std::vector<int>& b, int qdim) {
+    const sanic_node& n = d->nodes[node];
+    if (row_free(d, node, b, qdim) || n.kind == SANIC_NODE_IOTA || n.kind == SANIC_NODE_COORDINATE) return true;
+    if (n.kind != SANIC_NODE_MAP) return false;
+    auto up = [&](int k) { return rising_edge(d, n.in[k], kid_bind(d, node, k, b), qdim); };
+    if (n.op == SANIC_OP_ADD) return up(0) && up(1);
+    if (n.op == SANIC_OP_SUB) return up(0) && row_free(d, n.in[1], kid_bind(d, node, 1, b), qdim);
+    if (n.op == SANIC_OP_MUL)
+        for (int k = 0; k < 2; k++)
+            if (d->nodes[n.in[k]].kind == SANIC_NODE_CONST && d->nodes[n.in[k]].value >= 0.0) return up(1 - k);
+    return false;
+}
+
 bool flash_plan(const sanic_program_desc* d, int si, FlashPlan& P) {
     const sanic_stage& st = d->stages[si];
     if (st.kind != SANIC_STAGE_FUSED || st.n_leaves != 2) return false;
@@ -217,7 +255,8 @@ bool flash_plan(const sanic_program_desc* d, int si, FlashPlan& P) {
     }
     if (!sym_access(d, st.leaf[P.vleaf], vcs, {P.NH, P.T, P.E}, P.vacc)) return false;
     if ((!P.qexpr && P.qacc.dtype != SANIC_BF16) || P.kacc.dtype != SANIC_BF16 || P.vacc.dtype != SANIC_BF16) return false;
-    if (P.HD != 64 || P.E != 64 || P.NQ % 128 != 0 || P.T % 64 != 0) return false;
+    if (P.HD != 64 || P.E != 64) return false;
+    P.ragged = P.NQ % 128 != 0 || P.T % 64 != 0;
     // Q: (h, d, i) with d contiguous; K: (⌊h/rep⌋, t, d) with d contiguous; V: (⌊h/rep⌋, t, e)
     std::vector<int64_t> qc, kc, vc;
     int qh, kh, vh;
@@ -230,6 +269,20 @@ bool flash_plan(const sanic_program_desc* d, int si, FlashPlan& P) {
     int repv = vh ? vh : (vc[0] ? 1 : (int)P.NH);
     if (repk != repv) return false;
     P.rep = repk;
+    // the block's and the wave's key ranges are read off their first and last rows: every edge
+    // must not decrease with the row
+    for (auto& w : honest_window(d, st))
+        if (!rising_edge(d, w.node, w.bind, P.qdim)) return false;
+    if (P.ragged) {
+        // Lengths off the tiles go here only where the schedule is the backend's to choose and
+        // the tile rows are whole 16-byte chunks of row-major K and V
+        if (!sched_is_auto(st.sched) || vc[2] != 1) return false;
+        for (int64_t v : {kc[0], kc[1], khc, P.kacc.addr.c0, vc[0], vc[1], vhc, P.vacc.addr.c0})
+            if (v % 8) return false;
+        if (!P.qexpr)
+            for (int64_t v : {qc[0], qc[3], P.qacc.addr.c0})
+                if (v % 8) return false;
+    }
     return true;
 }
 
@@ -267,7 +320,22 @@ bool lower_flash_prefill(const sanic_program_desc* d, int si, int64_t& scratch, 
     const sanic_stage& st = d->stages[si];
     const sanic_carrier& c = st.carrier;
     const int64_t NH = P.NH, NQ = P.NQ, T = P.T, E = P.E, HD = P.HD;
-    const int64_t NQB = NQ / 128;
+    // Lengths off the tiles (a prompt nobody padded) were folded in f32 by the generic fold: here
+    // the softmax weights, and a query side that is an expression, go to the MFMA as hi + lo bf16
+    // pairs (16 significant bits), so they keep that precision at two MFMAs per fragment; one
+    // query tile per wave holds the second operands in the registers the second tile had (115
+    // VGPRs) and gives short prompts twice the workgroups. 32/8 heads, S = 1000, window 256, with
+    // the RoPE stages: 20.0 ms in the generic fold (it forms q·k again for each of the 64 value
+    // columns) → 23.3 µs, the same 2.2e-3 from a 64-bit evaluation.
+    const bool hilo = P.ragged;
+    const int fvar = P.ragged ? 0 : d->stages[si].sched.variant;
+    const int QT = P.ragged ? 1 : 2;                 // 16-row query tiles per wave
+    const int RB = 64 * QT;                          // query rows per workgroup (4 waves)
+    const int64_t NQB = (NQ + RB - 1) / RB;
+    const std::string QTs = std::to_string(QT), RBs = std::to_string(RB);
+    // the last row or key of the operands, where a tile runs past it
+    auto row_clamp = [&](const std::string& r) { return P.ragged ? "sanic_min(" + r + ", (idx_t)" + std::to_string(NQ - 1) + ")" : "(" + r + ")"; };
+    auto key_clamp = [&](const std::string& r) { return P.ragged ? "sanic_min(" + r + ", (idx_t)" + std::to_string(T - 1) + ")" : "(" + r + ")"; };
     std::vector<int64_t> qc, kc, vc;
     int qh, kh, vh;
     int64_t qhc, khc, vhc;
@@ -369,13 +437,17 @@ bool lower_flash_prefill(const sanic_program_desc* d, int si, int64_t& scratch, 
     // of the block's key tiles; they exchange their (m, ℓ, o) partials through scratch and the
     // second to arrive combines them (the carrier's ExpShifted combine with its −∞ guard) and
     // projects. It evens out launches whose equal-sized blocks overfill the resident slots.
-    const int fvar = d->stages[si].sched.variant;
     int SPL = fvar == 2 ? 2 : 1;
     src << (SPL > 1 ? R.args_struct({"float* __restrict__ scratch"}) : R.args_struct({}));
     src << "typedef __bf16 sanic_bf16x2 __attribute__((ext_vector_type(2)));\n";
     src << "typedef float sanic_f32x2 __attribute__((ext_vector_type(2)));\n";
     src << "__device__ __forceinline__ unsigned pk_bf16(float x, float y) {\n"
            "  return __builtin_bit_cast(unsigned, __builtin_convertvector((sanic_f32x2){x, y}, sanic_bf16x2));\n}\n";
+    src << "__device__ __forceinline__ idx_t sanic_min(idx_t a, idx_t b) { return a < b ? a : b; }\n";
+    src << "__device__ __forceinline__ void split_bf16(float x, float y, unsigned& hi, unsigned& lo) {\n"
+           "  const unsigned h = pk_bf16(x, y);\n"
+           "  hi = h;\n"
+           "  lo = pk_bf16(x - __uint_as_float(h << 16), y - __uint_as_float(h & 0xFFFF0000u));\n}\n";
     // max across the 4 lane groups of a query column (lanes l, l^16, l^32, l^48): gfx950
     // permlane swaps, no LDS round trip
     // compiler-visible maxima: the compiler forms v_max3_f32 itself and, unlike for inline asm
@@ -445,13 +517,13 @@ bool lower_flash_prefill(const sanic_program_desc* d, int si, int64_t& scratch, 
         k.line("const idx_t hh = bid % " + std::to_string(NH) + ";");
         k.line("const idx_t qb = " + std::to_string(NQB - 1) + " - bid / " + std::to_string(NH) + ";");
     }
-    k.line("const idx_t q0 = qb * 128 + wv * 32;");   // this wave's 32 query rows
+    k.line("const idx_t q0 = qb * " + RBs + " + wv * " + std::to_string(16 * QT) + ";");   // this wave's query rows
     // block and wave key ranges from the honest window of the first and last rows
     k.line("idx_t blo_a, bhi_a, blo_b, bhi_b, wlo_a, whi_a, wlo_b, whi_b;");
-    k.line("window(a, hh, qb * 128, blo_a, bhi_a);");
-    k.line("window(a, hh, qb * 128 + 127, blo_b, bhi_b);");
-    k.line("window(a, hh, q0, wlo_a, whi_a);");
-    k.line("window(a, hh, q0 + 31, wlo_b, whi_b);");
+    k.line("window(a, hh, qb * " + RBs + ", blo_a, bhi_a);");
+    k.line("window(a, hh, " + row_clamp("qb * " + RBs + " + " + std::to_string(RB - 1)) + ", blo_b, bhi_b);");
+    k.line("window(a, hh, " + row_clamp("q0") + ", wlo_a, whi_a);");
+    k.line("window(a, hh, " + row_clamp("q0 + " + std::to_string(16 * QT - 1)) + ", wlo_b, whi_b);");
     if (SPL > 1) {
         k.line("const idx_t klo0 = (blo_a < blo_b ? blo_a : blo_b) / 64 * 64;");
         k.line("const idx_t khi0 = bhi_a > bhi_b ? bhi_a : bhi_b;");
@@ -463,7 +535,16 @@ bool lower_flash_prefill(const sanic_program_desc* d, int si, int64_t& scratch, 
         k.line("const idx_t khi = bhi_a > bhi_b ? bhi_a : bhi_b;");
     }
     k.line("const idx_t wlo = wlo_a < wlo_b ? wlo_a : wlo_b, whi = whi_a > whi_b ? whi_a : whi_b;");
-    k.line("const idx_t flo = wlo_a > wlo_b ? wlo_a : wlo_b, fhi = whi_a < whi_b ? whi_a : whi_b;");
+    k.line("const idx_t flo = wlo_a > wlo_b ? wlo_a : wlo_b;");
+    // (a first or last row with no visible key stands for the whole stream and says nothing of
+    // the rows between: no tile is then full)
+    if (raw_ok) {
+        k.line("idx_t re_lo, re_hi;");
+        k.line("const bool wne = window_raw(a, hh, " + row_clamp("q0") + ", re_lo, re_hi) & window_raw(a, hh, " + row_clamp("q0 + " + std::to_string(16 * QT - 1)) + ", re_lo, re_hi);");
+        k.line("const idx_t fhi = !wne ? 0 : whi_a < whi_b ? whi_a : whi_b;");
+    } else {
+        k.line("const idx_t fhi = whi_a < whi_b ? whi_a : whi_b;");
+    }
     // the bounds are wave-uniform (they depend on the block and wave only): held in scalar
     // registers, the key loop's control and the tile classification run on the scalar unit
     k.line("const int klo_s = __builtin_amdgcn_readfirstlane((int)klo), khi_s = __builtin_amdgcn_readfirstlane((int)khi);");
@@ -484,14 +565,18 @@ bool lower_flash_prefill(const sanic_program_desc* d, int si, int64_t& scratch, 
     const bool edge_on = raw_ok && fvar != 3;
     // Q^T as the B operand (lane = query column l16 (+16·qt), d-slots lq·8 + 0..7 (+32·ds)),
     // held in registers for the whole key loop, loaded once from global memory
-    k.line("bf16x8 qf[2][2];");
+    k.line("bf16x8 qf[" + QTs + "][2];");
+    const bool qlo = hilo && P.qexpr;
+    if (qlo) k.line("bf16x8 ql[" + QTs + "][2];");
+    for (int qt = 0; qt < QT; qt++)
+        k.line("const idx_t qr" + std::to_string(qt) + " = " + row_clamp("q0 + " + std::to_string(qt * 16) + " + l16") + ";");
     if (!P.qexpr) {
         k.line("#pragma unroll");
-        k.line("for (int qt = 0; qt < 2; ++qt)");
+        k.line("for (int qt = 0; qt < " + QTs + "; ++qt)");
         k.line("  #pragma unroll");
         k.line("  for (int ds = 0; ds < 2; ++ds)");
         k.line("    qf[qt][ds] = *(const bf16x8*)(" + qp + " + " + std::to_string(P.qacc.addr.c0) + " + " + hterm(qc, qh, qhc) +
-               " + (q0 + qt * 16 + l16) * " + std::to_string(qc[3]) + " + (ds * 4 + lq) * 8);");
+               " + " + row_clamp("q0 + qt * 16 + l16") + " * " + std::to_string(qc[3]) + " + (ds * 4 + lq) * 8);");
     }
     // An expression query side is rendered element by element (the lane's 2 × 16 values), once
     // per workgroup, after the first K/V transfers are requested so its loads and arithmetic
@@ -505,11 +590,11 @@ bool lower_flash_prefill(const sanic_program_desc* d, int si, int64_t& scratch, 
     if (P.qexpr) {
         q_lc.indent = q_dc.indent = k.indent + 1;
         bool ok = true;
-        for (int qt = 0; qt < 2 && ok; qt++)
+        for (int qt = 0; qt < QT && ok; qt++)
             for (int ds = 0; ds < 2 && ok; ds++) {
                 const std::string sfx = "_q" + std::to_string(qt) + std::to_string(ds);
                 const std::vector<std::string> vars = {"hh", "(idx_t)0", "((idx_t)lq * 8 + " + std::to_string(ds * 32) + ")",
-                                                       "(q0 + " + std::to_string(qt * 16) + " + l16)"};
+                                                       "qr" + std::to_string(qt)};
                 std::vector<int> bufs, dts;
                 q_vals[qt][ds] = render_run(d, P.qnode, P.qcoords, {NH, T, HD, NQ}, vars, 2, q_lc, q_dc, sfx, bufs, dts, ok);
                 for (size_t b = 0; b < bufs.size() && ok; b++)
@@ -520,20 +605,31 @@ bool lower_flash_prefill(const sanic_program_desc* d, int si, int64_t& scratch, 
         if (q_runs) k.s << q_lc.str();
     }
     auto emit_qexpr = [&]() {
+        auto q_split = [&](int qt, int ds, const std::string* v) {
+            k.line("{");
+            k.line("  sanic_u32x4 h_, l_;");
+            for (int q = 0; q < 4; q++)
+                k.line("  { unsigned h1, l1; split_bf16(" + v[2 * q] + ", " + v[2 * q + 1] + ", h1, l1); h_[" + std::to_string(q) + "] = h1; l_[" + std::to_string(q) + "] = l1; }");
+            const std::string ix = "[" + std::to_string(qt) + "][" + std::to_string(ds) + "]";
+            k.line("  qf" + ix + " = __builtin_bit_cast(bf16x8, h_);");
+            k.line("  ql" + ix + " = __builtin_bit_cast(bf16x8, l_);");
+            k.line("}");
+        };
         if (q_runs) {
             k.s << q_dc.str();
-            for (int qt = 0; qt < 2; qt++)
+            for (int qt = 0; qt < QT; qt++)
                 for (int ds = 0; ds < 2; ds++) {
                     const auto& v = q_vals[qt][ds];
+                    if (qlo) { q_split(qt, ds, v.data()); continue; }
                     k.line("qf[" + std::to_string(qt) + "][" + std::to_string(ds) + "] = __builtin_bit_cast(bf16x8, (sanic_u32x4){pk_bf16(" + v[0] + ", " + v[1] +
                            "), pk_bf16(" + v[2] + ", " + v[3] + "), pk_bf16(" + v[4] + ", " + v[5] + "), pk_bf16(" + v[6] + ", " + v[7] + ")});");
                 }
             return;
         }
-        for (int qt = 0; qt < 2; qt++) {
+        for (int qt = 0; qt < QT; qt++) {
             k.line("{");
             k.indent++;
-            k.line("const idx_t qrow = q0 + " + std::to_string(qt * 16) + " + l16;");
+            k.line("const idx_t qrow = qr" + std::to_string(qt) + ";");
             R.memo.emplace_back();
             std::string vals[2][8];
             for (int ds = 0; ds < 2; ds++)
@@ -545,6 +641,7 @@ bool lower_flash_prefill(const sanic_program_desc* d, int si, int64_t& scratch, 
                 }
             R.memo.pop_back();
             for (int ds = 0; ds < 2; ds++) {
+                if (qlo) { q_split(qt, ds, vals[ds]); continue; }
                 std::string pk = "(sanic_u32x4){";
                 for (int q = 0; q < 4; q++)
                     pk += std::string(q ? ", " : "") + "pk_bf16(" + vals[ds][2 * q] + ", " + vals[ds][2 * q + 1] + ")";
@@ -554,12 +651,16 @@ bool lower_flash_prefill(const sanic_program_desc* d, int si, int64_t& scratch, 
             k.line("}");
         }
     };
-    k.line("f32x4 o[4][2];");
+    k.line("f32x4 o[4][" + QTs + "];");
     k.line("#pragma unroll");
-    k.line("for (int dt = 0; dt < 4; ++dt) { o[dt][0] = (f32x4){0, 0, 0, 0}; o[dt][1] = (f32x4){0, 0, 0, 0}; }");
-    k.line("float m_run[2] = {-__builtin_huge_valf(), -__builtin_huge_valf()};");
+    k.line("for (int dt = 0; dt < 4; ++dt)");
+    k.line("  #pragma unroll");
+    k.line("  for (int qt = 0; qt < " + QTs + "; ++qt) o[dt][qt] = (f32x4){0, 0, 0, 0};");
+    k.line("float m_run[" + QTs + "];");
     // row sums ℓ accumulate on the matrix cores: a row of ones times P^T (same bf16 P as O)
-    k.line("f32x4 lsum[2] = {(f32x4){0, 0, 0, 0}, (f32x4){0, 0, 0, 0}};");
+    k.line("f32x4 lsum[" + QTs + "];");
+    k.line("#pragma unroll");
+    k.line("for (int qt = 0; qt < " + QTs + "; ++qt) { m_run[qt] = -__builtin_huge_valf(); lsum[qt] = (f32x4){0, 0, 0, 0}; }");
     k.line("const bf16x8 ones = {0x3F80, 0x3F80, 0x3F80, 0x3F80, 0x3F80, 0x3F80, 0x3F80, 0x3F80};");
     const double LOG2E = 1.4426950408889634;
     // Lazy reference max: the running max moves only when a tile's max exceeds it by more than
@@ -581,14 +682,30 @@ bool lower_flash_prefill(const sanic_program_desc* d, int si, int64_t& scratch, 
     // Four transfers per lane per tile, counted by vmcnt like any global load.
     std::string kbase = std::to_string(P.kacc.addr.c0) + " + " + hterm(kc, kh, khc);
     std::string vbase = std::to_string(P.vacc.addr.c0) + " + " + hterm(vc, vh, vhc);
+    const std::string krow = key_clamp("tt + r"), vsrc = v_rows ? krow + " * " + std::to_string(vc[1]) + " + c * 8"
+                                                                 : "(idx_t)r * " + std::to_string(vc[2]) + " + tt + c * 8";
+    // The direct transfer moves aligned 16-byte chunks; a caller may bind K or V at any element,
+    // and the lengths that come here from the generic fold keep taking such a binding: its chunks
+    // pass through registers, complete in LDS before the barrier that publishes the tile.
+    if (P.ragged) k.line("const bool chunks = (((size_t)(" + kp + ") | (size_t)(" + vp + ")) & 15) == 0;");
     k.line("auto fetch = [&](idx_t tt, int b) {");
     k.line("  #pragma unroll");
     k.line("  for (int u = 0; u < 2; ++u) {");
     k.line("    const int r = 8 * (wv + 4 * u) + (lane >> 3), c = (lane & 7) ^ (lane >> 3);");
-    k.line("    __builtin_amdgcn_global_load_lds((const __attribute__((address_space(1))) void*)(" + kp + " + " + kbase + " + (tt + r) * " +
+    if (P.ragged) {
+        k.line("    if (!chunks) {");
+        k.line("      const unsigned short* kq = " + kp + " + " + kbase + " + " + krow + " * " + std::to_string(kc[1]) + " + c * 8;");
+        k.line("      const unsigned short* vq = " + vp + " + " + vbase + " + " + vsrc + ";");
+        k.line("      for (int i = 0; i < 8; ++i) {");
+        k.line("        kv_lds[b][0][(wv + 4 * u) * 512 + lane * 8 + i] = kq[i];");
+        k.line("        kv_lds[b][1][(wv + 4 * u) * 512 + lane * 8 + i] = vq[i];");
+        k.line("      }");
+        k.line("      asm volatile(\"s_waitcnt lgkmcnt(0)\" ::: \"memory\");");
+        k.line("      continue;");
+        k.line("    }");
+    }
+    k.line("    __builtin_amdgcn_global_load_lds((const __attribute__((address_space(1))) void*)(" + kp + " + " + kbase + " + " + krow + " * " +
            std::to_string(kc[1]) + " + c * 8), (__attribute__((address_space(3))) void*)(&kv_lds[b][0][(wv + 4 * u) * 512]), 16, 0, 0);");
-    const std::string vsrc = v_rows ? "(tt + r) * " + std::to_string(vc[1]) + " + c * 8"
-                                    : "(idx_t)r * " + std::to_string(vc[2]) + " + tt + c * 8";
     k.line("    __builtin_amdgcn_global_load_lds((const __attribute__((address_space(1))) void*)(" + vp + " + " + vbase + " + " + vsrc +
            "), (__attribute__((address_space(3))) void*)(&kv_lds[b][1][(wv + 4 * u) * 512]), 16, 0, 0);");
     k.line("  }");
@@ -620,9 +737,10 @@ bool lower_flash_prefill(const sanic_program_desc* d, int si, int64_t& scratch, 
     // The split variant and the rendered-mask reference variant keep one query tile's scores
     // live at a time (with both live they spill 12–13 registers); the products are the same
     // MFMAs in the same order either way.
-    const bool s_both = SPL == 1 && fvar != 3;
-    k.line("f32x4 s[4][2];");
-    k.line("sanic_u32x4 pw[2][2];");
+    const bool s_both = QT == 2 && SPL == 1 && fvar != 3;
+    k.line("f32x4 s[4][" + QTs + "];");
+    k.line("sanic_u32x4 pw[" + QTs + "][2];");
+    if (hilo) k.line("sanic_u32x4 pl[" + QTs + "][2];");
     auto scores = [&](bool both) {
         k.line("#pragma unroll");
         k.line("for (int kt = 0; kt < 4; ++kt) {");
@@ -638,6 +756,7 @@ bool lower_flash_prefill(const sanic_program_desc* d, int si, int64_t& scratch, 
             k.line("    {");
         }
         k.line("      s[kt][qt] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(ka, qf[qt][ds], s[kt][qt], 0, 0, 0);");
+        if (qlo) k.line("      s[kt][qt] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(ka, ql[qt][ds], s[kt][qt], 0, 0, 0);");
         k.line("    }");
         k.line("  }");
         k.line("}");
@@ -645,10 +764,10 @@ bool lower_flash_prefill(const sanic_program_desc* d, int si, int64_t& scratch, 
     if (s_both) scores(true);
     // online softmax per query column (lane-local; the max reduces across the 4 lane groups)
     k.line("#pragma unroll");
-    k.line("for (int qt = 0; qt < 2; ++qt) {");
+    k.line("for (int qt = 0; qt < " + QTs + "; ++qt) {");
     k.indent++;
     if (!s_both) scores(false);
-    k.line("const int qi = (int)(q0 + qt * 16 + l16);");
+    k.line("const int qi = (int)" + row_clamp("(q0 + qt * 16 + l16)") + ";");
     k.line("float sv[16];");
     k.line("float p[16];");
     k.line("float mn, alpha;");
@@ -722,14 +841,23 @@ bool lower_flash_prefill(const sanic_program_desc* d, int si, int64_t& scratch, 
     k.line("    #pragma unroll");
     k.line("    for (int r = 0; r < 4; ++r) {");
     k.line("      const int kj = kb + kt * 16 + r;");
-    k.line("      const float sf = score_full(a, s[kt][qt][r], (int)hh, qi, kj);");
+    k.line("      const float sf = score_full(a, s[kt][qt][r], (int)hh, qi, " + std::string(P.ragged ? "kj < " + std::to_string(T) + " ? kj : " + std::to_string(T - 1) : "kj") + ");");
     k.line("      sv[kt * 4 + r] = kj >= elo && kj < ehi ? sf : -1e30f;");
     k.line("    }");
     k.line("} else {");
     k.line("  #pragma unroll");
     k.line("  for (int kt = 0; kt < 4; ++kt)");
     k.line("    #pragma unroll");
-    k.line("    for (int r = 0; r < 4; ++r) sv[kt * 4 + r] = score_part(a, s[kt][qt][r], (int)hh, qi, kb + kt * 16 + r);");
+    if (P.ragged) {
+        // keys past the last weigh nothing
+        k.line("    for (int r = 0; r < 4; ++r) {");
+        k.line("      const int kj = kb + kt * 16 + r;");
+        k.line("      const float sp = score_part(a, s[kt][qt][r], (int)hh, qi, kj < " + std::to_string(T) + " ? kj : " + std::to_string(T - 1) + ");");
+        k.line("      sv[kt * 4 + r] = kj < " + std::to_string(T) + " ? sp : -__builtin_huge_valf();");
+        k.line("    }");
+    } else {
+        k.line("    for (int r = 0; r < 4; ++r) sv[kt * 4 + r] = score_part(a, s[kt][qt][r], (int)hh, qi, kb + kt * 16 + r);");
+    }
     k.line("}");
     k.line("float mt = fmaxf(fmaxf(sv[0], sv[1]), fmaxf(sv[2], sv[3]));");
     k.line("#pragma unroll");
@@ -761,21 +889,31 @@ bool lower_flash_prefill(const sanic_program_desc* d, int si, int64_t& scratch, 
     // slots 4..7 = keys 32ks + 16 + lq·4 + r (tile 2ks+1); two slots per dword, RNE in hardware
     k.line("#pragma unroll");
     k.line("for (int ks = 0; ks < 2; ++ks) {");
-    k.line("  pw[qt][ks].x = pk_bf16(p[8 * ks + 0], p[8 * ks + 1]);");
-    k.line("  pw[qt][ks].y = pk_bf16(p[8 * ks + 2], p[8 * ks + 3]);");
-    k.line("  pw[qt][ks].z = pk_bf16(p[8 * ks + 4], p[8 * ks + 5]);");
-    k.line("  pw[qt][ks].w = pk_bf16(p[8 * ks + 6], p[8 * ks + 7]);");
+    const char* comp[4] = {"x", "y", "z", "w"};
+    for (int q = 0; q < 4; q++) {
+        const std::string pp = "p[8 * ks + " + std::to_string(2 * q) + "], p[8 * ks + " + std::to_string(2 * q + 1) + "]";
+        if (hilo) k.line("  { unsigned h1, l1; split_bf16(" + pp + ", h1, l1); pw[qt][ks]." + comp[q] + " = h1; pl[qt][ks]." + comp[q] + " = l1; }");
+        else k.line("  pw[qt][ks]." + std::string(comp[q]) + " = pk_bf16(" + pp + ");");
+    }
     k.line("}");
     k.indent--;
     k.line("}");
-    k.line("bf16x8 pf[2][2];");
+    k.line("bf16x8 pf[" + QTs + "][2];");
     k.line("#pragma unroll");
-    k.line("for (int qt = 0; qt < 2; ++qt) { pf[qt][0] = __builtin_bit_cast(bf16x8, pw[qt][0]); pf[qt][1] = __builtin_bit_cast(bf16x8, pw[qt][1]); }");
+    k.line("for (int qt = 0; qt < " + QTs + "; ++qt) { pf[qt][0] = __builtin_bit_cast(bf16x8, pw[qt][0]); pf[qt][1] = __builtin_bit_cast(bf16x8, pw[qt][1]); }");
+    if (hilo) {
+        k.line("bf16x8 pfl[" + QTs + "][2];");
+        k.line("#pragma unroll");
+        k.line("for (int qt = 0; qt < " + QTs + "; ++qt) { pfl[qt][0] = __builtin_bit_cast(bf16x8, pl[qt][0]); pfl[qt][1] = __builtin_bit_cast(bf16x8, pl[qt][1]); }");
+    }
     // O^T += V^T · P^T ; V^T A operand: row e = dt·16 + l16, keys in the same slot order
     k.line("#pragma unroll");
     k.line("for (int ks = 0; ks < 2; ++ks) {");
-    k.line("  lsum[0] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(ones, pf[0][ks], lsum[0], 0, 0, 0);");
-    k.line("  lsum[1] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(ones, pf[1][ks], lsum[1], 0, 0, 0);");
+    for (int qt = 0; qt < QT; qt++)
+        for (int h = 0; h < (hilo ? 2 : 1); h++) {
+            const std::string q = std::to_string(qt);
+            k.line("  lsum[" + q + "] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(ones, " + (h ? "pfl[" : "pf[") + q + "][ks], lsum[" + q + "], 0, 0, 0);");
+        }
     k.line("}");
     if (v_rows) {
         // V rows in LDS, read transposed (ds_read_b64_tr_b16): in each 16-lane group, source
@@ -812,8 +950,11 @@ bool lower_flash_prefill(const sanic_program_desc* d, int si, int64_t& scratch, 
                 for (int ks = 0; ks < 2; ks++) {
                     const std::string ix = "[" + std::to_string(dt) + "][" + std::to_string(ks) + "]";
                     const std::string va = "__builtin_bit_cast(bf16x8, (sanic_s16x8)__builtin_shufflevector(vt" + ix + "[0], vt" + ix + "[1], 0, 1, 2, 3, 4, 5, 6, 7))";
-                    k.line("o[" + std::to_string(dt) + "][0] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(" + va + ", pf[0][" + std::to_string(ks) + "], o[" + std::to_string(dt) + "][0], 0, 0, 0);");
-                    k.line("o[" + std::to_string(dt) + "][1] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(" + va + ", pf[1][" + std::to_string(ks) + "], o[" + std::to_string(dt) + "][1], 0, 0, 0);");
+                    for (int qt = 0; qt < QT; qt++)
+                        for (int h = 0; h < (hilo ? 2 : 1); h++) {
+                            const std::string ov = "o[" + std::to_string(dt) + "][" + std::to_string(qt) + "]";
+                            k.line(ov + " = __builtin_amdgcn_mfma_f32_16x16x32_bf16(" + va + ", " + (h ? "pfl[" : "pf[") + std::to_string(qt) + "][" + std::to_string(ks) + "], " + ov + ", 0, 0, 0);");
+                        }
                 }
         };
         vreads(0);
@@ -893,10 +1034,11 @@ bool lower_flash_prefill(const sanic_program_desc* d, int si, int64_t& scratch, 
     }
     // finish: the row sum across the 4 lane groups, then project per output point
     k.line("#pragma unroll");
-    k.line("for (int qt = 0; qt < 2; ++qt) {");
+    k.line("for (int qt = 0; qt < " + QTs + "; ++qt) {");
     k.indent++;
     k.line("const float lt = lsum[qt][0];");
     k.line("const idx_t qi = q0 + qt * 16 + l16;");
+    if (P.ragged) k.line("if (qi >= " + std::to_string(NQ) + ") continue;");
     k.line("#pragma unroll");
     k.line("for (int dt = 0; dt < 4; ++dt)");
     k.line("  #pragma unroll");
@@ -914,11 +1056,11 @@ bool lower_flash_prefill(const sanic_program_desc* d, int si, int64_t& scratch, 
     // three waves per SIMD: the softmax of one wave overlaps the MFMAs of the others (the
     // register cap costs a few spilled values outside the inner loop)
     // tiling variants for the measured tuner: workgroups per CU {3, 2}
-    int occ = d->stages[si].sched.variant == 1 ? 2 : 3;
+    int occ = fvar == 1 ? 2 : 3;
     src << "extern \"C\" __global__ void __launch_bounds__(256, " << occ << ") " << kname << "(Args a) {\n" << R.entry() << k.str() << "}\n";
-    out.kernel_kind = "skeleton:flash_prefill[rep " + std::to_string(P.rep) + "]" + (SPL > 1 ? "+split2" : "");
+    out.kernel_kind = "skeleton:flash_prefill[rep " + std::to_string(P.rep) + (P.ragged ? ",any length" : "") + "]" + (SPL > 1 ? "+split2" : "");
     out.source = src.str();
-    out.variants = 4;
+    out.variants = P.ragged ? 1 : 4;
     std::vector<Arg> args = R.arg_list();
     if (SPL > 1) args.push_back({Arg::SCRATCH, soff});
     out.launches.push_back({kname, "", dim3((unsigned)(NB * SPL)), dim3(256), 0, args});

@@ -101,3 +101,36 @@ def test_flash_head_groupings(dev, NH, NKV):
     err = max_rel_err(got["O"], want)
     print(NH, NKV, err, floored_rel_err(got["O"], want))
     assert err < 2e-2
+
+
+@pytest.mark.parametrize("NH,NKV,S,window", [
+    (4, 2, 40, 0),        # one query block, one key tile, both partly past the end
+    (8, 8, 63, 0),
+    (4, 2, 129, 0),       # one row into a third block, one key into a third tile
+    (4, 2, 200, 100),     # a window ending inside a tile
+    (2, 1, 321, 70),
+    (6, 2, 512 + 64, 0),  # whole key tiles, rows not a multiple of 128
+])
+def test_flash_any_length(dev, monkeypatch, NH, NKV, S, window):
+    """Lengths off the tiles against the generic f32 fold of the same program: the skeleton keeps
+    q and the softmax weights to 16 significant bits (hi + lo), so the two differ by no more than
+    the bf16 store of values 2^-16 · Σ p|v| ≤ 1e-4 apart — at most one bf16 step beside that.
+    Once more with K and V bound one element off a 16-byte boundary: the same bits."""
+    prog = configs.flash_prefill(NH, NKV, S, window=window)
+    vals = _inputs(NH, NKV, S, seed=470 + S)
+    got, exe = run_on_gpu(dev, prog, vals)
+    assert exe.stage_kernel(2).startswith("skeleton:flash_prefill"), exe.stage_kernel(2)
+    bufs = {n: dev.from_values(v, ir.BF16) for n, v in vals.items()}
+    for n in ("K", "V"):
+        raw = bufs[n].download()
+        hold = dev.alloc(len(raw) + 16)
+        hold.upload(b"\0\0" + raw + b"\0\0")
+        bufs[n + "hold"], bufs[n] = hold, dev.wrap(hold.device_ptr + 2, len(raw))
+    off = exe.execute({n: bufs[n] for n in ("Q", "K", "V")})["O"].read(ir.BF16, NH * S * 64).reshape(NH, S, 64)
+    assert np.array_equal(off, got["O"])
+    monkeypatch.setenv("SANIC_HIP_GENERIC", "1")
+    want, exe = run_on_gpu(dev, prog, vals)
+    assert exe.stage_kernel(2).startswith("fold:"), exe.stage_kernel(2)
+    over = np.abs(got["O"] - want["O"]) - 2.0 ** -7 * np.abs(want["O"])
+    print(S, window, float(over.max()), max_rel_err(got["O"], want["O"]))
+    assert over.max() < 1e-4
