@@ -65,6 +65,9 @@ std::vector<WindowBound> honest_window(const sanic_program_desc* d, const sanic_
 void emit_window(Renderer& R, Code& code, const sanic_stage& st, const std::vector<WindowBound>& w,
                  const std::string& lo, const std::string& hi);
 int64_t dtype_bytes(int dt, int64_t n);
+// Fold the whole stream at grid point g0, g1, ... one element after another (the scalar generic
+// fold's arithmetic); slot k's accumulator is `acc`<k>.
+void emit_point_fold(Renderer& R, Code& code, const sanic_stage& st, const std::string& acc);
 // Last-arriver handshake: the workgroups sharing counter `cnt` each add 1 once their partials
 // are stored; `flag` (a __shared__ int it declares) is true in the one that arrives last.
 // With xcd_local every workgroup sharing `cnt` runs on one XCD and exchanges data through

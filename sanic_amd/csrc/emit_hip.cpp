@@ -954,7 +954,7 @@ void emit_window(Renderer& R, Code& code, const sanic_stage& st, const std::vect
 
 // ───────────────────────────── generic fold ───────────────────────────────────────────────
 
-static void emit_fold_body(Renderer& R, Code& code, const sanic_stage& st, const std::string& s) {
+static void emit_fold_body(Renderer& R, Code& code, const sanic_stage& st, const std::string& s, const std::string& acc = "acc") {
     const sanic_carrier& c = st.carrier;
     R.memo.emplace_back();
     for (int l = 0; l < st.n_leaves; l++) {
@@ -966,10 +966,25 @@ static void emit_fold_body(Renderer& R, Code& code, const sanic_stage& st, const
         code.line("const float el" + std::to_string(k) + " = " + v + ";");
     }
     for (int k = 0; k < c.slots; k++) {
-        std::string v = R.expr(code, c.combine[k], "", "acc", "el", "");
+        std::string v = R.expr(code, c.combine[k], "", acc, "el", "");
         code.line("const float nx" + std::to_string(k) + " = " + v + ";");
     }
-    for (int k = 0; k < c.slots; k++) code.line("acc" + std::to_string(k) + " = nx" + std::to_string(k) + ";");
+    for (int k = 0; k < c.slots; k++) code.line(acc + std::to_string(k) + " = nx" + std::to_string(k) + ";");
+    R.memo.pop_back();
+}
+
+void emit_point_fold(Renderer& R, Code& code, const sanic_stage& st, const std::string& acc) {
+    const sanic_carrier& c = st.carrier;
+    for (int k = 0; k < c.slots; k++) code.line("float " + acc + std::to_string(k) + " = " + flit(c.identity[k]) + ";");
+    auto win = honest_window(R.d, st);
+    R.memo.emplace_back();
+    emit_window(R, code, st, win, "pf_lo", "pf_hi");
+    code.line("#pragma nounroll");
+    code.line("for (idx_t s = pf_lo; s < pf_hi; ++s) {");
+    code.indent++;
+    emit_fold_body(R, code, st, "s", acc);
+    code.indent--;
+    code.line("}");
     R.memo.pop_back();
 }
 

@@ -76,7 +76,7 @@ bool gemm_plan(const sanic_program_desc* d, int si, GemmPlan& P) {
         if (c.kind[k].kind != SANIC_SLOT_PLAIN || c.kind[k].monoid != SANIC_MON_ADD) return false;
     std::vector<int> big;
     for (int j = 0; j < st.rank; j++) if (st.grid[j] > 1) big.push_back(j);
-    if (big.size() != 2 || st.stream % 64) return false;
+    if (big.size() != 2 || st.stream % 8 || st.stream < 64) return false;
     P = GemmPlan();
     P.K = st.stream;
     // leaves bound to a big grid dim (plus the stream); the rest depend on the stream only
@@ -149,8 +149,20 @@ bool gemm_plan(const sanic_program_desc* d, int si, GemmPlan& P) {
     P.M = st.grid[P.mdim];
     P.N = st.grid[P.ndim];
     if (P.cslots.size() != 1) return false;
-    if (P.M < 64 || P.M % 64 || P.N % 32) return false;
     return true;
+}
+
+// The contraction slot's factor beside the weight is a stored bf16 value or the product of two:
+// at most 16 significant bits, so hi + lo bf16 hold it exactly.
+bool exact_in_two(const sanic_program_desc* d, const sanic_stage& st, int e, int w, int& factors) {
+    const sanic_expr& x = d->exprs[e];
+    if (x.op == SANIC_EX_ITEM) {
+        if (x.index == w) return true;
+        int n = st.leaf[x.index];
+        while (d->nodes[n].kind == SANIC_NODE_VIEW || d->nodes[n].kind == SANIC_NODE_REINDEX) n = d->nodes[n].in[0];
+        return ++factors <= 2 && d->nodes[n].kind == SANIC_NODE_INPUT && d->nodes[n].dtype == SANIC_BF16;
+    }
+    return x.op == SANIC_OP_MUL && exact_in_two(d, st, x.a, w, factors) && exact_in_two(d, st, x.b, w, factors);
 }
 
 }  // namespace
@@ -174,10 +186,34 @@ bool lower_gemm(const sanic_program_desc* d, int si, int64_t& scratch, LoweredSt
     const sanic_stage& st = d->stages[si];
     const sanic_carrier& c = st.carrier;
     const int64_t M = P.M, N = P.N, K = P.K;
-    int BM = M % 128 == 0 ? 128 : 64;
+    int BM = M % 128 == 0 || (M % 64 && M > 64) ? 128 : 64;
+    const int64_t NMB = (M + BM - 1) / BM;
     int BN = 128;
-    while (BN > 32 && (M / BM) * (N / BN) < 256) BN /= 2;
-    if (N % BN) return false;
+    while (BN > 32 && NMB * (N / BN) < 256) BN /= 2;
+    if (N < BN) return false;
+    // Sizes off the tiles: a row block past the last row repeats it (nothing of it is stored), the
+    // last column block starts BN columns before the end and stores only the columns that are
+    // its own, and the K tiles end at K, the first one's operand A zero where the second overlaps
+    // it. Only for operands the MFMA takes exactly (these calls were folded in f32). Generic fold →
+    // here, calls through sanic_hip_execute_static: M = 200, K = 2048, N = 8192 567 → 28.5 µs;
+    // 4-bit weights, M = 16 248 → 15.9 µs; the error against 64 bits is the bf16 store's in both.
+    const bool rag = M % 64 || N % BN || K % 64;
+    if (rag) {
+        int factors = 0;
+        if (!sched_is_auto(st.sched) || !exact_in_two(d, st, c.into[P.cslots[0]], P.w, factors)) return false;
+    }
+    const int64_t NNB = (N + BN - 1) / BN;
+    const bool ragN = N % BN != 0;
+    const int64_t NKT = (K + 63) / 64, dup = NKT * 64 - K;   // dup: k the second tile shares with the first
+    const int64_t MP = NMB * BM, KP = NKT * 64;              // plane extents
+    auto row_clamp = [&](const std::string& r) {
+        return M % BM ? "(" + r + " < " + std::to_string(M) + " ? " + r + " : (idx_t)" + std::to_string(M - 1) + ")" : r;
+    };
+    // the tile's first k, from its index · 64
+    auto tile_k = [&](const std::string& kt0) {
+        if (!dup) return kt0;
+        return "(" + kt0 + " >= " + std::to_string(dup) + " ? " + kt0 + " - " + std::to_string(dup) + " : (idx_t)0)";
+    };
     // 8 waves (4 × 2, two per SIMD) when the tile is 128 rows and at least 64 columns, so one
     // wave's LDS operand reads and global loads proceed under the other's MFMAs; else 4 (2 × 2)
     int NTH = (BM == 128 && BN >= 64) ? 512 : 256;
@@ -288,23 +324,25 @@ bool lower_gemm(const sanic_program_desc* d, int si, int64_t& scratch, LoweredSt
         Code l1, d1;
         render_weight_run(d, st.leaf[l], cr, {M, K}, l1, d1, "mm", "k0", "_p", rb, rd, rok, rc, rr, false);
         if (!rok || !rc) return false;
+        if (rag && rr.empty()) return false;      // a row leaf that is not one stored bf16 run
         if (rr.empty()) rawA = false;
         crow.push_back(cr);
     }
     if (!rawA) grouped = false;
     if (grouped) splitB = false;
+    if (rag && splitB) return false;             // a rebuilt weight has more than 16 bits
     // grouped tiles: tiling variants {8 waves, load depth 4; 4 waves, depth 4; 8 waves, depth 2}
     const int gvar = grouped && st.sched.variant > 0 && st.sched.variant < 3 ? st.sched.variant : 0;
     if (grouped && BM == 128 && BN == 32 && gvar != 1) NTH = 512;
     // A operands that need arithmetic (x·g of the fused RMSNorm) are built once by a first
     // launch into bf16 hi/lo planes [M][K] (plus the row slots), instead of by every one of the
     // N/BN column workgroups
-    const bool pre = splitA && N / BN >= 4 && K % 512 == 0;
-    const int64_t NKT = K / 64;
+    const bool pre = splitA && N / BN >= 4 && (rag ? NKT >= 2 : K % 512 == 0);
     int DEPTH = grouped ? (gvar == 2 ? 2 : 4) : 2;
     if (!grouped && st.sched.variant == 1) DEPTH = 4;
-    if (NKT % DEPTH || NKT < 2 * DEPTH) DEPTH = 2;
-    const bool deep = NKT % DEPTH == 0 && NKT >= 2 * DEPTH;
+    if ((!rag && NKT % DEPTH) || NKT < 2 * DEPTH) DEPTH = 2;
+    // (off the tiles the unrolled steps past the last K tile are skipped)
+    const bool deep = rag ? NKT >= DEPTH : NKT % DEPTH == 0 && NKT >= 2 * DEPTH;
     // With the x·g planes written by the first launch, each wave loads its own A fragments
     // instead of staging A through LDS: the A tile's LDS stores and fragment reads were over half
     // of a K step's LDS traffic (B2: ≈96 of ≈176 KB per CU). The planes are then stored in
@@ -312,10 +350,11 @@ bool lower_gemm(const sanic_program_desc* d, int si, int64_t& scratch, LoweredSt
     // so every fragment load is 1 KB contiguous (in 4-wave tiles, where two waves share rows,
     // both load them; the second from L1)
     const bool adirect = pre && deep && !getenv("SANIC_HIP_GEMM_ALDS");
+    if (rag && pre && !adirect) return false;
     // element offset of (row, k) in a plane: row-major, or fragment order (k a multiple of 8)
     auto plane_off = [&](const std::string& row, const std::string& k8) {
         if (!adirect) return "(" + row + ") * " + std::to_string(K) + " + " + k8;
-        return "((" + row + ") / 16 * " + std::to_string(K / 32) + " + (" + k8 + ") / 32) * 512 + ((" + row + ") % 16 + 16 * (((" + k8 + ") % 32) / 8)) * 8";
+        return "((" + row + ") / 16 * " + std::to_string(KP / 32) + " + (" + k8 + ") / 32) * 512 + ((" + row + ") % 16 + 16 * (((" + k8 + ") % 32) / 8)) * 8";
     };
     // waves along m and n: 4 × 2 / 2 × 2; grouped 32-column tiles of 8 waves 8 × 1, so no two
     // waves form the same rows' Σ x; 8 × 1 also for fragment-loaded A (each wave its own rows,
@@ -331,16 +370,18 @@ bool lower_gemm(const sanic_program_desc* d, int si, int64_t& scratch, LoweredSt
     int64_t hi_off = 0, lo_off = 0, rs_off = 0;
     // K slices of the first launch in fragment order (8 at K = 2048: 256 workgroups for M = 512)
     int PKS = 1;
-    while (adirect && PKS < 8 && K % (PKS * 2 * 4 * 32) == 0 && K / (PKS * 2) >= 256) PKS *= 2;
+    while (adirect && PKS < 8 && KP / (PKS * 2) >= 256) PKS *= 2;
+    // 32-deep k blocks of a row block, PKS slices × 4 waves of them at a time
+    const int64_t KB32 = KP / 32, PIT32 = (KB32 + PKS * 4 - 1) / (PKS * 4);
     Code kp;
     kp.indent = 1;
     if (pre) {
         hi_off = scratch;
-        scratch += ((M * K * 2 + 255) / 256) * 256;
+        scratch += ((MP * KP * 2 + 255) / 256) * 256;
         lo_off = scratch;
-        scratch += ((M * K * 2 + 255) / 256) * 256;
+        scratch += ((MP * KP * 2 + 255) / 256) * 256;
         rs_off = scratch;
-        scratch += ((PKS * M * std::max(SR, 1) * 4 + 255) / 256) * 256;
+        scratch += ((PKS * MP * std::max(SR, 1) * 4 + 255) / 256) * 256;
         kp.line("const int t = threadIdx.x, lane = t & 63, wv = t >> 6;");
         if (adirect) {
             // fragment order: a workgroup takes one 16-row block and one of PKS K slices, each
@@ -348,19 +389,24 @@ bool lower_gemm(const sanic_program_desc* d, int si, int64_t& scratch, LoweredSt
             // block and stores it at 16·lane bytes, so every wave store is 1 KB contiguous
             kp.line("const idx_t mp = (idx_t)(blockIdx.x / " + std::to_string(PKS) + ") * 16 + (lane & 15);");
             kp.line("const int pks = blockIdx.x % " + std::to_string(PKS) + ";");
+            kp.line("const idx_t mr = " + row_clamp("mp") + ";");
         } else {
             kp.line("const idx_t mp = (idx_t)blockIdx.x * 4 + wv;");
         }
         kp.line("unsigned short* ahi = (unsigned short*)((char*)a.scratch + " + std::to_string(hi_off) + ");");
         kp.line("unsigned short* alo = (unsigned short*)((char*)a.scratch + " + std::to_string(lo_off) + ");");
         for (int i = 0; i < SR; i++) kp.line("float rp" + std::to_string(i) + " = 0.0f;");
-        const int64_t PIT = adirect ? K / PKS / 4 / 32 : K / 512;   // runs per lane
+        const int64_t PIT = adirect ? PIT32 : K / 512;   // runs per lane
         for (int64_t i = 0; i < PIT; i++) {
             const std::string is = std::to_string(i);
-            const std::string k0 = adirect ? "(pks * " + std::to_string(K / PKS) + " + wv * " + std::to_string(K / PKS / 4) + " + " + std::to_string(i * 32) + " + (lane >> 4) * 8)"
-                                           : "(" + std::to_string(i * 512) + " + lane * 8)";
-            kp.line("{");
+            // the run's place in the planes; its k is `dup` less from the second tile on
+            const std::string kplane = adirect ? "((pks * " + std::to_string(PIT32 * 4) + " + wv * " + std::to_string(PIT32) + " + " + is + ") * 32 + (lane >> 4) * 8)"
+                                               : "(" + std::to_string(i * 512) + " + lane * 8)";
+            const std::string k0 = dup ? "(" + kplane + " < 64 ? " + kplane + " : " + kplane + " - " + std::to_string(dup) + ")" : kplane;
+            const bool guard = adirect && PIT32 * 4 * PKS != KB32;
+            kp.line(guard ? "if (" + kplane + " < " + std::to_string(KP) + ") {" : "{");
             kp.indent++;
+            if (dup) kp.line("const bool own = " + kplane + " < " + std::to_string(64 - dup) + " || " + kplane + " >= 64;");
             R.memo.emplace_back();
             std::vector<std::vector<std::string>> vals(P.rows.size());
             for (size_t li = 0; li < P.rows.size(); li++) {
@@ -369,7 +415,7 @@ bool lower_gemm(const sanic_program_desc* d, int si, int64_t& scratch, LoweredSt
                 std::string rr;
                 Code l1, d1;
                 l1.indent = d1.indent = kp.indent;
-                vals[li] = render_weight_run(d, st.leaf[P.rows[li]], crow[li], {M, K}, l1, d1, "mp", k0, "_p" + std::to_string(li) + "_" + is, rb, rd, rok, rc, rr, false);
+                vals[li] = render_weight_run(d, st.leaf[P.rows[li]], crow[li], {M, K}, l1, d1, adirect ? "mr" : "mp", k0, "_p" + std::to_string(li) + "_" + is, rb, rd, rok, rc, rr, false);
                 for (size_t b = 0; b < rb.size(); b++)
                     kp.line("const " + std::string(ctype_of(rd[b])) + "* __restrict__ wb" + std::to_string(b) + "_p" + std::to_string(li) + "_" + is + " = " + R.param(rb[b]) + ";");
                 kp.s << l1.str() << d1.str();
@@ -382,15 +428,18 @@ bool lower_gemm(const sanic_program_desc* d, int si, int64_t& scratch, LoweredSt
                     return "0.0f";
                 };
                 av[j] = expr_rest(R, kp, c.into[P.cslots[0]], P.w, item);
-                for (int sidx = 0; sidx < SR; sidx++)
-                    kp.line("rp" + std::to_string(sidx) + " += " + expr_rest(R, kp, c.into[P.rslots[sidx]], -1, item) + ";");
+                if (dup) av[j] = "(own ? " + av[j] + " : 0.0f)";
+                for (int sidx = 0; sidx < SR; sidx++) {
+                    const std::string rv = expr_rest(R, kp, c.into[P.rslots[sidx]], -1, item);
+                    kp.line("rp" + std::to_string(sidx) + " += " + (dup ? "own ? " + rv + " : 0.0f" : rv) + ";");
+                }
             }
             R.memo.pop_back();
             kp.line("unsigned h_[4], l_[4];");
             for (int q = 0; q < 4; q++)
                 kp.line("split_bf16(" + av[2 * q] + ", " + av[2 * q + 1] + ", h_[" + std::to_string(q) + "], l_[" + std::to_string(q) + "]);");
-            kp.line("*(sanic_u32x4*)(ahi + " + plane_off("mp", k0) + ") = (sanic_u32x4){h_[0], h_[1], h_[2], h_[3]};");
-            kp.line("*(sanic_u32x4*)(alo + " + plane_off("mp", k0) + ") = (sanic_u32x4){l_[0], l_[1], l_[2], l_[3]};");
+            kp.line("*(sanic_u32x4*)(ahi + " + plane_off("mp", kplane) + ") = (sanic_u32x4){h_[0], h_[1], h_[2], h_[3]};");
+            kp.line("*(sanic_u32x4*)(alo + " + plane_off("mp", kplane) + ") = (sanic_u32x4){l_[0], l_[1], l_[2], l_[3]};");
             kp.indent--;
             kp.line("}");
         }
@@ -405,7 +454,7 @@ bool lower_gemm(const sanic_program_desc* d, int si, int64_t& scratch, LoweredSt
             kp.line("__syncthreads();");
             kp.line("if (t < " + std::to_string(16 * SR) + ") {");
             kp.line("  const int r = t / " + std::to_string(SR) + ", sl = t % " + std::to_string(SR) + ";");
-            kp.line("  ((float*)((char*)a.scratch + " + std::to_string(rs_off) + "))[((idx_t)pks * " + std::to_string(M) + " + (blockIdx.x / " + std::to_string(PKS) +
+            kp.line("  ((float*)((char*)a.scratch + " + std::to_string(rs_off) + "))[((idx_t)pks * " + std::to_string(MP) + " + (blockIdx.x / " + std::to_string(PKS) +
                     ") * 16 + r) * " + std::to_string(SR) + " + sl] = ((rps[0][r][sl] + rps[1][r][sl]) + rps[2][r][sl]) + rps[3][r][sl];");
             kp.line("}");
         }
@@ -431,8 +480,9 @@ bool lower_gemm(const sanic_program_desc* d, int si, int64_t& scratch, LoweredSt
     }
     k.line("const int tid = threadIdx.x, lane = tid & 63, wv = tid >> 6;");
     k.line("const int l16 = lane & 15, lq = lane >> 4;");
-    k.line("const idx_t nb = blockIdx.x % " + std::to_string(N / BN) + ", mb = blockIdx.x / " + std::to_string(N / BN) + ";");
-    k.line("const idx_t m0 = mb * " + std::to_string(BM) + ", n0 = nb * " + std::to_string(BN) + ";");
+    k.line("const idx_t nb = blockIdx.x % " + std::to_string(NNB) + ", mb = blockIdx.x / " + std::to_string(NNB) + ";");
+    k.line("const idx_t m0 = mb * " + std::to_string(BM) + ", n_own = nb * " + std::to_string(BN) + ";");
+    k.line("const idx_t n0 = " + (ragN ? "n_own < " + std::to_string(N - BN) + " ? n_own : (idx_t)" + std::to_string(N - BN) : std::string("n_own")) + ";");
     k.line("const int wm = (wv / " + std::to_string(WGN) + ") * " + std::to_string(WM) + ", wn = (wv % " + std::to_string(WGN) + ") * " + std::to_string(WN) + ";");
     k.line("f32x4 acc[" + std::to_string(MT) + "][" + std::to_string(NT) + "];");
     k.line("#pragma unroll");
@@ -450,13 +500,16 @@ bool lower_gemm(const sanic_program_desc* d, int si, int64_t& scratch, LoweredSt
     const int RUNS_B = BN * 8 / BTH;
     auto emit_loads = [&](Code& c2, const std::string& kt0, const std::string& sfx) {
         // A runs
-        c2.line("const idx_t mm" + sfx + " = m0 + tid / " + std::to_string(TPR) + ";");
+        c2.line("const idx_t mt" + sfx + " = m0 + tid / " + std::to_string(TPR) + ";");
+        c2.line("const idx_t mm" + sfx + " = " + row_clamp("mt" + sfx) + ";");
+        if (dup) c2.line("const idx_t tk" + sfx + " = " + tile_k(kt0) + ";");
+        const std::string tk = dup ? "tk" + sfx : kt0;
         for (int i = 0; i < MT && adirect; i++)
             for (int ks = 0; ks < 2; ks++) {
                 // the operand fragment itself: lane (l16, lq) holds row wm + 16·i + l16, k run lq·8
                 // of the tile's 32-deep half ks (16 contiguous bytes of the row)
                 const std::string nm = std::to_string(i) + "_" + std::to_string(ks) + sfx;
-                const std::string at = "((m0 + wm + " + std::to_string(i * 16) + ") / 16 * " + std::to_string(K / 32) + " + (" + kt0 + " + " + std::to_string(ks * 32) + ") / 32) * 512 + lane * 8";
+                const std::string at = "((m0 + wm + " + std::to_string(i * 16) + ") / 16 * " + std::to_string(KP / 32) + " + (" + kt0 + " + " + std::to_string(ks * 32) + ") / 32) * 512 + lane * 8";
                 c2.line("const sanic_u32x4 pah" + nm + " = *(const sanic_u32x4*)((const unsigned short*)((const char*)a.scratch + " + std::to_string(hi_off) + ") + " + at + ");");
                 c2.line("const sanic_u32x4 pal" + nm + " = *(const sanic_u32x4*)((const unsigned short*)((const char*)a.scratch + " + std::to_string(lo_off) + ") + " + at + ");");
             }
@@ -469,7 +522,7 @@ bool lower_gemm(const sanic_program_desc* d, int si, int64_t& scratch, LoweredSt
                     " * " + std::to_string(K) + " + " + k0 + ");");
         }
         for (int r = 0; r < RUNS_A && !pre; r++) {
-            std::string k0 = "(" + kt0 + " + (tid % " + std::to_string(TPR) + ") * " + std::to_string(64 / TPR) + " + " + std::to_string(r * 8) + ")";
+            std::string k0 = "(" + tk + " + (tid % " + std::to_string(TPR) + ") * " + std::to_string(64 / TPR) + " + " + std::to_string(r * 8) + ")";
             for (size_t li = 0; li < P.rows.size(); li++) {
                 std::vector<int> rb, rd;
                 bool rok = true, rc = true;
@@ -497,14 +550,14 @@ bool lower_gemm(const sanic_program_desc* d, int si, int64_t& scratch, LoweredSt
             if (bkn) {
                 // chunk c = tid + 256·r: k row c / (BN/8), 8 columns from (c % (BN/8))·8
                 const std::string cc = "(" + btid + " + " + std::to_string(r * BTH) + ")";
-                kk = "(" + kt0 + " + " + cc + " / " + std::to_string(BN / 8) + ")";
+                kk = "(" + tk + " + " + cc + " / " + std::to_string(BN / 8) + ")";
                 nn = "(n0 + (" + cc + " % " + std::to_string(BN / 8) + ") * 8)";
             } else if (contig) {
                 nn = "(n0 + (" + btid + " / 8) + " + std::to_string(r * (BTH / 8)) + ")";
-                kk = "(" + kt0 + " + (" + btid + " % 8) * 8)";
+                kk = "(" + tk + " + (" + btid + " % 8) * 8)";
             } else {
                 nn = "(n0 + (" + btid + " % " + std::to_string(BN) + "))";
-                kk = "(" + kt0 + " + ((" + btid + " / " + std::to_string(BN) + ") + " + std::to_string(r * (BTH / BN)) + ") * 8)";
+                kk = "(" + tk + " + ((" + btid + " / " + std::to_string(BN) + ") + " + std::to_string(r * (BTH / BN)) + ") * 8)";
             }
             std::vector<int> rb, rd;
             bool rok = true, rc = true;
@@ -547,10 +600,12 @@ bool lower_gemm(const sanic_program_desc* d, int si, int64_t& scratch, LoweredSt
             }
         }
     };
-    auto emit_stores = [&](Code& c2, const std::string& buf, const std::string& sfx) {
+    // `first`: the first tile, whose k from 64 − dup on are the second's
+    auto emit_stores = [&](Code& c2, const std::string& buf, const std::string& sfx, bool first = false) {
         c2.line("{");
         c2.indent++;
         c2.line("const int ar = tid / " + std::to_string(TPR) + ";");
+        auto own = [&](int r) { return "(tid % " + std::to_string(TPR) + ") * " + std::to_string(64 / TPR) + " + " + std::to_string(r * 8) + " < " + std::to_string(64 - dup); };
         for (int r = 0; r < RUNS_A && pre && !adirect; r++) {
             const std::string rs = std::to_string(r);
             const std::string aoff = koff("ar", "(tid % " + std::to_string(TPR) + ") * " + std::to_string(64 / TPR) + " + " + std::to_string(r * 8), AS);
@@ -559,7 +614,7 @@ bool lower_gemm(const sanic_program_desc* d, int si, int64_t& scratch, LoweredSt
         }
         for (int r = 0; r < RUNS_A && !pre && rawA; r++) {
             const std::string aoff = koff("ar", "(tid % " + std::to_string(TPR) + ") * " + std::to_string(64 / TPR) + " + " + std::to_string(r * 8), AS);
-            c2.line("*(sanic_u32x4*)(&a_lds[" + buf + "][" + aoff + "]) = rawa" + std::to_string(r) + sfx + ";");
+            c2.line("*(sanic_u32x4*)(&a_lds[" + buf + "][" + aoff + "]) = " + (first && dup ? own(r) + " ? rawa" + std::to_string(r) + sfx + " : (sanic_u32x4){0, 0, 0, 0}" : "rawa" + std::to_string(r) + sfx) + ";");
         }
 
         for (int r = 0; r < RUNS_A && !pre && !rawA; r++) {
@@ -574,10 +629,10 @@ bool lower_gemm(const sanic_program_desc* d, int si, int64_t& scratch, LoweredSt
                     return "0.0f";
                 };
                 std::string v = expr_rest(R, c2, c.into[P.cslots[0]], P.w, item);
-                av[j] = v;
+                av[j] = first && dup ? "(" + own(r) + " ? " + v + " : 0.0f)" : v;
                 for (int sidx = 0; sidx < SR; sidx++) {
                     std::string rv = expr_rest(R, c2, c.into[P.rslots[sidx]], -1, item);
-                    c2.line("racc" + std::to_string(sidx) + " += " + rv + ";");
+                    c2.line("racc" + std::to_string(sidx) + " += " + (first && dup ? own(r) + " ? " + rv + " : 0.0f" : rv) + ";");
                 }
             }
             const std::string aoff = koff("ar", "(tid % " + std::to_string(TPR) + ") * " + std::to_string(64 / TPR) + " + " + std::to_string(r * 8), AS);
@@ -758,7 +813,7 @@ bool lower_gemm(const sanic_program_desc* d, int si, int64_t& scratch, LoweredSt
         k.line("{");
         k.indent++;
         emit_loads(k, "(idx_t)0", "_0");
-        emit_stores(k, "0", "_0");
+        emit_stores(k, "0", "_0", true);
         k.indent--;
         k.line("}");
         k.line("__syncthreads();");
@@ -811,6 +866,7 @@ bool lower_gemm(const sanic_program_desc* d, int si, int64_t& scratch, LoweredSt
         k.s << decl.str();
         if (adirect) {
             // tile 0's set: its A fragments stay in registers for the first step, its B goes to LDS
+            // (the planes hold the zeros where the second tile overlaps the first)
             load_into("(idx_t)0", set_sfx(0), names[0]);
             emit_stores(k, "0", set_sfx(0));
             k.line("__syncthreads();");
@@ -820,6 +876,8 @@ bool lower_gemm(const sanic_program_desc* d, int si, int64_t& scratch, LoweredSt
         k.line("for (idx_t kt = 0; kt < " + N2 + "; kt += " + DS + ") {");
         k.indent++;
         for (int u = 0; u < DEPTH; u++) {
+            const bool skip = u && NKT % DEPTH;
+            if (skip) k.line("if (kt + " + std::to_string(u) + " < " + N2 + ") {");
             // step kt+u: tile kt+u is in LDS buffer u % 2; its set takes tile kt+u+DEPTH
             // (A fragments in the set: the MFMAs take them before the set is reloaded)
             if (!adirect) load_into("(((kt + " + std::to_string(u + DEPTH) + ") % " + N2 + ") * 64)", set_sfx(u), names[u]);
@@ -836,6 +894,7 @@ bool lower_gemm(const sanic_program_desc* d, int si, int64_t& scratch, LoweredSt
                 k.line("}");
             }
             k.line("__syncthreads();");
+            if (skip) k.line("}");
         }
         k.indent--;
         k.line("}");
@@ -860,7 +919,7 @@ bool lower_gemm(const sanic_program_desc* d, int si, int64_t& scratch, LoweredSt
     if (SR && pre) {
         std::string sum;
         for (int q = 0; q < PKS; q++) {
-            const std::string pq = "((const float*)((const char*)a.scratch + " + std::to_string(rs_off) + "))[" + std::to_string((int64_t)q * M * SR) + " + m0 * " + std::to_string(SR) + " + i]";
+            const std::string pq = "((const float*)((const char*)a.scratch + " + std::to_string(rs_off) + "))[" + std::to_string((int64_t)q * MP * SR) + " + m0 * " + std::to_string(SR) + " + i]";
             sum = q ? "(" + sum + " + " + pq + ")" : pq;
         }
         k.line("for (int i = tid; i < " + std::to_string(BM * SR) + "; i += " + std::to_string(NTH) + ") rs_lds[i] = " + sum + ";");
@@ -877,6 +936,7 @@ bool lower_gemm(const sanic_program_desc* d, int si, int64_t& scratch, LoweredSt
         k.line("__syncthreads();");
     }
     // finish: project, epilogue, narrowing store per element
+    if (rag) k.line("bool odd = false;");
     k.line("#pragma unroll");
     k.line("for (int i = 0; i < " + std::to_string(MT) + "; ++i)");
     k.line("  #pragma unroll");
@@ -886,27 +946,52 @@ bool lower_gemm(const sanic_program_desc* d, int si, int64_t& scratch, LoweredSt
     k.indent += 3;
     k.line("const int ml = wm + i * 16 + lq * 4 + r;");
     k.line("const idx_t gm = m0 + ml, gn = n0 + wn + j * 16 + l16;");
+    if (M % BM || ragN) k.line(std::string("if (") + (M % BM ? "gm >= " + std::to_string(M) : "") + (M % BM && ragN ? " || " : "") + (ragN ? "gn < n_own" : "") + ") continue;");
     k.line("const float fs" + std::to_string(P.cslots[0]) + " = acc[i][j][r];");
     for (int i = 0; i < SR; i++)
         k.line("const float fs" + std::to_string(P.rslots[i]) + " = rs_lds[ml * " + std::to_string(SR) + " + " + std::to_string(i) + "];");
-    R.memo.emplace_back();
-    std::string f = R.expr(k, c.project, "", "", "", "fs");
-    k.line("const float fold_v = " + f + ";");
     std::vector<std::string> gc(st.rank, "0");
     gc[P.mdim] = "gm";
     gc[P.ndim] = "gn";
-    std::string v = "fold_v";
-    if (st.epilogue >= 0) {
-        R.fold_var = "fold_v";
-        v = R.value(k, st.epilogue, gc);
-    }
-    R.memo.pop_back();
     std::string lin;
     for (int j = 0; j < st.rank; j++)
         lin = j == 0 ? "(idx_t)(" + gc[0] + ")" : "(" + lin + " * " + std::to_string(st.grid[j]) + " + (idx_t)(" + gc[j] + "))";
-    k.line(store_stmt(R.param(st.out_buffer), lin, st.out_dtype, v, false, d->buffers[st.out_buffer].scale));
+    // project, epilogue and the narrowing store at (gm, gn)
+    auto finish = [&]() {
+        R.memo.emplace_back();
+        std::string f = R.expr(k, c.project, "", "", "", "fs");
+        k.line("const float fold_v = " + f + ";");
+        std::string v = "fold_v";
+        if (st.epilogue >= 0) {
+            R.fold_var = "fold_v";
+            v = R.value(k, st.epilogue, gc);
+        }
+        R.memo.pop_back();
+        k.line(store_stmt(R.param(st.out_buffer), lin, st.out_dtype, v, false, d->buffers[st.out_buffer].scale));
+    };
+    if (rag) k.line("odd |= !(__builtin_fabsf(acc[i][j][r]) <= 3.402823466e38f);");
+    finish();
     k.indent -= 3;
     k.line("    }");
+    if (rag) {
+        // Infinities and NaNs: the hi + lo split of an infinity, the repeated rows and the zeroed
+        // overlap do not carry them as the fold does, so a lane with such a sum folds its points
+        // again, element by element.
+        k.line("if (odd) {");
+        k.indent++;
+        k.line("#pragma nounroll");
+        k.line("for (int p = 0; p < " + std::to_string(MT * NT * 4) + "; ++p) {");
+        k.indent++;
+        k.line("const idx_t gm = m0 + wm + p / " + std::to_string(NT * 4) + " * 16 + lq * 4 + p % 4, gn = n0 + wn + p / 4 % " + std::to_string(NT) + " * 16 + l16;");
+        k.line("if (gm >= " + std::to_string(M) + " || gn < n_own) continue;");
+        for (int j = 0; j < st.rank; j++) k.line("const idx_t g" + std::to_string(j) + " = " + gc[j] + ";");
+        emit_point_fold(R, k, st, "fs");
+        finish();
+        k.indent--;
+        k.line("}");
+        k.indent--;
+        k.line("}");
+    }
 
     const std::string kname = "sanic_gemm_" + std::to_string(M) + "x" + std::to_string(N) + "x" + std::to_string(K);
     std::ostringstream src;
@@ -926,18 +1011,18 @@ bool lower_gemm(const sanic_program_desc* d, int si, int64_t& scratch, LoweredSt
     src << R.args_struct(pre ? std::vector<std::string>{"float* __restrict__ scratch"} : std::vector<std::string>{});
     if (pre) src << "extern \"C\" __global__ void __launch_bounds__(256) " << kname << "_pre(Args a) {\n" << R.entry() << kp.str() << "}\n";
     src << "extern \"C\" __global__ void __launch_bounds__(" << NTH << ") " << kname << "(Args a) {\n" << R.entry() << k.str() << "}\n";
-    out.kernel_kind = "skeleton:gemm[" + std::to_string(BM) + "x" + std::to_string(BN) + (splitA ? ",a2" : "") + (splitB ? ",b2" : "") +
+    out.kernel_kind = "skeleton:gemm[" + std::to_string(BM) + "x" + std::to_string(BN) + (splitA ? ",a2" : "") + (splitB ? ",b2" : "") + (rag ? ",any size" : "") +
                       (grouped ? ",grp" : "") + (bkn ? ",kn" : "") + (pre ? ",pre" : "") + (deep ? ",d" + std::to_string(DEPTH) : "") + ",w" + std::to_string(NTH / 64) + (adirect ? ",ad" : "") + "]";
-    out.variants = grouped ? 3 : 2;
+    out.variants = rag ? 1 : grouped ? 3 : 2;
     // dequantized-weight tiles (int4): the ILP-maximising machine scheduler, D2 25.1 → 22.9 µs;
     // bf16 tiles keep the default strategy (no measurable difference)
     out.source = (splitB || grouped ? std::string("// sched-strategy: iterative-ilp\n") : std::string()) + src.str();
     std::vector<Arg> args = R.arg_list();
     if (pre) {
         args.push_back({Arg::SCRATCH, 0});
-        out.launches.push_back({kname + "_pre", "", dim3((unsigned)(adirect ? M / 16 * PKS : M / 4)), dim3(256), 0, args});
+        out.launches.push_back({kname + "_pre", "", dim3((unsigned)(adirect ? MP / 16 * PKS : M / 4)), dim3(256), 0, args});
     }
-    out.launches.push_back({kname, "", dim3((unsigned)((M / BM) * (N / BN))), dim3(NTH), 0, args});
+    out.launches.push_back({kname, "", dim3((unsigned)(NMB * NNB)), dim3(NTH), 0, args});
     return true;
 }
 

@@ -99,3 +99,57 @@ def test_int4_gemm(dev, M, K, N, G, zk, variant):
     assert exe.stage_kernel(0).startswith("skeleton:gemm")
     assert ("grp" in exe.stage_kernel(0)) == (G % 64 == 0)
     assert err < 2e-2
+
+
+def _same_as_generic(dev, monkeypatch, prog, vals, scale):
+    """The skeleton's bf16 output against the generic f32 fold of the same program: both sum the
+    same exact products in f32, so before the store they differ by at most K · 2^-24 of Σ|terms|
+    (`scale`), and the store adds one bf16 step; infinities and NaNs sit at the same points."""
+    got, exe = run_on_gpu(dev, prog, vals)
+    kind = exe.stage_kernel(0)
+    monkeypatch.setenv("SANIC_HIP_GENERIC", "1")
+    want, exe = run_on_gpu(dev, prog, vals)
+    monkeypatch.delenv("SANIC_HIP_GENERIC")
+    assert exe.stage_kernel(0).startswith("fold:")
+    a, b = np.asarray(got["y"], np.float64), np.asarray(want["y"], np.float64)
+    fin = np.isfinite(b)
+    assert np.array_equal(np.isnan(a), np.isnan(b)) and np.array_equal(a[~fin & ~np.isnan(b)], b[~fin & ~np.isnan(b)]), kind
+    over = np.abs(a[fin] - b[fin]) - 2.0 ** -7 * np.abs(b)[fin]
+    print(kind, float(over.max() / scale))
+    assert over.max() <= 2.0 ** -13 * scale, kind
+    return kind
+
+
+# rows, k and columns off every tile: below one tile, one past it, K tiles odd in number and
+# overlapping, columns not a multiple of 8
+RAGGED = [(2, 64, 32), (65, 128, 96), (200, 2048, 8192), (33, 200, 77), (100, 72, 1003), (129, 1000, 333),
+          (256, 128, 8224), (127, 832, 5184)]
+
+
+@pytest.mark.parametrize("kmajor", [False, True])
+@pytest.mark.parametrize("M,K,N", RAGGED)
+def test_rmsnorm_gemm_any_size(dev, monkeypatch, M, K, N, kmajor):
+    prog = configs.rmsnorm_projection(M=M, K=K, N=N, kmajor=kmajor)
+    x = _bf16_vals(321, M * K).reshape(M, K)
+    w = _bf16_vals(323, K * N, 0.0, 0.02).reshape((K, N) if kmajor else (N, K))
+    vals = {"x": x, "g": _bf16_vals(322, K, 1.0, 0.02), "W": w}
+    assert "skeleton" in _same_as_generic(dev, monkeypatch, prog, vals, scale=0.02 * K)
+    # an infinite activation in the last row, a NaN weight in the last column's last k
+    x[M - 1, K - 1] = np.inf
+    w[(K - 1, N - 1) if kmajor else (N - 1, K - 1)] = np.nan
+    w[(0, 0)] = np.inf
+    _same_as_generic(dev, monkeypatch, prog, vals, scale=0.02 * K)
+
+
+@pytest.mark.parametrize("M,K,N,G", [(2, 64, 32, 64), (16, 2048, 8192, 64), (100, 1152, 777, 64), (65, 384, 1000, 128),
+                                     (33, 192, 64, 64), (17, 256, 300, 32)])
+def test_int4_gemm_any_size(dev, monkeypatch, M, K, N, G):
+    prog = configs.int4_matmul(M=M, K=K, N=N, G=G)
+    s = _bf16_vals(331, N * K // G, 0.001, 0.02, kind="uniform").reshape(N, K // G)
+    z = _bf16_vals(332, N * K // G, -0.1, 0.1, kind="uniform").reshape(s.shape)
+    x = _bf16_vals(333, M * K).reshape(M, K)
+    vals = {"x": x, "Wq": np.random.default_rng(5).integers(0, 16, size=(N, K // G, G)), "S": s, "Z": z}
+    _same_as_generic(dev, monkeypatch, prog, vals, scale=0.2 * K)
+    x[0, 0] = -np.inf
+    s[N - 1, 0] = np.nan
+    _same_as_generic(dev, monkeypatch, prog, vals, scale=0.2 * K)
