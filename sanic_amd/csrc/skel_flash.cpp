@@ -438,6 +438,11 @@ bool lower_flash_prefill(const sanic_program_desc* d, int si, int64_t& scratch, 
     // second to arrive combines them (the carrier's ExpShifted combine with its −∞ guard) and
     // projects. It evens out launches whose equal-sized blocks overfill the resident slots.
     int SPL = fvar == 2 ? 2 : 1;
+    if (P.ragged) {
+        // register every buffer the element-by-element fold reads before the argument struct is written
+        Code scratch_code;
+        emit_point_fold(R, scratch_code, st, "pf");
+    }
     src << (SPL > 1 ? R.args_struct({"float* __restrict__ scratch"}) : R.args_struct({}));
     src << "typedef __bf16 sanic_bf16x2 __attribute__((ext_vector_type(2)));\n";
     src << "typedef float sanic_f32x2 __attribute__((ext_vector_type(2)));\n";
@@ -1038,7 +1043,10 @@ bool lower_flash_prefill(const sanic_program_desc* d, int si, int64_t& scratch, 
     k.indent++;
     k.line("const float lt = lsum[qt][0];");
     k.line("const idx_t qi = q0 + qt * 16 + l16;");
-    if (P.ragged) k.line("if (qi >= " + std::to_string(NQ) + ") continue;");
+    if (P.ragged) {
+        k.line("if (qi >= " + std::to_string(NQ) + ") continue;");
+        k.line("bool odd = !(__builtin_fabsf(lt) <= 3.402823466e38f);");
+    }
     k.line("#pragma unroll");
     k.line("for (int dt = 0; dt < 4; ++dt)");
     k.line("  #pragma unroll");
@@ -1048,8 +1056,30 @@ bool lower_flash_prefill(const sanic_program_desc* d, int si, int64_t& scratch, 
     for (size_t s = 0; s < P.scalar_slots.size(); s++)
         k.line("    fs[" + std::to_string(P.scalar_slots[s]) + "] = " + flit(P.scalar_into[s]) + " * lt;");
     k.line("    fs[" + std::to_string(P.vec_slots[0]) + "] = o[dt][qt][r];");
+    if (P.ragged) k.line("    odd |= !(__builtin_fabsf(o[dt][qt][r]) <= 3.402823466e38f);");
     k.line("    finish(a, fs, hh, qi, dt * 16 + lq * 4 + r);");
     k.line("  }");
+    if (P.ragged) {
+        // Infinities and NaNs: a masked key of the same tile weighs 0 here, and 0 · ∞ is not what the
+        // fold over the honest window gives; a lane with such a sum folds its points again.
+        k.line("if (odd) {");
+        k.line("  #pragma nounroll");
+        k.line("  for (int p = 0; p < 16; ++p) {");
+        k.indent += 2;
+        std::vector<std::string> gc(st.rank, "0");
+        gc[P.hdim] = "hh";
+        gc[P.qdim] = "qi";
+        gc[P.edim] = "(p / 4 * 16 + lq * 4 + p % 4)";
+        for (int j = 0; j < st.rank; j++) k.line("const idx_t g" + std::to_string(j) + " = " + gc[j] + ";");
+        emit_point_fold(R, k, st, "pf");
+        std::string arr;
+        for (int sl2 = 0; sl2 < c.slots; sl2++) arr += (sl2 ? ", pf" : "pf") + std::to_string(sl2);
+        k.line("const float fs[" + std::to_string(c.slots) + "] = {" + arr + "};");
+        k.line("finish(a, fs, hh, qi, " + gc[P.edim] + ");");
+        k.indent -= 2;
+        k.line("  }");
+        k.line("}");
+    }
     k.indent--;
     k.line("}");
 

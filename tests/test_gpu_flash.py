@@ -134,3 +134,22 @@ def test_flash_any_length(dev, monkeypatch, NH, NKV, S, window):
     over = np.abs(got["O"] - want["O"]) - 2.0 ** -7 * np.abs(want["O"])
     print(S, window, float(over.max()), max_rel_err(got["O"], want["O"]))
     assert over.max() < 1e-4
+
+
+def test_flash_any_length_keeps_infinities_and_nans(dev, monkeypatch):
+    """A NaN value row, an infinite value and an infinite key late in the prompt: the rows before
+    them see nothing of them, and every point is finite or not exactly where the generic fold's is."""
+    NH, NKV, S = 2, 1, 100
+    prog = configs.flash_prefill(NH, NKV, S, window=30)
+    vals = _inputs(NH, NKV, S, seed=490)
+    vals["V"][0, 50] = np.nan
+    vals["V"][0, 90, 3] = -np.inf
+    vals["K"][0, 75, 5] = np.inf
+    got, _ = run_on_gpu(dev, prog, vals)
+    monkeypatch.setenv("SANIC_HIP_GENERIC", "1")
+    want, _ = run_on_gpu(dev, prog, vals)
+    g, w = got["O"], want["O"]
+    assert np.isfinite(w).any() and np.isnan(w).any()
+    assert np.array_equal(np.isnan(g), np.isnan(w)) and np.array_equal(np.isinf(g), np.isinf(w))
+    fin = np.isfinite(w)
+    assert np.max(np.abs(g[fin] - w[fin]) - 2.0 ** -7 * np.abs(w[fin])) < 1e-4
