@@ -28,14 +28,6 @@ namespace sanic {
 
 namespace {
 
-struct GemmPlan {
-    int mdim = -1, ndim = -1;
-    int64_t M = 0, N = 0, K = 0;
-    int w = -1;
-    std::vector<int> rows;          // row leaves
-    std::vector<int> cslots, rslots;
-};
-
 bool expr_reads(const sanic_program_desc* d, int e, int item) {
     const sanic_expr& x = d->exprs[e];
     if (x.op == SANIC_EX_ITEM) return x.index == item;
@@ -54,6 +46,8 @@ bool linear_mul(const sanic_program_desc* d, int e, int w) {
     }
     return false;
 }
+
+}  // namespace
 
 // Render an Expr with item w read as 1 and items named by `item(i)`.
 std::string expr_rest(Renderer& R, Code& code, int e, int w, const std::function<std::string(int)>& item) {
@@ -142,7 +136,9 @@ bool gemm_plan(const sanic_program_desc* d, int si, GemmPlan& P) {
         const int64_t cost = (a_raw ? 0 : Mq * ((Nq + 127) / 128)) + (raw_leaf(Q.w) ? 0 : Nq * ((Mq + 127) / 128));
         // ties: keep the stored bf16 operand on the A side (its tile needs no arithmetic)
         const int64_t key = cost * 2 + (a_raw ? 0 : 1);
-        if (best_cost < 0 || key < best_cost) { best = Q; best_cost = key; }
+        // (and of two stored operands the longer side as the weight when the other is below a tile)
+        const bool longer = key == best_cost && st.grid[best.ndim] < 32 && st.grid[Q.ndim] > st.grid[best.ndim];
+        if (best_cost < 0 || key < best_cost || longer) { best = Q; best_cost = key; }
     }
     P = best;
     if (P.w < 0) return false;
@@ -164,21 +160,6 @@ bool exact_in_two(const sanic_program_desc* d, const sanic_stage& st, int e, int
     }
     return x.op == SANIC_OP_MUL && exact_in_two(d, st, x.a, w, factors) && exact_in_two(d, st, x.b, w, factors);
 }
-
-}  // namespace
-
-// the vector weight renderer lives in skeletons.cpp
-std::vector<std::string> render_weight_run(const sanic_program_desc* d, int node, const std::vector<Sym>& c,
-                                           const std::vector<int64_t>& ext, Code& lc, Code& dc, const std::string& nn,
-                                           const std::string& k0, const std::string& sfx, std::vector<int>& bufs,
-                                           std::vector<int>& dtypes, bool& ok, bool& contiguous, std::string& raw_bf16,
-                                           bool stream);
-
-bool render_weight_affine(const sanic_program_desc* d, int node, const std::vector<Sym>& c,
-                          const std::vector<int64_t>& ext, Code& lc, Code& dc, const std::string& nn,
-                          const std::string& k0, const std::string& sfx, std::vector<int>& bufs,
-                          std::vector<int>& dtypes, std::vector<std::string>& q, std::string& A, std::string& B,
-                          bool& negB, int64_t& uniform_div, bool stream, bool raw_loads = false);
 
 bool lower_gemm(const sanic_program_desc* d, int si, int64_t& scratch, LoweredStage& out) {
     GemmPlan P;

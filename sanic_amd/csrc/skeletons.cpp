@@ -1839,6 +1839,7 @@ bool lower_gemv_kmajor(const sanic_program_desc* d, int si, int64_t& scratch, Lo
 
 bool lower_skeleton(const sanic_program_desc* d, int si, int64_t& scratch, LoweredStage& out) {
     if (lower_gemv_kmajor(d, si, scratch, out)) return true;
+    if (lower_skinny(d, si, out)) return true;
     if (lower_gemm(d, si, scratch, out)) return true;
     if (lower_flash_prefill(d, si, scratch, out)) return true;
     if (lower_attn_decode(d, si, scratch, out)) return true;

@@ -1,5 +1,6 @@
 // Structural analysis shared by the skeletons: symbolic affine coordinates and accesses.
 #pragma once
+#include <functional>
 #include <set>
 #include <string>
 #include <vector>
@@ -53,7 +54,34 @@ std::vector<std::string> render_run(const sanic_program_desc* d, int node, const
                                     Code& lc, Code& dc, const std::string& sfx, std::vector<int>& bufs,
                                     std::vector<int>& dtypes, bool& ok);
 
+// One run of 8 of a weight or row leaf at (nn, k0), and a packed 4-bit weight as q·A ± B
+// (skeletons.cpp).
+std::vector<std::string> render_weight_run(const sanic_program_desc* d, int node, const std::vector<Sym>& c,
+                                           const std::vector<int64_t>& ext, Code& lc, Code& dc, const std::string& nn,
+                                           const std::string& k0, const std::string& sfx, std::vector<int>& bufs,
+                                           std::vector<int>& dtypes, bool& ok, bool& contiguous, std::string& raw_bf16,
+                                           bool stream);
+bool render_weight_affine(const sanic_program_desc* d, int node, const std::vector<Sym>& c,
+                          const std::vector<int64_t>& ext, Code& lc, Code& dc, const std::string& nn,
+                          const std::string& k0, const std::string& sfx, std::vector<int>& bufs,
+                          std::vector<int>& dtypes, std::vector<std::string>& q, std::string& A, std::string& B,
+                          bool& negB, int64_t& uniform_div, bool stream, bool raw_loads = false);
+
+// A Plain(Add) stage over two output axes as a contraction (skel_gemm.cpp): one slot W·rest(row
+// items) summed over the stream, the other slots free of W.
+struct GemmPlan {
+    int mdim = -1, ndim = -1;
+    int64_t M = 0, N = 0, K = 0;
+    int w = -1;
+    std::vector<int> rows;          // row leaves
+    std::vector<int> cslots, rslots;
+};
+bool gemm_plan(const sanic_program_desc* d, int si, GemmPlan& P);
+bool exact_in_two(const sanic_program_desc* d, const sanic_stage& st, int e, int w, int& factors);
+std::string expr_rest(Renderer& R, Code& code, int e, int w, const std::function<std::string(int)>& item);
+
 bool lower_gemm(const sanic_program_desc* d, int si, int64_t& scratch, LoweredStage& out);
+bool lower_skinny(const sanic_program_desc* d, int si, LoweredStage& out);
 bool lower_flash_prefill(const sanic_program_desc* d, int si, int64_t& scratch, LoweredStage& out);
 bool lower_attn_decode(const sanic_program_desc* d, int si, int64_t& scratch, LoweredStage& out);
 

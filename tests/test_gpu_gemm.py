@@ -123,7 +123,7 @@ def _same_as_generic(dev, monkeypatch, prog, vals, scale):
 # rows, k and columns off every tile: below one tile, one past it, K tiles odd in number and
 # overlapping, columns not a multiple of 8
 RAGGED = [(2, 64, 32), (65, 128, 96), (200, 2048, 8192), (33, 200, 77), (100, 72, 1003), (129, 1000, 333),
-          (256, 128, 8224), (127, 832, 5184)]
+          (256, 128, 8224), (127, 832, 5184), (8, 4160, 96), (20, 2200, 49), (40, 2048, 8192)]
 
 
 @pytest.mark.parametrize("kmajor", [False, True])
@@ -142,7 +142,8 @@ def test_rmsnorm_gemm_any_size(dev, monkeypatch, M, K, N, kmajor):
 
 
 @pytest.mark.parametrize("M,K,N,G", [(2, 64, 32, 64), (16, 2048, 8192, 64), (100, 1152, 777, 64), (65, 384, 1000, 128),
-                                     (33, 192, 64, 64), (17, 256, 300, 32)])
+                                     (33, 192, 64, 64), (17, 256, 300, 32), (31, 8320, 48, 64),
+                                     (16, 512, 16, 512)])
 def test_int4_gemm_any_size(dev, monkeypatch, M, K, N, G):
     prog = configs.int4_matmul(M=M, K=K, N=N, G=G)
     s = _bf16_vals(331, N * K // G, 0.001, 0.02, kind="uniform").reshape(N, K // G)
@@ -153,3 +154,22 @@ def test_int4_gemm_any_size(dev, monkeypatch, M, K, N, G):
     x[0, 0] = -np.inf
     s[N - 1, 0] = np.nan
     _same_as_generic(dev, monkeypatch, prog, vals, scale=0.2 * K)
+
+
+@pytest.mark.parametrize("kmajor", [False, True])
+@pytest.mark.parametrize("M,K,N", [(8, 256, 64), (100, 320, 4096 + 24)])
+def test_rmsnorm_gemm_any_address(dev, M, K, N, kmajor):
+    """Rows and weights bound one element off a 16-byte boundary (the sizes that the generic fold
+    took at any address): the same bits as bound on one."""
+    prog = configs.rmsnorm_projection(M=M, K=K, N=N, kmajor=kmajor)
+    vals = {"x": _bf16_vals(341, M * K), "g": _bf16_vals(342, K, 1.0, 0.02), "W": _bf16_vals(343, K * N, 0.0, 0.02)}
+    exe = dev.prepare(prog)
+    assert exe.stage_kernel(0).startswith("skeleton:gemm")
+    bufs = {n: dev.from_values(v, ir.BF16) for n, v in vals.items()}
+    want = exe.execute(bufs)["y"].download()
+    for n in ("x", "W"):
+        raw = bufs[n].download()
+        hold = dev.alloc(len(raw) + 16)
+        hold.upload(b"\0\0" + raw)
+        bufs["hold" + n], bufs[n] = hold, dev.wrap(hold.device_ptr + 2, len(raw))
+    assert exe.execute({n: bufs[n] for n in vals})["y"].download() == want
