@@ -186,7 +186,8 @@ bool rising_edge(const sanic_program_desc* d, int node, const std::vector<int>& 
     return false;
 }
 
-bool flash_plan(const sanic_program_desc* d, int si, FlashPlan& P) {
+// The attention structure of a stage: carrier, dims and the affine K and V (any storage dtype).
+bool attention_plan(const sanic_program_desc* d, int si, FlashPlan& P) {
     const sanic_stage& st = d->stages[si];
     if (st.kind != SANIC_STAGE_FUSED || st.n_leaves != 2) return false;
     const sanic_carrier& c = st.carrier;
@@ -231,14 +232,15 @@ bool flash_plan(const sanic_program_desc* d, int si, FlashPlan& P) {
             qdims.push_back(j);
         }
     }
-    if (P.edim < 0 || qdims.size() != 2) return false;
-    // the head dim is the one the value leaf reads; the query row is read only by the score
+    if (P.edim < 0 || qdims.empty() || qdims.size() > 2) return false;
+    // the head dim (none for a single head) is the one the value leaf reads; the query row is
+    // read only by the score
     for (int j : qdims) {
         if (in_v[j]) P.hdim = j;
         else P.qdim = j;
     }
-    if (P.hdim < 0 || P.qdim < 0) return false;
-    P.NH = st.grid[P.hdim];
+    if (P.qdim < 0 || (P.hdim < 0) != (qdims.size() == 1)) return false;
+    P.NH = P.hdim < 0 ? 1 : st.grid[P.hdim];
     P.NQ = st.grid[P.qdim];
     P.E = st.grid[P.edim];
     P.T = st.stream;
@@ -254,9 +256,19 @@ bool flash_plan(const sanic_program_desc* d, int si, FlashPlan& P) {
         vcs[j] = b == SANIC_BIND_STREAM ? Sym::var(1) : b == P.hdim ? Sym::var(0) : b == P.edim ? Sym::var(2) : Sym();
     }
     if (!sym_access(d, st.leaf[P.vleaf], vcs, {P.NH, P.T, P.E}, P.vacc)) return false;
+    // a block's and a wave's key ranges are read off their first and last rows: every edge must
+    // not decrease with the row
+    for (auto& w : honest_window(d, st))
+        if (!rising_edge(d, w.node, w.bind, P.qdim)) return false;
+    return true;
+}
+
+bool flash_plan(const sanic_program_desc* d, int si, FlashPlan& P) {
+    if (!attention_plan(d, si, P)) return false;
+    const sanic_stage& st = d->stages[si];
     if ((!P.qexpr && P.qacc.dtype != SANIC_BF16) || P.kacc.dtype != SANIC_BF16 || P.vacc.dtype != SANIC_BF16) return false;
     if (P.HD != 64 || P.E != 64) return false;
-    P.ragged = P.NQ % 128 != 0 || P.T % 64 != 0;
+    P.ragged = P.NQ % 128 != 0 || P.T % 64 != 0 || P.hdim < 0;
     // Q: (h, d, i) with d contiguous; K: (⌊h/rep⌋, t, d) with d contiguous; V: (⌊h/rep⌋, t, e)
     std::vector<int64_t> qc, kc, vc;
     int qh, kh, vh;
@@ -269,12 +281,8 @@ bool flash_plan(const sanic_program_desc* d, int si, FlashPlan& P) {
     int repv = vh ? vh : (vc[0] ? 1 : (int)P.NH);
     if (repk != repv) return false;
     P.rep = repk;
-    // the block's and the wave's key ranges are read off their first and last rows: every edge
-    // must not decrease with the row
-    for (auto& w : honest_window(d, st))
-        if (!rising_edge(d, w.node, w.bind, P.qdim)) return false;
     if (P.ragged) {
-        // Lengths off the tiles go here only where the schedule is the backend's to choose and
+        // They go here only where the schedule is the backend's to choose and
         // the tile rows are whole 16-byte chunks of row-major K and V
         if (!sched_is_auto(st.sched) || vc[2] != 1) return false;
         for (int64_t v : {kc[0], kc[1], khc, P.kacc.addr.c0, vc[0], vc[1], vhc, P.vacc.addr.c0})
@@ -320,7 +328,7 @@ bool lower_flash_prefill(const sanic_program_desc* d, int si, int64_t& scratch, 
     const sanic_stage& st = d->stages[si];
     const sanic_carrier& c = st.carrier;
     const int64_t NH = P.NH, NQ = P.NQ, T = P.T, E = P.E, HD = P.HD;
-    // Lengths off the tiles (a prompt nobody padded) were folded in f32 by the generic fold: here
+    // Lengths off the tiles (a prompt nobody padded) and a single head were folded in f32 by the generic fold: here
     // the softmax weights, and a query side that is an expression, go to the MFMA as hi + lo bf16
     // pairs (16 significant bits), so they keep that precision at two MFMAs per fragment; one
     // query tile per wave holds the second operands in the registers the second tile had (115
@@ -380,7 +388,7 @@ bool lower_flash_prefill(const sanic_program_desc* d, int si, int64_t& scratch, 
     wc.indent = 1;
     Renderer Rw(d);
     std::vector<std::string> gcw(st.rank, "0");
-    gcw[P.hdim] = "hh";
+    if (P.hdim >= 0) gcw[P.hdim] = "hh";
     gcw[P.qdim] = "qrow";
     {
         Code tmp;
@@ -401,7 +409,7 @@ bool lower_flash_prefill(const sanic_program_desc* d, int si, int64_t& scratch, 
         std::string f = Ro.expr(fo, c.project, "", "", "", "fs");
         fo.line("const float fold_v = " + f + ";");
         std::vector<std::string> gc(st.rank, "0");
-        gc[P.hdim] = "hh";
+        if (P.hdim >= 0) gc[P.hdim] = "hh";
         gc[P.qdim] = "qi";
         gc[P.edim] = "ee";
         std::string v = "fold_v";
@@ -1067,7 +1075,7 @@ bool lower_flash_prefill(const sanic_program_desc* d, int si, int64_t& scratch, 
         k.line("  for (int p = 0; p < 16; ++p) {");
         k.indent += 2;
         std::vector<std::string> gc(st.rank, "0");
-        gc[P.hdim] = "hh";
+        if (P.hdim >= 0) gc[P.hdim] = "hh";
         gc[P.qdim] = "qi";
         gc[P.edim] = "(p / 4 * 16 + lq * 4 + p % 4)";
         for (int j = 0; j < st.rank; j++) k.line("const idx_t g" + std::to_string(j) + " = " + gc[j] + ";");
@@ -1094,6 +1102,215 @@ bool lower_flash_prefill(const sanic_program_desc* d, int si, int64_t& scratch, 
     std::vector<Arg> args = R.arg_list();
     if (SPL > 1) args.push_back({Arg::SCRATCH, soff});
     out.launches.push_back({kname, "", dim3((unsigned)(NB * SPL)), dim3(256), 0, args});
+    return true;
+}
+
+// ───────────────────────── float32 attention ───────────────────────────────────────────────
+// The same carrier with operands that bf16 MFMAs do not hold: f32 Q, K or V (bf16 ones beside
+// them widen on load), head sizes a multiple of 16, any lengths, f32 MFMAs (16x16x4) and expf
+// throughout, so nothing is narrower than the generic fold's arithmetic.
+//
+// One workgroup = one head × 16 query rows; its 8 waves take every 8th tile of 16 keys, each with
+// a running (m, ℓ, o) of its own, and merge in LDS by the carrier's combine in wave order. Sᵀ =
+// K·Qᵀ, so a lane owns one query column and its P values are the next MFMA's B operand as they
+// stand; K and V rows come straight from global memory (whole rows per 16 lanes), one tile ahead.
+// The bound is the f32 MFMA rate of a row block's CU (16 rows × 1024 keys × 64: 7 µs). S = 1024,
+// d = 64, causal: 1099 µs in the generic fold, which forms q·k for each of the 64 value columns.
+bool lower_flash_f32(const sanic_program_desc* d, int si, LoweredStage& out) {
+    FlashPlan P;
+    if (!attention_plan(d, si, P)) return false;
+    const sanic_stage& st = d->stages[si];
+    const sanic_carrier& c = st.carrier;
+    if (!sched_is_auto(st.sched) || P.qexpr) return false;
+    auto wide = [](int dt) { return dt == SANIC_F32 || dt == SANIC_BF16; };
+    if (!wide(P.qacc.dtype) || !wide(P.kacc.dtype) || !wide(P.vacc.dtype)) return false;
+    const int64_t NH = P.NH, NQ = P.NQ, T = P.T, E = P.E, HD = P.HD;
+    if (HD % 16 || E % 16 || HD > 128 || E > 128 || (E / 16 & (E / 16 - 1))) return false;
+    std::vector<int64_t> qc, kc, vc;
+    int qh, kh, vh;
+    int64_t qhc, khc, vhc;
+    if (!split_addr(P.qacc.addr, 4, qc, qh, qhc) || !split_addr(P.kacc.addr, 4, kc, kh, khc) || !split_addr(P.vacc.addr, 3, vc, vh, vhc)) return false;
+    if (qc[2] != 1 || qc[1] != 0 || kc[2] != 1 || kc[3] != 0 || vc[2] != 1) return false;
+    const int ET = (int)(E / 16), DS = (int)(HD / 4);      // value tiles; contraction steps
+    const int NWV = 8;
+    auto S = [](int64_t v) { return std::to_string(v); };
+
+    Renderer R(d), Rs(d), Ro(d), Rw(d);
+    auto win = honest_window(d, st);
+    const sanic_node& sl = d->nodes[st.leaf[P.sleaf]];
+    std::vector<std::string> lc(sl.rank);
+    for (int j = 0; j < sl.rank; j++) {
+        int b = st.bind[P.sleaf][j];
+        lc[j] = b == SANIC_BIND_STREAM ? "kj" : b == P.hdim && b >= 0 ? "hh" : b == P.qdim ? "qi" : "0";
+    }
+    Code sp, wc, fo, k;
+    sp.indent = wc.indent = fo.indent = k.indent = 1;
+    Rs.subst[P.dot_reduce] = "dotv";
+    const std::string vpart = Rs.value(sp, st.leaf[P.sleaf], lc);
+    for (int j = 0; j < st.rank; j++) wc.line("const idx_t g" + S(j) + " = " + (j == P.hdim ? "hh" : j == P.qdim ? "qrow" : "0") + ";");
+    emit_window(Rw, wc, st, win, "wlo", "whi");
+    std::vector<std::string> gc(st.rank, "0");
+    if (P.hdim >= 0) gc[P.hdim] = "hh";
+    gc[P.qdim] = "qi";
+    gc[P.edim] = "ee";
+    {
+        const std::string f = Ro.expr(fo, c.project, "", "", "", "fs");
+        fo.line("const float fold_v = " + f + ";");
+        std::string v = "fold_v";
+        if (st.epilogue >= 0) {
+            Ro.fold_var = "fold_v";
+            v = Ro.value(fo, st.epilogue, gc);
+        }
+        std::string lin;
+        for (int j = 0; j < st.rank; j++)
+            lin = j == 0 ? "(idx_t)(" + gc[0] + ")" : "(" + lin + " * " + S(st.grid[j]) + " + (idx_t)(" + gc[j] + "))";
+        fo.line(store_stmt(Ro.param(st.out_buffer), lin, st.out_dtype, v, false, d->buffers[st.out_buffer].scale));
+    }
+    for (Renderer* r : {&Rs, &Rw, &Ro})
+        for (int b : r->bufs) R.param(b);
+    auto base = [&](const Access& acc, const std::vector<int64_t>& cf, int div, int64_t hcf) {
+        const std::string h = div ? "(hh / " + S(div) + ") * " + S(hcf) : "hh * " + S(cf[0]);
+        return R.param(acc.buffer) + " + " + S(acc.addr.c0) + " + " + h;
+    };
+    // n consecutive elements at p as floats into x[0..n)
+    auto load = [&](const Access& acc, const std::string& p, int n, const std::string& x) {
+        if (acc.dtype == SANIC_F32) {
+            const int w = n % 4 == 0 ? 4 : n;      // 1, 2 or runs of 4
+            for (int i = 0; i < n; i += w) {
+                if (w == 1) { k.line(x + "[" + S(i) + "] = (" + p + ")[" + S(i) + "];"); continue; }
+                k.line("{ const sanic_f32x" + S(w) + "_any t_ = *(const sanic_f32x" + S(w) + "_any*)(" + p + " + " + S(i) + ");");
+                for (int j = 0; j < w; j++) k.line("  " + x + "[" + S(i + j) + "] = t_[" + S(j) + "];");
+                k.line("}");
+            }
+        } else {
+            for (int i = 0; i < n; i++) k.line(x + "[" + S(i) + "] = sanic_bf16((" + p + ")[" + S(i) + "]);");
+        }
+    };
+    const int64_t NQB = (NQ + 15) / 16;
+    k.line("__shared__ float o_lds[" + S(NWV) + "][" + S(E) + "][16], m_lds[" + S(NWV) + "][16], l_lds[" + S(NWV) + "][16];");
+    k.line("const int tid = threadIdx.x, lane = tid & 63, wv = __builtin_amdgcn_readfirstlane(tid >> 6);");
+    k.line("const int l16 = lane & 15, lq = lane >> 4;");
+    // the longest (last) row blocks first
+    k.line("const idx_t hh = blockIdx.x % " + S(NH) + ", q0 = (" + S(NQB - 1) + " - blockIdx.x / " + S(NH) + ") * 16;");
+    k.line("const idx_t qlast = q0 + 15 < " + S(NQ) + " ? q0 + 15 : (idx_t)" + S(NQ - 1) + ";");
+    k.line("idx_t alo, ahi, blo, bhi;");
+    k.line("window(a, hh, q0, alo, ahi);");
+    k.line("window(a, hh, qlast, blo, bhi);");
+    k.line("const int klo = __builtin_amdgcn_readfirstlane((int)(alo < blo ? alo : blo)) / 16 * 16, khi = __builtin_amdgcn_readfirstlane((int)(ahi > bhi ? ahi : bhi));");
+    k.line("const int qi = (int)(q0 + l16 < qlast ? q0 + l16 : qlast);");
+    // step s contracts d = lq·DS + s: a lane's operands of all steps are one contiguous run
+    k.line("float qv[" + S(DS) + "];");
+    load(P.qacc, "(" + base(P.qacc, qc, qh, qhc) + " + (idx_t)qi * " + S(qc[3]) + " + lq * " + S(DS) + ")", DS, "qv");
+    k.line("f32x4 o[" + S(ET) + "];");
+    for (int e = 0; e < ET; e++) k.line("o[" + S(e) + "] = (f32x4){0, 0, 0, 0};");
+    k.line("float m = -__builtin_huge_valf(), l = 0.0f;");
+    // K row of key t0 + l16 (run lq); V rows of keys t0 + lq·4 + r, values l16·ET .. + ET
+    k.line("auto fetch = [&](int t0, float (&kv)[" + S(DS) + "], float (&vv)[4][" + S(ET) + "]) {");
+    k.indent++;
+    k.line("const idx_t kt = t0 + l16 < " + S(T) + " ? t0 + l16 : " + S(T - 1) + ";");
+    load(P.kacc, "(" + base(P.kacc, kc, kh, khc) + " + kt * " + S(kc[1]) + " + lq * " + S(DS) + ")", DS, "kv");
+    for (int r = 0; r < 4; r++) {
+        k.line("const idx_t vt" + S(r) + " = t0 + lq * 4 + " + S(r) + " < " + S(T) + " ? t0 + lq * 4 + " + S(r) + " : " + S(T - 1) + ";");
+        load(P.vacc, "(" + base(P.vacc, vc, vh, vhc) + " + vt" + S(r) + " * " + S(vc[1]) + " + l16 * " + S(ET) + ")", ET, "vv[" + S(r) + "]");
+    }
+    k.indent--;
+    k.line("};");
+    k.line("auto fold = [&](int t0, float (&kv)[" + S(DS) + "], float (&vv)[4][" + S(ET) + "]) {");
+    k.indent++;
+    k.line("f32x4 s0 = (f32x4){0, 0, 0, 0}, s1 = (f32x4){0, 0, 0, 0};");
+    for (int s = 0; s < DS; s++)
+        k.line(std::string(s % 2 ? "s1" : "s0") + " = __builtin_amdgcn_mfma_f32_16x16x4f32(kv[" + S(s) + "], qv[" + S(s) + "], " + (s % 2 ? "s1" : "s0") + ", 0, 0, 0);");
+    k.line("float sv[4], p[4];");
+    k.line("#pragma unroll");
+    k.line("for (int r = 0; r < 4; ++r) {");
+    k.line("  const int kj = t0 + lq * 4 + r;");
+    k.line("  const float x = score(a, s0[r] + s1[r], (int)hh, qi, kj < " + S(T) + " ? kj : " + S(T - 1) + ");");
+    k.line("  sv[r] = kj < " + S(T) + " ? x : -__builtin_huge_valf();");
+    k.line("}");
+    k.line("const float mt = sanic_rows_max(fmaxf(fmaxf(sv[0], sv[1]), fmaxf(sv[2], sv[3])));");
+    k.line("const float mn = fmaxf(m, mt);");
+    // the carrier's guarded rescale: a side whose max is −∞ weighs 0
+    k.line("const float alpha = m == -__builtin_huge_valf() ? 0.0f : expf(m - mn);");
+    k.line("#pragma unroll");
+    k.line("for (int r = 0; r < 4; ++r) p[r] = sv[r] == -__builtin_huge_valf() ? 0.0f : expf(sv[r] - mn);");
+    k.line("m = mn;");
+    k.line("l = l * alpha + ((p[0] + p[1]) + (p[2] + p[3]));");
+    for (int e = 0; e < ET; e++) k.line("o[" + S(e) + "] *= alpha;");
+    for (int r = 0; r < 4; r++)
+        for (int e = 0; e < ET; e++)
+            k.line("o[" + S(e) + "] = __builtin_amdgcn_mfma_f32_16x16x4f32(vv[" + S(r) + "][" + S(e) + "], p[" + S(r) + "], o[" + S(e) + "], 0, 0, 0);");
+    k.indent--;
+    k.line("};");
+    k.line("float ka[" + S(DS) + "], kb[" + S(DS) + "], va[4][" + S(ET) + "], vb[4][" + S(ET) + "];");
+    const std::string step = S(16 * NWV);
+    k.line("int t = klo + wv * 16;");
+    k.line("if (t < khi) fetch(t, ka, va);");
+    k.line("for (; t < khi; t += 2 * " + step + ") {");
+    k.line("  if (t + " + step + " < khi) fetch(t + " + step + ", kb, vb);");
+    k.line("  fold(t, ka, va);");
+    k.line("  if (t + " + step + " >= khi) break;");
+    k.line("  if (t + 2 * " + step + " < khi) fetch(t + 2 * " + step + ", ka, va);");
+    k.line("  fold(t + " + step + ", kb, vb);");
+    k.line("}");
+    k.line("l = sanic_rows_sum(l);");
+    k.line("if (lane < 16) { m_lds[wv][lane] = m; l_lds[wv][lane] = l; }");
+    for (int e = 0; e < ET; e++)
+        for (int r = 0; r < 4; r++) k.line("o_lds[wv][(lq * 4 + " + S(r) + ") * " + S(ET) + " + " + S(e) + "][l16] = o[" + S(e) + "][" + S(r) + "];");
+    k.line("__syncthreads();");
+    k.line("for (int p = tid; p < " + S(16 * E) + "; p += " + S(64 * NWV) + ") {");
+    k.indent++;
+    k.line("const int ee = p % " + S(E) + ", row = p / " + S(E) + ";");
+    k.line("const idx_t qi = q0 + row;");
+    k.line("if (qi >= " + S(NQ) + ") continue;");
+    k.line("float M = m_lds[0][row];");
+    for (int w = 1; w < NWV; w++) k.line("M = fmaxf(M, m_lds[" + S(w) + "][row]);");
+    k.line("float L = 0.0f, O = 0.0f;");
+    k.line("#pragma unroll");
+    k.line("for (int w = 0; w < " + S(NWV) + "; ++w) {");
+    k.line("  const float mw = m_lds[w][row], x = mw == -__builtin_huge_valf() ? 0.0f : expf(mw - M);");
+    k.line("  L = fmaf(x, l_lds[w][row], L);");
+    k.line("  O = fmaf(x, o_lds[w][ee][row], O);");
+    k.line("}");
+    k.line("float fs" + S(P.max_slot) + " = M;");
+    for (size_t s = 0; s < P.scalar_slots.size(); s++) k.line("float fs" + S(P.scalar_slots[s]) + " = " + flit(P.scalar_into[s]) + " * L;");
+    k.line("float fs" + S(P.vec_slots[0]) + " = O;");
+    // Infinities and NaNs: a masked key weighs 0 here, and 0 · ∞ is not what the fold over the
+    // honest window gives; such a point is folded again
+    k.line("if (!(__builtin_fabsf(O) <= 3.402823466e38f) || !(__builtin_fabsf(L) <= 3.402823466e38f) || !(__builtin_fabsf(M) <= 3.402823466e38f)) {");
+    k.indent++;
+    {
+        std::vector<std::string> g = gc;
+        for (int j = 0; j < st.rank; j++) k.line("const idx_t g" + S(j) + " = " + g[j] + ";");
+        emit_point_fold(R, k, st, "pf");
+        for (int s = 0; s < c.slots; s++) k.line("fs" + S(s) + " = pf" + S(s) + ";");
+    }
+    k.indent--;
+    k.line("}");
+    std::string fargs;
+    for (int s = 0; s < c.slots; s++) fargs += ", fs" + S(s);
+    k.line("finish(a, hh, qi, ee" + fargs + ");");
+    k.indent--;
+    k.line("}");
+
+    const std::string kname = "sanic_attn32_h" + S(NH) + "_s" + S(NQ) + "_t" + S(T);
+    std::ostringstream src;
+    src << kPrelude;
+    src << "typedef __attribute__((__vector_size__(4 * sizeof(float)))) float f32x4;\n";
+    src << "typedef float sanic_f32x4_any __attribute__((ext_vector_type(4), aligned(4)));\n";
+    src << "typedef float sanic_f32x2_any __attribute__((ext_vector_type(2), aligned(4)));\n";
+    src << R.args_struct({});
+    src << "__device__ __forceinline__ float score(const Args& a, float dotv, int hh, int qi, int kj) {\n"
+        << Rs.entry() << sp.str() << "  return " << vpart << ";\n}\n";
+    src << "__device__ __forceinline__ void window(const Args& a, idx_t hh, idx_t qrow, idx_t& lo, idx_t& hi) {\n"
+        << Rw.entry() << wc.str() << "  lo = wlo; hi = whi;\n}\n";
+    src << "__device__ __forceinline__ void finish(const Args& a, idx_t hh, idx_t qi, idx_t ee";
+    for (int s = 0; s < c.slots; s++) src << ", float fs" << s;
+    src << ") {\n" << Ro.entry() << fo.str() << "}\n";
+    src << "extern \"C\" __global__ void __launch_bounds__(" << 64 * NWV << ") " << kname << "(Args a) {\n" << R.entry() << k.str() << "}\n";
+    out.kernel_kind = "skeleton:attn_f32[d " + S(HD) + "]";
+    out.source = src.str();
+    out.variants = 1;
+    out.launches.push_back({kname, "", dim3((unsigned)(NH * NQB)), dim3(64 * NWV), 0, R.arg_list()});
     return true;
 }
 

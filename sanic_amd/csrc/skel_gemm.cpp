@@ -314,13 +314,15 @@ bool lower_gemm(const sanic_program_desc* d, int si, int64_t& scratch, LoweredSt
     if (rag && splitB) return false;             // a rebuilt weight has more than 16 bits
     // grouped tiles: tiling variants {8 waves, load depth 4; 4 waves, depth 4; 8 waves, depth 2}
     const int gvar = grouped && st.sched.variant > 0 && st.sched.variant < 3 ? st.sched.variant : 0;
-    if (grouped && BM == 128 && BN == 32 && gvar != 1) NTH = 512;
     // A operands that need arithmetic (x·g of the fused RMSNorm) are built once by a first
     // launch into bf16 hi/lo planes [M][K] (plus the row slots), instead of by every one of the
     // N/BN column workgroups
     const bool pre = splitA && N / BN >= 4 && (rag ? NKT >= 2 : K % 512 == 0);
-    int DEPTH = grouped ? (gvar == 2 ? 2 : 4) : 2;
-    if (!grouped && st.sched.variant == 1) DEPTH = 4;
+    // (64 × 32 tiles with fragment-loaded A: 4, K = 2048, N = 8192, M = 64 16.9 → 14.6 µs; larger
+    // tiles 2, M = 128 22.5 against 23.4, M = 512 38.2 against 39.4)
+    const int other = pre && BM == 64 && BN == 32 ? 4 : 2;
+    int DEPTH = grouped ? (gvar == 2 ? 2 : 4) : other;
+    if (!grouped && st.sched.variant == 1) DEPTH = 6 - other;
     if ((!rag && NKT % DEPTH) || NKT < 2 * DEPTH) DEPTH = 2;
     // (off the tiles the unrolled steps past the last K tile are skipped)
     const bool deep = rag ? NKT >= DEPTH : NKT % DEPTH == 0 && NKT >= 2 * DEPTH;
@@ -332,6 +334,12 @@ bool lower_gemm(const sanic_program_desc* d, int si, int64_t& scratch, LoweredSt
     // both load them; the second from L1)
     const bool adirect = pre && deep && !getenv("SANIC_HIP_GEMM_ALDS");
     if (rag && pre && !adirect) return false;
+    if (grouped && BM == 128 && BN == 32 && gvar != 1) NTH = 512;
+    // fragment-loaded A: every wave its own 16 rows of the block and all its columns, so that no A
+    // fragment is loaded twice — a CU takes in ≈ 30 bytes a clock that miss L1, and A is most of
+    // them (4 waves 2 × 2 → 8 × 1: K = 2048, N = 8192, M = 128 27.1 → 22.5 µs; 4 × 1 for 64 rows:
+    // M = 64 18.4 → 16.9 µs)
+    if (adirect && BM == 128) NTH = 512;
     // element offset of (row, k) in a plane: row-major, or fragment order (k a multiple of 8)
     auto plane_off = [&](const std::string& row, const std::string& k8) {
         if (!adirect) return "(" + row + ") * " + std::to_string(K) + " + " + k8;
@@ -340,7 +348,7 @@ bool lower_gemm(const sanic_program_desc* d, int si, int64_t& scratch, LoweredSt
     // waves along m and n: 4 × 2 / 2 × 2; grouped 32-column tiles of 8 waves 8 × 1, so no two
     // waves form the same rows' Σ x; 8 × 1 also for fragment-loaded A (each wave its own rows,
     // so no A fragment is loaded twice: B2 45.9 → 42.9 µs against 4 × 2)
-    const int WGN = ((grouped && NTH == 512 && BN == 32 && BM == 128) || (adirect && NTH == 512 && BM == 128)) ? 1 : 2;
+    const int WGN = adirect || (grouped && NTH == 512 && BN == 32 && BM == 128) ? 1 : 2;
     const int WGM = NTH / 64 / WGN;
     const int WM = BM / WGM, WN = BN / WGN;   // per-wave tile
     const int MT = WM / 16, NT = WN / 16;

@@ -153,16 +153,16 @@ bool lower_skinny(const sanic_program_desc* d, int si, LoweredStage& out) {
     const int NT = BN / 16;
     // Rounds of workgroups over the 256 CUs against the GEMM's (lower_gemm's tiles), in µs at the
     // measured cost of each (K = 2048, N = 8192): a round here 9.5 at 32 rows and 5 at 16, a
-    // quarter more for a [K, N] weight; a 64-deep K step of a GEMM tile 0.42 (64 × 32), 0.7 (128 × 32 and
-    // 128 × 64), 1.05 (128 × 128), and 5 for its operand launch. Up to 32 rows the GEMM's tile is
-    // half empty (M = 32: 13.4 here, 19.0 there); M = 48: 22.5 and 18.8; N = 1088, K = 1968: M = 200
+    // quarter more for a [K, N] weight; a 64-deep K step of a GEMM tile 0.3 (64 × 32), 0.55 (128 × 32),
+    // 0.68 (128 × 64), 1.05 (128 × 128), and 5 for its operand launch. Up to 32 rows the GEMM's tile is
+    // half empty (M = 32: 13.4 here, 15.0 there); M = 48: 22.5 and 15.0; N = 1088, K = 1968: M = 200
     // 13.8 and 33.7, M = 400 24.5 and 35.9.
     if (M > 32) {
         const double here = 3.0 + (double)((NMB * NNB + 255) / 256) * ((double)K / 2048.0) * (MT > 1 ? 9.5 : 5.0) * (kn ? 1.25 : 1.0);
         const int64_t bm = M > 64 ? 128 : 64, mb = (M + bm - 1) / bm;
         int64_t bn = 128;
         while (bn > 32 && mb * (N / bn) < 256) bn /= 2;
-        const double step = bn == 128 ? 1.05 : bm == 64 && bn == 32 ? 0.42 : 0.7;
+        const double step = bn == 128 ? 1.05 : bn == 64 ? 0.68 : bm == 64 ? 0.3 : 0.55;
         const double there = (split ? 5.0 : 0.0) + (double)((mb * ((N + bn - 1) / bn) + 255) / 256) * (double)((K + 63) / 64) * step;
         if (N >= bn && there < here) return false;
     }

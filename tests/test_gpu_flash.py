@@ -110,6 +110,8 @@ def test_flash_head_groupings(dev, NH, NKV):
     (4, 2, 200, 100),     # a window ending inside a tile
     (2, 1, 321, 70),
     (6, 2, 512 + 64, 0),  # whole key tiles, rows not a multiple of 128
+    (1, 1, 256, 0),       # a single head: no head dim in the grid
+    (1, 1, 100, 30),
 ])
 def test_flash_any_length(dev, monkeypatch, NH, NKV, S, window):
     """Lengths off the tiles against the generic f32 fold of the same program: the skeleton keeps
@@ -153,3 +155,60 @@ def test_flash_any_length_keeps_infinities_and_nans(dev, monkeypatch):
     assert np.array_equal(np.isnan(g), np.isnan(w)) and np.array_equal(np.isinf(g), np.isinf(w))
     fin = np.isfinite(w)
     assert np.max(np.abs(g[fin] - w[fin]) - 2.0 ** -7 * np.abs(w[fin])) < 1e-4
+
+
+def _attention_f32(NH, NKV, NQ, T, HD, E, causal, dtypes):
+    """softmax(q·kᵀ/√HD + mask)·v with f32 output; NH = 0: no head dim."""
+    from sanic_amd import carrier as C
+    from sanic_amd.program import STREAM, Program
+    p = Program()
+    lead, klead = ((NH,), (NKV,)) if NH else ((), ())
+    q, k, v = (p.input(n, shp, dt) for n, shp, dt in zip("QKV", (lead + (NQ, HD), klead + (T, HD), klead + (T, E)), dtypes))
+    if NH:
+        k, v = ir.expand_heads(k, 0, NH // NKV), ir.expand_heads(v, 0, NH // NKV)
+        s = ir.reduce(ir.map_(ir.MUL, ir.unsqueeze(q, 2), ir.unsqueeze(k, 1)), 3, ir.M_ADD)
+    else:
+        s = ir.matmul(q, ir.transpose(k, 0, 1))
+    s = ir.map_(ir.MUL, s, ir.const(HD ** -0.5))
+    h = len(lead)
+    if causal:
+        s = ir.map_(ir.ADD, s, ir.causal_mask_like(s, h, h + 1))
+    sb, vb = ((0, 1, STREAM), (0, STREAM, 2)) if NH else ((0, STREAM), (STREAM, 1))
+    p.fused("O", lead + (NQ, E), T, [(s, sb), (v, vb)], C.online_softmax_weighted(), ir.F32)
+    return p
+
+
+F, B = ir.F32, ir.BF16
+
+
+@pytest.mark.parametrize("NH,NKV,NQ,T,HD,E,causal,dtypes", [
+    (0, 0, 128, 128, 64, 64, True, (F, F, F)),
+    (0, 0, 33, 33, 32, 32, True, (F, F, F)),      # one row into a third block
+    (0, 0, 1000, 1000, 64, 64, True, (F, F, F)),
+    (0, 0, 17, 300, 16, 128, False, (F, F, F)),   # more keys than rows, value tiles of 8
+    (6, 2, 50, 50, 128, 16, True, (F, F, F)),     # grouped heads, d above the value size
+    (4, 4, 20, 5, 48, 32, False, (B, F, B)),      # fewer keys than a tile, stored types mixed
+])
+def test_attention_f32_matches_generic(dev, monkeypatch, NH, NKV, NQ, T, HD, E, causal, dtypes):
+    """Both evaluations are f32 throughout: scores within HD · 2^-24 of Σ|q·k| ≤ HD of each other,
+    so the weights and outputs (|v| ≲ 4) within a few 1e-5 at most; and infinities and NaNs in the
+    keys and values that some rows do not see sit at the same points."""
+    prog = _attention_f32(NH, NKV, NQ, T, HD, E, causal, dtypes)
+    vals = {n: oracle.synth(500 + i, int(np.prod(prog.by_name[n].shape)), dtype=prog.by_name[n].dtype).reshape(prog.by_name[n].shape)
+            for i, n in enumerate("QKV")}
+    for odd in (False, True):
+        if odd:
+            vals["V"][..., T - 1, 0] = np.nan
+            vals["K"][..., T // 2, 1] = np.inf
+        got, exe = run_on_gpu(dev, prog, vals)
+        assert exe.stage_kernel(0).startswith("skeleton:attn_f32"), exe.stage_kernel(0)
+        monkeypatch.setenv("SANIC_HIP_GENERIC", "1")
+        want, _ = run_on_gpu(dev, prog, vals)
+        monkeypatch.delenv("SANIC_HIP_GENERIC")
+        g, w = got["O"], want["O"]
+        fin = np.isfinite(w)
+        assert np.array_equal(np.isnan(g), np.isnan(w)) and np.array_equal(fin, np.isfinite(g))
+        if fin.any():
+            err = max_rel_err(g[fin], w[fin])
+            print(odd, err)
+            assert err < 2e-5
