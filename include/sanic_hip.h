@@ -299,8 +299,8 @@ int sanic_hip_execute(sanic_hip_exe* exe, sanic_hip_buffer* const* bindings, int
  * arena live in the library's static device scratch — 32 MiB per GPU, held until the process
  * ends; a program that needs more is refused with SANIC_ERR_ARG. The stages are enqueued on the
  * device's stream and the call returns without waiting (a download on the same buffers waits).
- * Every call on one GPU shares that scratch; the arena's counters are cleared at the start of
- * each call, its other contents are whatever the last call left. Eager calls are ordered per GPU:
+ * Every call on one GPU shares that scratch; the arrival counters (apart from it) are zero between
+ * calls, its other contents are whatever the last call left. Eager calls are ordered per GPU:
  * each waits for the previous eager call's work on that GPU, whichever device handle (stream)
  * made it. A call made while the device's stream is being captured into a HIP graph is not
  * ordered that way: replays of such a graph that overlap other calls on the GPU race on the

@@ -188,6 +188,11 @@ class Executable:
         self.dev = dev
         self.prog = prog
         self.handle = handle
+        n = len(prog.buffers)
+        self._array = VP * n
+        self._index = {b.name: b.index for b in prog.buffers}
+        self._outputs = [b.index for b in prog.buffers if b.role == OUTPUT]
+        self._run_static = abi.lib().sanic_hip_execute_static
 
     def stage_kernel(self, i: int) -> str:
         buf = ctypes.create_string_buffer(256)
@@ -200,13 +205,14 @@ class Executable:
         return buf.value.decode()
 
     def _bindings(self, bindings: Dict[str, Buffer]):
-        arr = (VP * len(self.prog.buffers))()
-        for b in self.prog.buffers:
-            if b.name in bindings:
-                arr[b.index] = bindings[b.name].handle
-        unknown = set(bindings) - set(self.prog.by_name)
-        if unknown:
-            raise KeyError(f"unknown bindings {sorted(unknown)} (RunError::UnknownInput)")
+        arr = self._array()
+        index = self._index
+        try:
+            for name, b in bindings.items():
+                arr[index[name]] = b.handle
+        except KeyError:
+            unknown = set(bindings) - set(index)
+            raise KeyError(f"unknown bindings {sorted(unknown)} (RunError::UnknownInput)") from None
         return arr
 
     def execute(self, bindings: Dict[str, Buffer]) -> Dict[str, Buffer]:
@@ -224,11 +230,15 @@ class Executable:
         """sanic_hip_execute_static: run once with no device allocation — `bindings` holds the
         caller's buffers for every INPUT, STATE and OUTPUT buffer; intermediates and the
         split/counter arena use the library's static scratch. Returns without waiting."""
-        missing = [b.name for b in self.prog.buffers if b.role == OUTPUT and b.name not in bindings]
-        if missing:
-            raise KeyError(f"outputs must be bound: {missing}")
         arr = self._bindings(bindings)
-        abi.check(abi.lib().sanic_hip_execute_static(self.handle, arr, len(self.prog.buffers)))
+        for i in self._outputs:
+            if not arr[i]:
+                missing = [b.name for b in self.prog.buffers if b.role == OUTPUT and b.name not in bindings]
+                if missing:
+                    raise KeyError(f"outputs must be bound: {missing}")
+        status = self._run_static(self.handle, arr, len(arr))
+        if status:
+            abi.check(status)
 
     def capture(self, bindings: Dict[str, Buffer], feedback: Sequence = ()) -> "Replay":
         """Program::capture: freeze the bindings into one hipGraph; `feedback` pairs

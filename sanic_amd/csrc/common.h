@@ -33,9 +33,9 @@ void set_last_error(const std::string& s);
 [[noreturn]] inline void fail(int code, const std::string& m) { throw Error(code, m); }
 
 // One kernel argument: a program buffer's device address, a byte offset into the executable's
-// scratch arena, or an immediate 64-bit value.
+// scratch arena or its arrival counters, or an immediate 64-bit value.
 struct Arg {
-    enum Kind { BUF, SCRATCH, IMM } kind;
+    enum Kind { BUF, SCRATCH, COUNTERS, IMM } kind;
     int64_t v;
 };
 
@@ -47,8 +47,6 @@ struct Launch {
     uint32_t lds = 0;          // dynamic LDS bytes
     std::vector<Arg> args;
     hipFunction_t fn = nullptr;
-    bool zero_scratch = false; // clear `zero_bytes` of scratch at zero_off before this launch
-    int64_t zero_off = 0, zero_bytes = 0;
 };
 
 // A stage lowered onto one or more launches.
@@ -62,6 +60,9 @@ struct LoweredStage {
 struct Lowered {
     std::vector<LoweredStage> stages;
     int64_t scratch_bytes = 0;
+    // arrival counters, apart from the arena: zero before a program's first launch, and every
+    // kernel leaves those it used at zero
+    int64_t counter_bytes = 0;
 };
 
 // Validate a descriptor and lower every stage (emit_hip.cpp).

@@ -68,6 +68,9 @@ int64_t dtype_bytes(int dt, int64_t n);
 // Fold the whole stream at grid point g0, g1, ... one element after another (the scalar generic
 // fold's arithmetic); slot k's accumulator is `acc`<k>.
 void emit_point_fold(Renderer& R, Code& code, const sanic_stage& st, const std::string& acc);
+// `n` arrival counters of the program being lowered on this thread: their byte offset from the
+// program's first (a kernel argument Arg::COUNTERS).
+int64_t take_counters(int64_t n);
 // Last-arriver handshake: the workgroups sharing counter `cnt` each add 1 once their partials
 // are stored; `flag` (a __shared__ int it declares) is true in the one that arrives last.
 // With xcd_local every workgroup sharing `cnt` runs on one XCD and exchanges data through

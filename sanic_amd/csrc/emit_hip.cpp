@@ -50,6 +50,13 @@ static std::atomic<bool> g_xcd_local{true};
 void set_xcd_local(bool on) { g_xcd_local.store(on, std::memory_order_relaxed); }
 bool xcd_local_enabled() { return g_xcd_local.load(std::memory_order_relaxed) && !getenv("SANIC_HIP_AGENT_MERGE"); }
 
+static thread_local int64_t t_counter_bytes = 0;
+int64_t take_counters(int64_t n) {
+    const int64_t at = t_counter_bytes;
+    t_counter_bytes += (n * 4 + 255) / 256 * 256;
+    return at;
+}
+
 void emit_arrival(Code& k, const std::string& flag, const std::string& tid, const std::string& cnt,
                   const std::string& expected, bool xcd_local) {
     k.line("__shared__ int " + flag + ";");
@@ -1183,7 +1190,7 @@ LoweredStage lower_generic_fold(const sanic_program_desc* d, int si, int64_t& sc
     int64_t part_off = scratch;
     const bool fused_merge = split > 1 && gvol <= 4096;
     const int64_t part_bytes = ((gvol * split * c.slots * 4 + 255) / 256) * 256;
-    if (split > 1) scratch += part_bytes + (fused_merge ? 256 : 0);
+    if (split > 1) scratch += part_bytes;
     body.line("const idx_t gid = (idx_t)blockIdx.x / " + std::to_string(split) + ";");
     body.line("const int part = (int)(blockIdx.x % " + std::to_string(split) + ");");
     body.line("const int t = threadIdx.x, lane = t & 63, wv = t >> 6;");
@@ -1276,7 +1283,7 @@ LoweredStage lower_generic_fold(const sanic_program_desc* d, int si, int64_t& sc
     };
     if (fused_merge) {
         body.line("}");
-        body.line("unsigned* cnt = (unsigned*)((char*)a.scratch + " + std::to_string(part_bytes) + ");");
+        body.line("unsigned* cnt = a.counters;");
         emit_arrival(body, "sanic_last", "t", "cnt", "gridDim.x");
         body.line("if (!sanic_last) return;");
         // Few output points: L = split rounded up to a power of two lanes per point load one
@@ -1342,10 +1349,11 @@ LoweredStage lower_generic_fold(const sanic_program_desc* d, int si, int64_t& sc
             emit_pointwise_loop(R, body, d, ts, "(idx_t)t", nth);
         }
         body.line("if (t == 0) sanic_st(cnt, 0u);");
-        src << R.args_struct({"float* __restrict__ scratch"});
+        src << R.args_struct({"float* __restrict__ scratch", "unsigned* counters"});
         src << "extern \"C\" __global__ void __launch_bounds__(" << nth << ") sanic_fold_split(Args a) {\n" << R.entry() << body.str() << "}\n";
         std::vector<Arg> args = R.arg_list();
         args.push_back({Arg::SCRATCH, part_off});
+        args.push_back({Arg::COUNTERS, take_counters(1)});
         L.launches.push_back({"sanic_fold_split", "", dim3((unsigned)(gvol * split)), dim3(nth), 0, args});
         L.kernel_kind = "fold:split+merge" + auto_tag + std::string(tails.empty() ? "" : "+tail" + std::to_string(tails.size()));
         L.source = src.str();
@@ -1491,6 +1499,7 @@ static bool stage_touches_q8(const sanic_program_desc* d, int s) {
 Lowered lower_program(const sanic_program_desc* d) {
     validate(d);
     Lowered out;
+    t_counter_bytes = 0;
     for (int s = 0; s < d->n_stages;) {
         const sanic_stage& st = d->stages[s];
         // skeletons may batch or absorb the next few stages: none of them may touch Q8 either
@@ -1545,6 +1554,7 @@ Lowered lower_program(const sanic_program_desc* d) {
         }
         s++;
     }
+    out.counter_bytes = t_counter_bytes;
     return out;
 }
 

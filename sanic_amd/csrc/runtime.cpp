@@ -30,7 +30,8 @@ struct sanic_hip_device {
     int ordinal = 0;
     hipStream_t stream = nullptr;
     hipDeviceProp_t props{};
-    char* scratch_ptr = nullptr;   // this GPU's copy of `scratch` (execute_static)
+    char* scratch_ptr = nullptr;   // this GPU's copies of `scratch` and `counters` (execute_static)
+    char* counters_ptr = nullptr;
 };
 
 // ── the static scratch of sanic_hip_execute_static ─────────────────────────────────────────
@@ -42,6 +43,11 @@ struct sanic_hip_device {
 // (sanic_hip_device::scratch_ptr, taken in sanic_hip_open with the device current).
 static const size_t kStaticScratchBytes = size_t(32) << 20;
 static __device__ __align__(256) char scratch[kStaticScratchBytes];
+// The arrival counters of that entry point's programs, apart from the scratch so that no
+// program's data lies on them: zero at load, and every kernel leaves those it used at zero, so a
+// call clears nothing (a program with more of them takes them from the scratch and clears them).
+static const size_t kStaticCounterBytes = size_t(64) << 10;
+static __device__ __align__(256) unsigned counters[kStaticCounterBytes / 4];
 
 // Which XCD each workgroup of a launch runs on (the hardware register XCC_ID): kernels that let
 // the workgroups sharing an arrival counter exchange partials through one XCD's L2 rely on the
@@ -74,12 +80,19 @@ static bool probe_xcd_round_robin(hipStream_t stream, char* dev_buf) {
     return true;
 }
 
-// One event per GPU marking the end of the last sanic_hip_execute_static call's work on that
-// GPU. Each call makes its stream wait on it before touching the scratch and records it after
-// enqueueing, so calls from different device handles (each with its own stream) on one GPU are
-// ordered instead of racing on the shared scratch. Created once per ordinal in sanic_hip_open.
+// The order of sanic_hip_execute_static calls on one GPU: the stream that ran the last one. A call
+// on the same stream is ordered by it; a call on another device handle's stream waits for an event
+// recorded on the last one first, so calls are ordered instead of racing on the shared scratch. The
+// mutex is held while a call is enqueued. `marked`: the event already stands behind everything the
+// last stream was given (recorded ahead of a capture of that stream, which could not take it).
+// Created once per ordinal in sanic_hip_open.
+struct StaticOrder {
+    hipEvent_t done = nullptr;
+    hipStream_t last = nullptr;
+    bool marked = false;
+};
 static std::mutex g_static_mu;
-static std::map<int, hipEvent_t> g_static_done;
+static std::map<int, StaticOrder> g_static;
 
 struct Storage {
     void* ptr = nullptr;
@@ -257,33 +270,32 @@ static void compile_all(sanic_hip_exe* exe, bool load) {
 }
 
 // Enqueue every stage's launches on the device stream. `bound[i]` is program buffer i.
-static void enqueue(sanic_hip_exe* exe, const std::vector<sanic_hip_buffer*>& bound, char* arena,
-                    hipEvent_t* stage_events = nullptr) {
+static void enqueue(sanic_hip_exe* exe, char* const* bound, char* arena, char* counts, hipEvent_t* stage_events = nullptr) {
     hipStream_t s = exe->dev->stream;
+    uint64_t kargs[64];
     for (size_t si = 0; si < exe->low.stages.size(); si++) {
         if (stage_events) SANIC_HIP(hipEventRecord(stage_events[si], s));
         for (auto& l : exe->low.stages[si].launches) {
-            if (l.zero_scratch && l.zero_bytes > 0) {
-                int64_t words = l.zero_bytes / 4;
-                unsigned blocks = (unsigned)std::min<int64_t>((words + 255) / 256, 4096);
-                hipLaunchKernelGGL(sanic_zero_words, dim3(blocks), dim3(256), 0, s, (uint32_t*)(arena + l.zero_off), words);
-                SANIC_HIP(hipGetLastError());
+            std::vector<uint64_t> many;
+            uint64_t* ka = kargs;
+            if (l.args.size() > 64) {
+                many.resize(l.args.size());
+                ka = many.data();
             }
-            std::vector<uint64_t> kargs;
+            size_t na = 0;
             for (auto& a : l.args) {
                 switch (a.kind) {
-                case Arg::BUF: {
-                    sanic_hip_buffer* b = bound[a.v];
-                    if (!b) fail(SANIC_ERR_MISSING_INPUT, "buffer " + std::to_string(a.v) + " is not bound");
-                    kargs.push_back((uint64_t)(uintptr_t)b->ptr());
+                case Arg::BUF:
+                    if (!bound[a.v]) fail(SANIC_ERR_MISSING_INPUT, "buffer " + std::to_string(a.v) + " is not bound");
+                    ka[na++] = (uint64_t)(uintptr_t)bound[a.v];
                     break;
-                }
-                case Arg::SCRATCH: kargs.push_back((uint64_t)(uintptr_t)(arena + a.v)); break;
-                case Arg::IMM: kargs.push_back((uint64_t)a.v); break;
+                case Arg::SCRATCH: ka[na++] = (uint64_t)(uintptr_t)(arena + a.v); break;
+                case Arg::COUNTERS: ka[na++] = (uint64_t)(uintptr_t)(counts + a.v); break;
+                case Arg::IMM: ka[na++] = (uint64_t)a.v; break;
                 }
             }
-            size_t sz = kargs.size() * 8;
-            void* cfg[] = {HIP_LAUNCH_PARAM_BUFFER_POINTER, kargs.data(), HIP_LAUNCH_PARAM_BUFFER_SIZE, &sz,
+            size_t sz = na * 8;
+            void* cfg[] = {HIP_LAUNCH_PARAM_BUFFER_POINTER, ka, HIP_LAUNCH_PARAM_BUFFER_SIZE, &sz,
                            HIP_LAUNCH_PARAM_END};
             SANIC_HIP(hipModuleLaunchKernel(l.fn, l.grid.x, l.grid.y, l.grid.z, l.block.x, l.block.y, l.block.z,
                                             l.lds, s, nullptr, cfg));
@@ -381,9 +393,17 @@ int sanic_hip_open(int ordinal, sanic_hip_device** out) {
             fail(SANIC_ERR_BACKEND, std::string("hipGetSymbolAddress(scratch): ") + hipGetErrorString(se));
         }
         d->scratch_ptr = (char*)sp;
+        void* cp = nullptr;
+        se = hipGetSymbolAddress(&cp, HIP_SYMBOL(counters));
+        if (se != hipSuccess || !cp) {
+            hipStreamDestroy(d->stream);
+            delete d;
+            fail(SANIC_ERR_BACKEND, std::string("hipGetSymbolAddress(counters): ") + hipGetErrorString(se));
+        }
+        d->counters_ptr = (char*)cp;
         {
             std::lock_guard<std::mutex> lk(g_static_mu);
-            if (!g_static_done.count(ordinal)) {
+            if (!g_static.count(ordinal)) {
                 hipEvent_t ev = nullptr;
                 hipError_t ee = hipEventCreateWithFlags(&ev, hipEventDisableTiming);
                 if (ee != hipSuccess) {
@@ -391,7 +411,7 @@ int sanic_hip_open(int ordinal, sanic_hip_device** out) {
                     delete d;
                     fail(SANIC_ERR_BACKEND, std::string("hipEventCreateWithFlags: ") + hipGetErrorString(ee));
                 }
-                g_static_done[ordinal] = ev;
+                g_static[ordinal].done = ev;
                 // first open of this GPU: nothing has used its static scratch yet
                 if (!probe_xcd_round_robin(d->stream, d->scratch_ptr)) set_xcd_local(false);
             }
@@ -405,6 +425,12 @@ void sanic_hip_close(sanic_hip_device* dev) {
     hipSetDevice(dev->ordinal);
     if (dev->stream) {
         hipStreamSynchronize(dev->stream);
+        {
+            // its work is done: nothing is left to wait for
+            std::lock_guard<std::mutex> lk(g_static_mu);
+            auto it = g_static.find(dev->ordinal);
+            if (it != g_static.end() && it->second.last == dev->stream) it->second.last = nullptr;
+        }
         hipStreamDestroy(dev->stream);
     }
     delete dev;
@@ -551,10 +577,22 @@ static void bind_all(sanic_hip_exe* exe, sanic_hip_buffer* const* bindings, int 
             bound[i] = owned.back().get();
         }
     }
-    scratch.reset(new_buffer(exe->dev, (size_t)std::max<int64_t>(exe->low.scratch_bytes, 256)));
-    // arrival counters in the arena must start at zero; kernels re-arm them after each launch
-    SANIC_HIP(hipMemsetAsync(scratch->ptr(), 0, scratch->bytes, exe->dev->stream));
+    // the arena, then the arrival counters, which must start at zero; kernels re-arm them
+    const size_t arena = (size_t)(exe->low.scratch_bytes + 255) / 256 * 256, counts = (size_t)exe->low.counter_bytes;
+    scratch.reset(new_buffer(exe->dev, std::max<size_t>(arena + counts, 256)));
+    if (counts) SANIC_HIP(hipMemsetAsync(scratch->ptr() + arena, 0, counts, exe->dev->stream));
     SANIC_HIP(hipStreamSynchronize(exe->dev->stream));
+}
+
+static std::vector<char*> addresses(const std::vector<sanic_hip_buffer*>& bound) {
+    std::vector<char*> at(bound.size(), nullptr);
+    for (size_t i = 0; i < bound.size(); i++)
+        if (bound[i]) at[i] = bound[i]->ptr();
+    return at;
+}
+
+static char* counters_of(const sanic_hip_exe* exe, sanic_hip_buffer* scratch) {
+    return scratch->ptr() + (exe->low.scratch_bytes + 255) / 256 * 256;
 }
 
 int sanic_hip_execute(sanic_hip_exe* exe, sanic_hip_buffer* const* bindings, int n_bindings, sanic_hip_buffer** outputs) {
@@ -568,7 +606,7 @@ int sanic_hip_execute(sanic_hip_exe* exe, sanic_hip_buffer* const* bindings, int
         std::vector<std::unique_ptr<sanic_hip_buffer>> owned;
         std::unique_ptr<sanic_hip_buffer> scratch;
         bind_all(exe, bindings, n_bindings, bound, owned, scratch);
-        enqueue(exe, bound, scratch->ptr());
+        enqueue(exe, addresses(bound).data(), scratch->ptr(), counters_of(exe, scratch.get()));
         SANIC_HIP(hipStreamSynchronize(exe->dev->stream));
         for (int i = 0; i < (int)exe->buffers.size(); i++) outputs[i] = nullptr;
         for (auto& o : owned) {
@@ -588,59 +626,60 @@ int sanic_hip_execute_static(sanic_hip_exe* exe, sanic_hip_buffer* const* bindin
         if (n_bindings != nb) fail(SANIC_ERR_ARG, "expected " + std::to_string(nb) + " bindings, got " + std::to_string(n_bindings));
         char* base = exe->dev->scratch_ptr;
         if (!base) fail(SANIC_ERR_BACKEND, "the device has no static scratch address");
-        // layout: the arena first, then every SCRATCH-role buffer, each at 256-byte alignment
+        // layout: the arena first, then every SCRATCH-role buffer, each at 256-byte alignment, then
+        // the counters of a program that has more than the static ones
         auto up = [](int64_t v) { return (v + 255) / 256 * 256; };
-        const int64_t arena = up(std::max<int64_t>(exe->low.scratch_bytes, 0));
-        int64_t need = arena;
-        std::vector<int64_t> at(nb, -1);
-        for (int i = 0; i < nb; i++)
+        int64_t need = up(std::max<int64_t>(exe->low.scratch_bytes, 0));
+        char* few[64];
+        std::vector<char*> more;
+        char** at = few;
+        if (nb > 64) {
+            more.resize(nb);
+            at = more.data();
+        }
+        for (int i = 0; i < nb; i++) {
             if (exe->buffers[i].role == SANIC_BUF_SCRATCH) {
-                at[i] = need;
+                at[i] = base + need;
                 need += up(buffer_bytes(exe->buffers[i]));
+            } else {
+                check_binding(exe, i, bindings[i]);
+                at[i] = bindings[i]->ptr();
             }
+        }
+        const int64_t counts = exe->low.counter_bytes;
+        const bool own = counts > (int64_t)kStaticCounterBytes;
+        char* cnt = own ? base + need : exe->dev->counters_ptr;
+        if (own) need += counts;
         if (need > (int64_t)kStaticScratchBytes)
             fail(SANIC_ERR_ARG, "this program needs " + std::to_string(need) + " bytes of scratch; the static scratch holds " +
                                     std::to_string(kStaticScratchBytes));
-        std::vector<sanic_hip_buffer> views(nb);
-        std::vector<sanic_hip_buffer*> bound(nb, nullptr);
-        auto whole = std::make_shared<Storage>();     // not owned: never freed
-        whole->ptr = base;
-        whole->bytes = kStaticScratchBytes;
-        for (int i = 0; i < nb; i++) {
-            if (at[i] >= 0) {
-                views[i].dev = exe->dev;
-                views[i].storage = whole;
-                views[i].offset = (size_t)at[i];
-                views[i].bytes = (size_t)buffer_bytes(exe->buffers[i]);
-                bound[i] = &views[i];
-            } else {
-                check_binding(exe, i, bindings[i]);
-                bound[i] = bindings[i];
-            }
-        }
         SANIC_HIP(hipSetDevice(exe->dev->ordinal));
         hipStream_t s = exe->dev->stream;
-        hipEvent_t done;
-        {
-            std::lock_guard<std::mutex> lk(g_static_mu);
-            done = g_static_done.at(exe->dev->ordinal);
-        }
-        // after the previous call's work on this GPU, whichever stream it ran on (a wait on a
-        // never-recorded event is satisfied at once); not under graph capture, where an event
-        // recorded outside the graph is no dependency the graph can hold
+        std::lock_guard<std::mutex> lk(g_static_mu);
+        StaticOrder& o = g_static.at(exe->dev->ordinal);
+        // after the previous call's work on this GPU, whichever stream it ran on; not under graph
+        // capture, where an event recorded outside the graph is no dependency the graph can hold
         hipStreamCaptureStatus cap = hipStreamCaptureStatusNone;
         SANIC_HIP(hipStreamIsCapturing(s, &cap));
         const bool eager = cap == hipStreamCaptureStatusNone;
-        if (eager) SANIC_HIP(hipStreamWaitEvent(s, done, 0));
-        // arrival counters start at zero (a fill kernel, not a memset: safe under graph capture)
-        if (arena > 0) {
-            const int64_t words = arena / 4;
+        if (eager && o.last && o.last != s) {
+            if (!o.marked) SANIC_HIP(hipEventRecord(o.done, o.last));
+            SANIC_HIP(hipStreamWaitEvent(s, o.done, 0));
+        }
+        if (eager) {
+            o.last = s;
+            o.marked = false;
+        }
+        // counters start at zero: the static ones are (the last program's kernels re-armed theirs),
+        // except behind a captured graph's replays that raced on them, so a graph clears its own (a
+        // fill kernel, not a memset: safe under graph capture)
+        if (counts > 0 && (own || !eager)) {
+            const int64_t words = counts / 4;
             hipLaunchKernelGGL(sanic_zero_words, dim3((unsigned)std::min<int64_t>((words + 255) / 256, 4096)), dim3(256), 0, s,
-                               (uint32_t*)base, words);
+                               (uint32_t*)cnt, words);
             SANIC_HIP(hipGetLastError());
         }
-        enqueue(exe, bound, base);
-        if (eager) SANIC_HIP(hipEventRecord(done, s));
+        enqueue(exe, at, base, cnt);
     });
 }
 
@@ -652,10 +691,21 @@ static const int kMultiStep = 8;
 static void capture_steps(sanic_hip_replay* rp, int steps, hipGraph_t* graph, hipGraphExec_t* exec) {
     sanic_hip_exe* exe = rp->exe;
     hipStream_t s = exe->dev->stream;
+    const std::vector<char*> at = addresses(rp->bound);
+    {
+        // a sanic_hip_execute_static call on another stream waits for this one's work: the event it
+        // waits for cannot be recorded while the stream is capturing
+        std::lock_guard<std::mutex> lk(g_static_mu);
+        StaticOrder& o = g_static.at(exe->dev->ordinal);
+        if (o.last == s && !o.marked) {
+            SANIC_HIP(hipEventRecord(o.done, s));
+            o.marked = true;
+        }
+    }
     SANIC_HIP(hipStreamBeginCapture(s, hipStreamCaptureModeThreadLocal));
     try {
         for (int step = 0; step < steps; step++) {
-            enqueue(exe, rp->bound, rp->scratch->ptr());
+            enqueue(exe, at.data(), rp->scratch->ptr(), counters_of(exe, rp->scratch.get()));
             for (auto& fb : rp->feedback) {
                 const auto& ob = exe->buffers[fb.first];
                 const auto& ib = exe->buffers[fb.second];
@@ -746,7 +796,7 @@ int sanic_hip_step_many(sanic_hip_replay* rp, int n, double* gpu_seconds) {
             const auto& st = rp->exe->low.stages;
             std::vector<hipEvent_t> ev(st.size() + 1);
             for (auto& e : ev) SANIC_HIP(hipEventCreate(&e));
-            enqueue(rp->exe, rp->bound, rp->scratch->ptr(), ev.data());
+            enqueue(rp->exe, addresses(rp->bound).data(), rp->scratch->ptr(), counters_of(rp->exe, rp->scratch.get()), ev.data());
             SANIC_HIP(hipEventSynchronize(ev[st.size()]));
             float tot = 0;
             SANIC_HIP(hipEventElapsedTime(&tot, ev[0], ev[st.size()]));
@@ -805,7 +855,7 @@ int sanic_hip_profile_stages(sanic_hip_replay* rp, double* seconds, int n) {
         if (n < ns) fail(SANIC_ERR_ARG, "seconds[] is shorter than the stage count");
         std::vector<hipEvent_t> ev(ns + 1);
         for (auto& e : ev) SANIC_HIP(hipEventCreate(&e));
-        enqueue(rp->exe, rp->bound, rp->scratch->ptr(), ev.data());
+        enqueue(rp->exe, addresses(rp->bound).data(), rp->scratch->ptr(), counters_of(rp->exe, rp->scratch.get()), ev.data());
         SANIC_HIP(hipEventSynchronize(ev[ns]));
         for (int i = 0; i < ns; i++) {
             float ms = 0;

@@ -785,13 +785,11 @@ bool lower_attn_decode(const sanic_program_desc* d, int si, int64_t& scratch, Lo
     // applied to all chunks at once): M = max_c m_c, w_c = [−∞ < m_c]·exp(m_c − M), every
     // ExpShifted slot = Σ_c w_c·x_c. This is the pairwise combine of run_carrier_split
     // (interp.rs:555-643) regrouped — no chain of NCH dependent steps.
-    const int64_t counter_off = scratch - sbase;
-    scratch += ((NG * 4 + 255) / 256) * 256;
     const int64_t GP = NPART * REP * PSZ;       // floats of one group's partials
     if (GP * 4 > 64 * 1024) return false;
     k.line("{");
     k.indent++;
-    k.line("unsigned* cnt = (unsigned*)((char*)a.scratch + " + std::to_string(counter_off) + ") + grp;");
+    k.line("unsigned* cnt = a.counters + grp;");
     emit_arrival(k, "sanic_last", "tid", "cnt", std::to_string(NPART) + "u");
     k.line("if (!sanic_last) return;");
     k.line("__shared__ __attribute__((aligned(16))) float g_lds[" + std::to_string(GP) + "];");
@@ -893,7 +891,7 @@ bool lower_attn_decode(const sanic_program_desc* d, int si, int64_t& scratch, Lo
     const std::string tag = "h" + std::to_string(NH) + "_t" + std::to_string(T);
     const std::string kpart = "sanic_attn_decode_" + tag;
     std::ostringstream src;
-    src << kPrelude << R.args_struct({"float* __restrict__ scratch"});
+    src << kPrelude << R.args_struct({"float* __restrict__ scratch", "unsigned* counters"});
     src << "extern \"C\" __global__ void __launch_bounds__(" << NT << ") " << kpart << "(Args a) {\n" << R.entry() << k.str() << "}\n";
     out.kernel_kind = "skeleton:attn_decode[rep " + std::to_string(REP) + "]" + (writes.empty() ? "" : "+writes" + std::to_string(writes.size())) + (sep ? "+rowwg" : "");
     // the ILP-maximising machine scheduler: C3 11.2 → 10.75 µs (the default strategy interleaves
@@ -902,6 +900,7 @@ bool lower_attn_decode(const sanic_program_desc* d, int si, int64_t& scratch, Lo
     out.variants = nvar;
     std::vector<Arg> args = R.arg_list();
     args.push_back({Arg::SCRATCH, sbase});
+    args.push_back({Arg::COUNTERS, take_counters(NG)});
     out.launches.push_back({kpart, "", dim3((unsigned)NG, (unsigned)NPART), dim3((unsigned)NT), 0, args});
     return true;
 }

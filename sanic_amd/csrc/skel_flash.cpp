@@ -451,7 +451,7 @@ bool lower_flash_prefill(const sanic_program_desc* d, int si, int64_t& scratch, 
         Code scratch_code;
         emit_point_fold(R, scratch_code, st, "pf");
     }
-    src << (SPL > 1 ? R.args_struct({"float* __restrict__ scratch"}) : R.args_struct({}));
+    src << (SPL > 1 ? R.args_struct({"float* __restrict__ scratch", "unsigned* counters"}) : R.args_struct({}));
     src << "typedef __bf16 sanic_bf16x2 __attribute__((ext_vector_type(2)));\n";
     src << "typedef float sanic_f32x2 __attribute__((ext_vector_type(2)));\n";
     src << "__device__ __forceinline__ unsigned pk_bf16(float x, float y) {\n"
@@ -1002,11 +1002,11 @@ bool lower_flash_prefill(const sanic_program_desc* d, int si, int64_t& scratch, 
     k.line("}");
     int64_t soff = -1;
     if (SPL > 1) {
-        // partials [block][part][36][256 lanes] (o in accumulator order, m, ℓ), then one arrival
-        // counter per block (zeroed at bind time, re-armed by the combining workgroup)
+        // partials [block][part][36][256 lanes] (o in accumulator order, m, ℓ), and one arrival
+        // counter per block, re-armed by the combining workgroup
         soff = scratch;
         const int64_t pbytes = NB * 2 * 36 * 256 * 4;
-        scratch += pbytes + ((NB * 4 + 255) / 256) * 256;
+        scratch += pbytes;
         k.line("{");
         k.indent++;
         k.line("float* pw = a.scratch + ((idx_t)bid * 2 + part) * 9216 + tid;");
@@ -1017,7 +1017,7 @@ bool lower_flash_prefill(const sanic_program_desc* d, int si, int64_t& scratch, 
         k.line("    #pragma unroll");
         k.line("    for (int r = 0; r < 4; ++r) sanic_st(pw + ((dt * 2 + qt) * 4 + r) * 256, o[dt][qt][r]);");
         k.line("for (int qt = 0; qt < 2; ++qt) { sanic_st(pw + (32 + qt) * 256, m_run[qt]); sanic_st(pw + (34 + qt) * 256, lsum[qt][0]); }");
-        k.line("unsigned* cnt = (unsigned*)((char*)a.scratch + " + std::to_string(pbytes) + ") + bid;");
+        k.line("unsigned* cnt = a.counters + bid;");
         emit_arrival(k, "sp_last", "tid", "cnt", "2u");
         k.line("if (!sp_last) return;");
         k.line("if (tid == 0) sanic_st(cnt, 0u);");
@@ -1100,7 +1100,10 @@ bool lower_flash_prefill(const sanic_program_desc* d, int si, int64_t& scratch, 
     out.source = src.str();
     out.variants = P.ragged ? 1 : 4;
     std::vector<Arg> args = R.arg_list();
-    if (SPL > 1) args.push_back({Arg::SCRATCH, soff});
+    if (SPL > 1) {
+        args.push_back({Arg::SCRATCH, soff});
+        args.push_back({Arg::COUNTERS, take_counters(NB)});
+    }
     out.launches.push_back({kname, "", dim3((unsigned)(NB * SPL)), dim3(256), 0, args});
     return true;
 }

@@ -903,8 +903,7 @@ bool lower_gemv_group(const sanic_program_desc* d, int si, int64_t& scratch, std
     int64_t blocks = std::min<int64_t>((waves + 3) / 4, max_blocks);
     int64_t counter_off = -1;
     if (!tails.empty()) {
-        counter_off = scratch;
-        scratch += 256;
+        counter_off = take_counters(1);
     }
 
     // ── split-K form: the 4 waves of a workgroup take one quarter of K each, every lane keeps
@@ -1179,10 +1178,10 @@ bool lower_gemv_group(const sanic_program_desc* d, int si, int64_t& scratch, std
             }
         }
         if (!tails.empty())
-            emit_tail(R, k, d, tails, "(unsigned*)a.scratch", "gridDim.x");
+            emit_tail(R, k, d, tails, "a.counters", "gridDim.x");
         const std::string kname = "sanic_gemv_" + std::to_string(NTOT) + "x" + std::to_string(K);
         std::ostringstream src;
-        src << kPrelude << R.args_struct(tails.empty() ? std::vector<std::string>{} : std::vector<std::string>{"float* __restrict__ scratch"})
+        src << kPrelude << R.args_struct(tails.empty() ? std::vector<std::string>{} : std::vector<std::string>{"unsigned* counters"})
             << "extern \"C\" __global__ void __launch_bounds__(256) " << kname << "(Args a) {\n" << R.entry() << k.str() << "}\n";
         LoweredStage L;
         L.kernel_kind = "skeleton:gemv" + std::string(group.size() > 1 ? "[batched " + std::to_string(group.size()) + "]" : "") +
@@ -1197,7 +1196,7 @@ bool lower_gemv_group(const sanic_program_desc* d, int si, int64_t& scratch, std
         L.source = (strat ? std::string("// sched-strategy: ") + strat + "\n" : std::string()) + src.str();
         L.variants = nvar;
         std::vector<Arg> args = R.arg_list();
-        if (!tails.empty()) args.push_back({Arg::SCRATCH, counter_off});   // the tail counter: relative offset 0
+        if (!tails.empty()) args.push_back({Arg::COUNTERS, counter_off});
         L.launches.push_back({kname, "", dim3((unsigned)nblocks), dim3(256), 0, args});
         out.push_back(std::move(L));
         for (size_t g = 1; g < group.size(); g++) {
@@ -1432,12 +1431,12 @@ bool lower_gemv_group(const sanic_program_desc* d, int si, int64_t& scratch, std
     k.indent--;
     k.line("}");
     if (!tails.empty())
-        emit_tail(R, k, d, tails, "(unsigned*)a.scratch", "gridDim.x");
+        emit_tail(R, k, d, tails, "a.counters", "gridDim.x");
 
     // kernel names carry the shape so profiles tell the launches apart
     const std::string kname = "sanic_gemv_" + std::to_string(NTOT) + "x" + std::to_string(K);
     std::ostringstream src;
-    src << kPrelude << R.args_struct(tails.empty() ? std::vector<std::string>{} : std::vector<std::string>{"float* __restrict__ scratch"})
+    src << kPrelude << R.args_struct(tails.empty() ? std::vector<std::string>{} : std::vector<std::string>{"unsigned* counters"})
         << "extern \"C\" __global__ void __launch_bounds__(256) " << kname << "(Args a) {\n" << R.entry() << k.str() << "}\n";
     LoweredStage L;
     L.kernel_kind = "skeleton:gemv" + std::string(group.size() > 1 ? "[batched " + std::to_string(group.size()) + "]" : "") +
@@ -1446,7 +1445,7 @@ bool lower_gemv_group(const sanic_program_desc* d, int si, int64_t& scratch, std
     L.source = src.str();
     uint32_t lds = (uint32_t)((SC * K + 4 * std::max(SR, 1)) * 4);
     std::vector<Arg> args = R.arg_list();
-    if (!tails.empty()) args.push_back({Arg::SCRATCH, counter_off});   // the tail counter: relative offset 0
+    if (!tails.empty()) args.push_back({Arg::COUNTERS, counter_off});
     L.launches.push_back({kname, "", dim3((unsigned)blocks), dim3(256), lds, args});
     out.push_back(std::move(L));
     for (size_t g = 1; g < group.size(); g++) {
@@ -1523,8 +1522,7 @@ bool lower_gemv_kmajor(const sanic_program_desc* d, int si, int64_t& scratch, Lo
         if (KSL > 1) {
             part_off = scratch;
             scratch += ((KSL * SC * N * 4 + 255) / 256) * 256;
-            counter_off = scratch;
-            scratch += ((NS * 4 + 255) / 256) * 256;
+            counter_off = take_counters(NS);
         }
         Renderer R(d);
         Code k;
@@ -1649,7 +1647,7 @@ bool lower_gemv_kmajor(const sanic_program_desc* d, int si, int64_t& scratch, Lo
                 k.line(std::string("  ") + (xl ? "sanic_stx" : "sanic_st") + "(a.scratch + " + std::to_string(part_off / 4) + " + (slice * " + std::to_string(SC) + " + " +
                        std::to_string(cs) + ") * " + std::to_string(N) + " + strip * " + std::to_string(SW) + " + t, " + wave_sum_of(cs) + ");");
             k.line("}");
-            k.line("unsigned* cnt = (unsigned*)((char*)a.scratch + " + std::to_string(counter_off) + ") + strip;");
+            k.line("unsigned* cnt = a.counters + strip;");
             emit_arrival(k, "sanic_last", "t", "cnt", std::to_string(KSL) + "u", xl);
             k.line("if (!sanic_last) return;");
             k.line("if (t == 0) sanic_st(cnt, 0u);");
@@ -1686,13 +1684,16 @@ bool lower_gemv_kmajor(const sanic_program_desc* d, int si, int64_t& scratch, Lo
         k.line("}");
         const std::string kname = "sanic_gemvt_" + std::to_string(N) + "x" + std::to_string(K);
         std::ostringstream src;
-        src << kPrelude << R.args_struct(KSL > 1 ? std::vector<std::string>{"float* __restrict__ scratch"} : std::vector<std::string>{})
+        src << kPrelude << R.args_struct(KSL > 1 ? std::vector<std::string>{"float* __restrict__ scratch", "unsigned* counters"} : std::vector<std::string>{})
             << "extern \"C\" __global__ void __launch_bounds__(" << NT << ") " << kname << "(Args a) {\n" << R.entry() << k.str() << "}\n";
         out.kernel_kind = "skeleton:gemv_kmajor[strips " + std::to_string(SW) + (KSL > 1 ? " x" + std::to_string(KSL) + " slices" : "") + "]" + (xl ? "+xcd" : "");
         out.source = "// sched-strategy: max-memory-clause\n" + src.str();   // B1 12.26 → 12.07 µs
         out.variants = 4;
         std::vector<Arg> args = R.arg_list();
-        if (KSL > 1) args.push_back({Arg::SCRATCH, 0});
+        if (KSL > 1) {
+            args.push_back({Arg::SCRATCH, 0});
+            args.push_back({Arg::COUNTERS, counter_off});
+        }
         out.launches.push_back({kname, "", dim3((unsigned)(NS * KSL)), dim3((unsigned)NT), 0, args});
         return true;
     }
@@ -1706,8 +1707,7 @@ bool lower_gemv_kmajor(const sanic_program_desc* d, int si, int64_t& scratch, Lo
     scratch += ((KS * SC * N * 4 + 255) / 256) * 256;
     int64_t rpart_off = scratch;                 // per-slice row-slot partials [NCG][KS][SR]
     scratch += ((NCG * KS * std::max(SR, 1) * 4 + 255) / 256) * 256;
-    int64_t counter_off = scratch;
-    scratch += ((NCG * 4 + 255) / 256) * 256;
+    const int64_t counter_off = take_counters(NCG);
 
     Renderer R(d);
     Code k;
@@ -1793,7 +1793,7 @@ bool lower_gemv_kmajor(const sanic_program_desc* d, int si, int64_t& scratch, Lo
     k.line("  const int cs = i / 512, col = i % 512;");
     k.line("  sanic_st(a.scratch + " + std::to_string(part_off / 4) + " + (ks * " + std::to_string(SC) + " + cs) * " + std::to_string(N) + " + cg * 512 + col, v);");
     k.line("}");
-    k.line("unsigned* cnt = (unsigned*)((char*)a.scratch + " + std::to_string(counter_off) + ") + cg;");
+    k.line("unsigned* cnt = a.counters + cg;");
     emit_arrival(k, "sanic_last", "t", "cnt", std::to_string(KS) + "u");
     k.line("if (!sanic_last) return;");
     k.line("if (t == 0) sanic_st(cnt, 0u);");
@@ -1827,12 +1827,13 @@ bool lower_gemv_kmajor(const sanic_program_desc* d, int si, int64_t& scratch, Lo
 
     const std::string kname = "sanic_gemvt_" + std::to_string(N) + "x" + std::to_string(K);
     std::ostringstream src;
-    src << kPrelude << R.args_struct({"float* __restrict__ scratch"})
+    src << kPrelude << R.args_struct({"float* __restrict__ scratch", "unsigned* counters"})
         << "extern \"C\" __global__ void __launch_bounds__(256) " << kname << "(Args a) {\n" << R.entry() << k.str() << "}\n";
     out.kernel_kind = "skeleton:gemv_kmajor[" + std::to_string(KS) + " slices]";   // the strip form's fallback
     out.source = src.str();
     std::vector<Arg> args = R.arg_list();
     args.push_back({Arg::SCRATCH, 0});
+    args.push_back({Arg::COUNTERS, counter_off});
     out.launches.push_back({kname, "", dim3((unsigned)(NCG * KS)), dim3(256), 0, args});
     return true;
 }

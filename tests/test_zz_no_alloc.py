@@ -74,3 +74,29 @@ def test_execute_static_refuses_programs_beyond_its_scratch(dev):
     with pytest.raises(SanicError) as e:
         exe.execute_static(bufs)
     assert "static scratch holds" in str(e.value)
+
+
+def test_execute_static_orders_handles_that_share_the_scratch(dev):
+    """Calls alternating between two device handles (a stream each) with nothing waited for in
+    between, a capture of one of them among the calls: every output as the first call's, bit for
+    bit, though all of them use the same scratch and arrival counters."""
+    from sanic_amd.backend import HipDevice
+    other = HipDevice(0)
+    runs = []
+    for d in (dev, other):
+        for prog, vals in (_flash(512), _argmax(70000)):
+            exe = d.prepare(prog)
+            bufs = {n: d.from_values(v, prog.by_name[n].dtype) for n, v in vals.items()}
+            name = [b.name for b in prog.buffers if b.role == OUTPUT][-1]
+            want = exe.execute(bufs)[name].download()
+            outs = [d.alloc(len(want)) for _ in range(6)]
+            runs.append((d, exe, bufs, name, want, outs))
+    for k in range(6):
+        for d, exe, bufs, name, want, outs in runs:
+            exe.execute_static({**bufs, name: outs[k]})
+            if k == 3:
+                exe.capture(bufs).step()
+    for d, exe, bufs, name, want, outs in runs:
+        assert all(o.download() == want for o in outs), name
+    del runs, exe, bufs, outs
+    other.close()
