@@ -1117,9 +1117,12 @@ bool lower_flash_prefill(const sanic_program_desc* d, int si, int64_t& scratch, 
 // a running (m, ℓ, o) of its own, and merge in LDS by the carrier's combine in wave order. Sᵀ =
 // K·Qᵀ, so a lane owns one query column and its P values are the next MFMA's B operand as they
 // stand; K and V rows come straight from global memory (whole rows per 16 lanes), one tile ahead.
-// The bound is the f32 MFMA rate of a row block's CU (16 rows × 1024 keys × 64: 7 µs). S = 1024,
-// d = 64, causal: 1099 µs in the generic fold, which forms q·k for each of the 64 value columns.
-bool lower_flash_f32(const sanic_program_desc* d, int si, LoweredStage& out) {
+// The bound is the f32 MFMA rate and the softmax arithmetic of a row block's CU, so where the row
+// blocks leave CUs idle up to 8 workgroups share one, a run of its key tiles each, and the last to
+// arrive merges their partials in order. S = 1024, d = 64, causal: 1099 µs in the generic fold,
+// which forms q·k for each of the 64 value columns; 18.6 with one workgroup per row block, 10.6
+// with 4 (256 in all; 11.8 with 512, 13.1 with 128).
+bool lower_flash_f32(const sanic_program_desc* d, int si, int64_t& scratch, LoweredStage& out) {
     FlashPlan P;
     if (!attention_plan(d, si, P)) return false;
     const sanic_stage& st = d->stages[si];
@@ -1129,6 +1132,10 @@ bool lower_flash_f32(const sanic_program_desc* d, int si, LoweredStage& out) {
     if (!wide(P.qacc.dtype) || !wide(P.kacc.dtype) || !wide(P.vacc.dtype)) return false;
     const int64_t NH = P.NH, NQ = P.NQ, T = P.T, E = P.E, HD = P.HD;
     if (HD % 16 || E % 16 || HD > 128 || E > 128 || (E / 16 & (E / 16 - 1))) return false;
+    // up to 128 × 128 scores the stage keeps the generic fold and its own choice of schedule (what a
+    // program of config A's size is expected to lower to): S = 128 22.3 µs at d = 64 and 8.1 at
+    // d = 32 there, 7.1 and 4.9 here
+    if (NH * NQ * T <= 128 * 128) return false;
     std::vector<int64_t> qc, kc, vc;
     int qh, kh, vh;
     int64_t qhc, khc, vhc;
@@ -1189,17 +1196,34 @@ bool lower_flash_f32(const sanic_program_desc* d, int si, LoweredStage& out) {
             for (int i = 0; i < n; i++) k.line(x + "[" + S(i) + "] = sanic_bf16((" + p + ")[" + S(i) + "]);");
         }
     };
-    const int64_t NQB = (NQ + 15) / 16;
-    k.line("__shared__ float o_lds[" + S(NWV) + "][" + S(E) + "][16], m_lds[" + S(NWV) + "][16], l_lds[" + S(NWV) + "][16];");
+    const int64_t NQB = (NQ + 15) / 16, NB = NH * NQB, NBP = (NB + 7) / 8 * 8;
+    const int SPL = (int)std::max<int64_t>(1, std::min<int64_t>({8, 256 / NB, (T + 127) / 128}));
+    // the workgroups of a row block are NBP apart, a multiple of 8: on one XCD
+    const bool xl = SPL > 1 && xcd_local_enabled();
+    const std::string stx = xl ? "sanic_stx" : "sanic_st", ldx = xl ? "sanic_ldx" : "sanic_ld";
+    const int64_t PSZ = 16 * E + 32;                  // floats of a partial: o, m, ℓ
+    const int64_t soff = scratch;
+    if (SPL > 1) scratch += (NB * SPL * PSZ * 4 + 255) / 256 * 256;
+    k.line("__shared__ float o_lds[" + S(NWV) + "][" + S(E) + "][17], m_lds[" + S(NWV) + "][16], l_lds[" + S(NWV) + "][16];");
     k.line("const int tid = threadIdx.x, lane = tid & 63, wv = __builtin_amdgcn_readfirstlane(tid >> 6);");
     k.line("const int l16 = lane & 15, lq = lane >> 4;");
     // the longest (last) row blocks first
-    k.line("const idx_t hh = blockIdx.x % " + S(NH) + ", q0 = (" + S(NQB - 1) + " - blockIdx.x / " + S(NH) + ") * 16;");
+    k.line("const int bid = blockIdx.x % " + S(SPL > 1 ? NBP : NB) + ", part = blockIdx.x / " + S(SPL > 1 ? NBP : NB) + ";");
+    if (SPL > 1 && NBP != NB) k.line("if (bid >= " + S(NB) + ") return;");
+    k.line("const idx_t hh = bid % " + S(NH) + ", q0 = (" + S(NQB - 1) + " - bid / " + S(NH) + ") * 16;");
     k.line("const idx_t qlast = q0 + 15 < " + S(NQ) + " ? q0 + 15 : (idx_t)" + S(NQ - 1) + ";");
     k.line("idx_t alo, ahi, blo, bhi;");
     k.line("window(a, hh, q0, alo, ahi);");
     k.line("window(a, hh, qlast, blo, bhi);");
-    k.line("const int klo = __builtin_amdgcn_readfirstlane((int)(alo < blo ? alo : blo)) / 16 * 16, khi = __builtin_amdgcn_readfirstlane((int)(ahi > bhi ? ahi : bhi));");
+    k.line("int klo = __builtin_amdgcn_readfirstlane((int)(alo < blo ? alo : blo)) / 16 * 16, khi = __builtin_amdgcn_readfirstlane((int)(ahi > bhi ? ahi : bhi));");
+    if (SPL > 1) {
+        // as many of them as have a tile for each wave
+        k.line("const int nt = (khi - klo + 15) / 16, nsp = nt <= 8 ? 1 : nt >= " + S(8 * SPL) + " ? " + S(SPL) + " : (nt + 7) / 8;");
+        k.line("if (part >= nsp) return;");
+        k.line("const int per = (nt + nsp - 1) / nsp * 16;");
+        k.line("klo += part * per;");
+        k.line("khi = klo + per < khi ? klo + per : khi;");
+    }
     k.line("const int qi = (int)(q0 + l16 < qlast ? q0 + l16 : qlast);");
     // step s contracts d = lq·DS + s: a lane's operands of all steps are one contiguous run
     k.line("float qv[" + S(DS) + "];");
@@ -1260,20 +1284,11 @@ bool lower_flash_f32(const sanic_program_desc* d, int si, LoweredStage& out) {
     for (int e = 0; e < ET; e++)
         for (int r = 0; r < 4; r++) k.line("o_lds[wv][(lq * 4 + " + S(r) + ") * " + S(ET) + " + " + S(e) + "][l16] = o[" + S(e) + "][" + S(r) + "];");
     k.line("__syncthreads();");
-    k.line("for (int p = tid; p < " + S(16 * E) + "; p += " + S(64 * NWV) + ") {");
+    // one output point from its merged carrier
+    k.line("auto point = [&](int row, int ee, float M, float L, float O) {");
     k.indent++;
-    k.line("const int ee = p % " + S(E) + ", row = p / " + S(E) + ";");
     k.line("const idx_t qi = q0 + row;");
-    k.line("if (qi >= " + S(NQ) + ") continue;");
-    k.line("float M = m_lds[0][row];");
-    for (int w = 1; w < NWV; w++) k.line("M = fmaxf(M, m_lds[" + S(w) + "][row]);");
-    k.line("float L = 0.0f, O = 0.0f;");
-    k.line("#pragma unroll");
-    k.line("for (int w = 0; w < " + S(NWV) + "; ++w) {");
-    k.line("  const float mw = m_lds[w][row], x = mw == -__builtin_huge_valf() ? 0.0f : expf(mw - M);");
-    k.line("  L = fmaf(x, l_lds[w][row], L);");
-    k.line("  O = fmaf(x, o_lds[w][ee][row], O);");
-    k.line("}");
+    k.line("if (qi >= " + S(NQ) + ") return;");
     k.line("float fs" + S(P.max_slot) + " = M;");
     for (size_t s = 0; s < P.scalar_slots.size(); s++) k.line("float fs" + S(P.scalar_slots[s]) + " = " + flit(P.scalar_into[s]) + " * L;");
     k.line("float fs" + S(P.vec_slots[0]) + " = O;");
@@ -1281,19 +1296,77 @@ bool lower_flash_f32(const sanic_program_desc* d, int si, LoweredStage& out) {
     // honest window gives; such a point is folded again
     k.line("if (!(__builtin_fabsf(O) <= 3.402823466e38f) || !(__builtin_fabsf(L) <= 3.402823466e38f) || !(__builtin_fabsf(M) <= 3.402823466e38f)) {");
     k.indent++;
-    {
-        std::vector<std::string> g = gc;
-        for (int j = 0; j < st.rank; j++) k.line("const idx_t g" + S(j) + " = " + g[j] + ";");
-        emit_point_fold(R, k, st, "pf");
-        for (int s = 0; s < c.slots; s++) k.line("fs" + S(s) + " = pf" + S(s) + ";");
-    }
+    for (int j = 0; j < st.rank; j++) k.line("const idx_t g" + S(j) + " = " + gc[j] + ";");
+    emit_point_fold(R, k, st, "pf");
+    for (int s = 0; s < c.slots; s++) k.line("fs" + S(s) + " = pf" + S(s) + ";");
     k.indent--;
     k.line("}");
     std::string fargs;
     for (int s = 0; s < c.slots; s++) fargs += ", fs" + S(s);
     k.line("finish(a, hh, qi, ee" + fargs + ");");
     k.indent--;
+    k.line("};");
+    // n partials in order: M = max m, each weighed by exp(m − M), a side whose m is −∞ by 0
+    auto merge = [&](const std::string& n, const std::string& m, const std::string& l, const std::string& o) {
+        k.line("float M = -__builtin_huge_valf();");
+        k.line("for (int w = 0; w < " + n + "; ++w) M = fmaxf(M, " + m + ");");
+        k.line("float L = 0.0f, O = 0.0f;");
+        k.line("for (int w = 0; w < " + n + "; ++w) {");
+        k.line("  const float mw = " + m + ", x = mw == -__builtin_huge_valf() ? 0.0f : expf(mw - M);");
+        k.line("  L = fmaf(x, " + l + ", L);");
+        k.line("  O = fmaf(x, " + o + ", O);");
+        k.line("}");
+    };
+    const std::string points = "for (int p = tid; p < " + S(16 * E) + "; p += " + S(64 * NWV) + ") {";
+    k.line(points);
+    k.indent++;
+    k.line("const int ee = p % " + S(E) + ", row = p / " + S(E) + ";");
+    merge(S(NWV), "m_lds[w][row]", "l_lds[w][row]", "o_lds[w][ee][row]");
+    if (SPL > 1) {
+        k.line("if (nsp > 1) {");
+        k.line("  float* to = a.scratch + ((idx_t)bid * " + S(SPL) + " + part) * " + S(PSZ) + ";");
+        k.line("  " + stx + "(to + p, O);");
+        k.line("  if (ee == 0) { " + stx + "(to + " + S(16 * E) + " + row, M); " + stx + "(to + " + S(16 * E + 16) + " + row, L); }");
+        k.line("  continue;");
+        k.line("}");
+    }
+    k.line("point(row, ee, M, L, O);");
+    k.indent--;
     k.line("}");
+    if (SPL > 1) {
+        k.line("if (nsp == 1) return;");
+        k.line("unsigned* cnt = a.counters + bid;");
+        emit_arrival(k, "sanic_last", "tid", "cnt", "(unsigned)nsp", xl);
+        k.line("if (!sanic_last) return;");
+        k.line("if (tid == 0) sanic_st(cnt, 0u);");
+        k.line("const float* from = a.scratch + (idx_t)bid * " + S(SPL * PSZ) + ";");
+        k.line(points);
+        k.indent++;
+        k.line("const int ee = p % " + S(E) + ", row = p / " + S(E) + ";");
+        // (every partial requested before the first is used)
+        k.line("float pm[" + S(SPL) + "], pl[" + S(SPL) + "], po[" + S(SPL) + "];");
+        k.line("#pragma unroll");
+        k.line("for (int w = 0; w < " + S(SPL) + "; ++w) {");
+        k.line("  const float* f = from + (w < nsp ? w : 0) * " + S(PSZ) + ";");
+        k.line("  pm[w] = " + ldx + "(f + " + S(16 * E) + " + row);");
+        k.line("  pl[w] = " + ldx + "(f + " + S(16 * E + 16) + " + row);");
+        k.line("  po[w] = " + ldx + "(f + p);");
+        k.line("}");
+        k.line("float M = -__builtin_huge_valf();");
+        k.line("#pragma unroll");
+        k.line("for (int w = 0; w < " + S(SPL) + "; ++w) { if (w >= nsp) pm[w] = -__builtin_huge_valf(); M = fmaxf(M, pm[w]); }");
+        k.line("float L = 0.0f, O = 0.0f;");
+        k.line("#pragma unroll");
+        k.line("for (int w = 0; w < " + S(SPL) + "; ++w) {");
+        k.line("  if (w >= nsp) continue;");
+        k.line("  const float x = pm[w] == -__builtin_huge_valf() ? 0.0f : expf(pm[w] - M);");
+        k.line("  L = fmaf(x, pl[w], L);");
+        k.line("  O = fmaf(x, po[w], O);");
+        k.line("}");
+        k.line("point(row, ee, M, L, O);");
+        k.indent--;
+        k.line("}");
+    }
 
     const std::string kname = "sanic_attn32_h" + S(NH) + "_s" + S(NQ) + "_t" + S(T);
     std::ostringstream src;
@@ -1301,7 +1374,7 @@ bool lower_flash_f32(const sanic_program_desc* d, int si, LoweredStage& out) {
     src << "typedef __attribute__((__vector_size__(4 * sizeof(float)))) float f32x4;\n";
     src << "typedef float sanic_f32x4_any __attribute__((ext_vector_type(4), aligned(4)));\n";
     src << "typedef float sanic_f32x2_any __attribute__((ext_vector_type(2), aligned(4)));\n";
-    src << R.args_struct({});
+    src << R.args_struct(SPL > 1 ? std::vector<std::string>{"float* __restrict__ scratch", "unsigned* counters"} : std::vector<std::string>{});
     src << "__device__ __forceinline__ float score(const Args& a, float dotv, int hh, int qi, int kj) {\n"
         << Rs.entry() << sp.str() << "  return " << vpart << ";\n}\n";
     src << "__device__ __forceinline__ void window(const Args& a, idx_t hh, idx_t qrow, idx_t& lo, idx_t& hi) {\n"
@@ -1310,10 +1383,15 @@ bool lower_flash_f32(const sanic_program_desc* d, int si, LoweredStage& out) {
     for (int s = 0; s < c.slots; s++) src << ", float fs" << s;
     src << ") {\n" << Ro.entry() << fo.str() << "}\n";
     src << "extern \"C\" __global__ void __launch_bounds__(" << 64 * NWV << ") " << kname << "(Args a) {\n" << R.entry() << k.str() << "}\n";
-    out.kernel_kind = "skeleton:attn_f32[d " + S(HD) + "]";
+    out.kernel_kind = "skeleton:attn_f32[d " + S(HD) + "]" + (SPL > 1 ? "+split" + S(SPL) : "") + (xl ? "+xcd" : "");
     out.source = src.str();
     out.variants = 1;
-    out.launches.push_back({kname, "", dim3((unsigned)(NH * NQB)), dim3(64 * NWV), 0, R.arg_list()});
+    std::vector<Arg> args = R.arg_list();
+    if (SPL > 1) {
+        args.push_back({Arg::SCRATCH, soff});
+        args.push_back({Arg::COUNTERS, take_counters(NB)});
+    }
+    out.launches.push_back({kname, "", dim3((unsigned)(SPL > 1 ? NBP * SPL : NB)), dim3(64 * NWV), 0, args});
     return true;
 }
 

@@ -1844,7 +1844,7 @@ bool lower_skeleton(const sanic_program_desc* d, int si, int64_t& scratch, Lower
     if (lower_gemm(d, si, scratch, out)) return true;
     if (lower_flash_prefill(d, si, scratch, out)) return true;
     if (lower_attn_decode(d, si, scratch, out)) return true;
-    if (lower_flash_f32(d, si, out)) return true;
+    if (lower_flash_f32(d, si, scratch, out)) return true;
     return false;
 }
 

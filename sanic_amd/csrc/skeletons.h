@@ -82,7 +82,7 @@ std::string expr_rest(Renderer& R, Code& code, int e, int w, const std::function
 
 bool lower_gemm(const sanic_program_desc* d, int si, int64_t& scratch, LoweredStage& out);
 bool lower_skinny(const sanic_program_desc* d, int si, LoweredStage& out);
-bool lower_flash_f32(const sanic_program_desc* d, int si, LoweredStage& out);
+bool lower_flash_f32(const sanic_program_desc* d, int si, int64_t& scratch, LoweredStage& out);
 bool lower_flash_prefill(const sanic_program_desc* d, int si, int64_t& scratch, LoweredStage& out);
 bool lower_attn_decode(const sanic_program_desc* d, int si, int64_t& scratch, LoweredStage& out);
 

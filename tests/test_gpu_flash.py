@@ -182,12 +182,12 @@ F, B = ir.F32, ir.BF16
 
 
 @pytest.mark.parametrize("NH,NKV,NQ,T,HD,E,causal,dtypes", [
-    (0, 0, 128, 128, 64, 64, True, (F, F, F)),
-    (0, 0, 33, 33, 32, 32, True, (F, F, F)),      # one row into a third block
+    (0, 0, 129, 129, 64, 64, True, (F, F, F)),    # one row into a ninth block
+    (0, 0, 400, 400, 32, 32, True, (F, F, F)),
     (0, 0, 1000, 1000, 64, 64, True, (F, F, F)),
-    (0, 0, 17, 300, 16, 128, False, (F, F, F)),   # more keys than rows, value tiles of 8
-    (6, 2, 50, 50, 128, 16, True, (F, F, F)),     # grouped heads, d above the value size
-    (4, 4, 20, 5, 48, 32, False, (B, F, B)),      # fewer keys than a tile, stored types mixed
+    (0, 0, 65, 300, 16, 128, False, (F, F, F)),   # more keys than rows, value tiles of 8
+    (6, 2, 60, 60, 128, 16, True, (F, F, F)),     # grouped heads, d above the value size
+    (16, 16, 260, 5, 48, 32, False, (B, F, B)),   # fewer keys than a tile, stored types mixed
 ])
 def test_attention_f32_matches_generic(dev, monkeypatch, NH, NKV, NQ, T, HD, E, causal, dtypes):
     """Both evaluations are f32 throughout: scores within HD · 2^-24 of Σ|q·k| ≤ HD of each other,
