@@ -186,6 +186,37 @@ bool rising_edge(const sanic_program_desc* d, int node, const std::vector<int>& 
     return false;
 }
 
+// The value of a window edge at a query row, where it is made of constants and the row alone.
+double edge_at(const sanic_program_desc* d, int node, const std::vector<int>& b, int qdim, double row, bool& known) {
+    const sanic_node& n = d->nodes[node];
+    if (n.kind == SANIC_NODE_CONST) return n.value;
+    if (n.kind == SANIC_NODE_COORDINATE && b[n.dim] == qdim) return row;
+    if (n.kind == SANIC_NODE_IOTA && b[0] == qdim) return row;
+    if (n.kind == SANIC_NODE_MAP && n.n_in == 2 && (n.op == SANIC_OP_ADD || n.op == SANIC_OP_SUB || n.op == SANIC_OP_MUL)) {
+        const double x = edge_at(d, n.in[0], kid_bind(d, node, 0, b), qdim, row, known);
+        const double y = edge_at(d, n.in[1], kid_bind(d, node, 1, b), qdim, row, known);
+        return n.op == SANIC_OP_ADD ? x + y : n.op == SANIC_OP_SUB ? x - y : x * y;
+    }
+    known = false;
+    return 0.0;
+}
+
+// Keys that the last `rows` query rows see between them (all, where an edge is not known here).
+int64_t longest_window(const sanic_program_desc* d, const sanic_stage& st, int qdim, int64_t nq, int64_t rows) {
+    double lo = 0.0, hi = (double)st.stream;
+    for (auto& w : honest_window(d, st)) {
+        bool known = true;
+        if (w.kind == WindowBound::LO_CEIL) {
+            const double v = edge_at(d, w.node, w.bind, qdim, (double)std::max<int64_t>(0, nq - rows), known);
+            if (known) lo = std::max(lo, v);
+        } else {
+            const double v = edge_at(d, w.node, w.bind, qdim, (double)(nq - 1), known);
+            if (known) hi = std::min(hi, v + 1.0);
+        }
+    }
+    return hi > lo ? (int64_t)(hi - lo) : st.stream;
+}
+
 // The attention structure of a stage: carrier, dims and the affine K and V (any storage dtype).
 bool attention_plan(const sanic_program_desc* d, int si, FlashPlan& P) {
     const sanic_stage& st = d->stages[si];
@@ -334,12 +365,26 @@ bool lower_flash_prefill(const sanic_program_desc* d, int si, int64_t& scratch, 
     // query tile per wave holds the second operands in the registers the second tile had (115
     // VGPRs) and gives short prompts twice the workgroups. 32/8 heads, S = 1000, window 256, with
     // the RoPE stages: 20.0 ms in the generic fold (it forms q·k again for each of the 64 value
-    // columns) → 23.3 µs, the same 2.2e-3 from a 64-bit evaluation.
+    // columns) → 20.1 µs, the same 2.2e-3 from a 64-bit evaluation.
     const bool hilo = P.ragged;
     const int fvar = P.ragged ? 0 : d->stages[si].sched.variant;
-    const int QT = P.ragged ? 1 : 2;                 // 16-row query tiles per wave
-    const int RB = 64 * QT;                          // query rows per workgroup (4 waves)
+    // Launches that leave CUs short of waves: 64-row blocks (up to 512 of 128 rows; 32 heads, S = 2048
+    // 58 → 47 µs, S = 4096, 1024 blocks, 108 against 123), and KS teams of 4 waves per block, each with
+    // every KS-th key tile, merged in LDS at the end — a wave's tile takes ≈ 1.5 µs of dependent phases
+    // whatever else the CU does, so the key loop's length is the time. One, 2 and 4 teams: 4/1 heads,
+    // S = 2048 40 / 30 / 24 µs; 8 heads, S = 4096 75 / 53 / 51; 16 heads, S = 2048 (512 blocks) 44 / 35 / 37;
+    // 16 heads, S = 4096 (1024 blocks) 78 / 70 / 87, S = 2048, 32 heads 47 / 49 / 63; and with few tiles the
+    // merge costs more: 6 tiles (S = 1000, window 256) 20 / 22 / 29, 2 tiles 11.6 / 12.4.
+    const bool few = P.ragged || (NH * (NQ / 128) <= 512 && (fvar == 0 || fvar == 3));
+    const int QT = few ? 1 : 2;                      // 16-row query tiles per wave
+    const int RB = 64 * QT;                          // query rows per workgroup (a team's 4 waves)
     const int64_t NQB = (NQ + RB - 1) / RB;
+    const int64_t tiles = longest_window(d, st, P.qdim, NQ, RB) / 64 + 1;
+    int KS = 1;
+    if (few && tiles >= 12 && NH * NQB <= 256) KS = 4;
+    else if (few && ((tiles >= 8 && NH * NQB <= 512) || (tiles >= 48 && NH * NQB <= 1024))) KS = 2;
+    const int NBUF = KS > 1 ? 2 : 3;                 // LDS buffers of a team's tile ring
+    const std::string KSs = std::to_string(KS), step = std::to_string(64 * KS);
     const std::string QTs = std::to_string(QT), RBs = std::to_string(RB);
     // the last row or key of the operands, where a tile runs past it
     auto row_clamp = [&](const std::string& r) { return P.ragged ? "sanic_min(" + r + ", (idx_t)" + std::to_string(NQ - 1) + ")" : "(" + r + ")"; };
@@ -508,10 +553,10 @@ bool lower_flash_prefill(const sanic_program_desc* d, int si, int64_t& scratch, 
     // unpadded with the 16-byte chunk index XORed by (row mod 8): a padded stride would put the
     // 16 rows of one fragment read into 2-way bank conflicts on gfx950, and the direct loads
     // write each wave's 1 KB contiguously, so the swizzle is applied to the source addresses.
-    k.line("__shared__ __attribute__((aligned(16))) unsigned short kv_lds[3][2][64 * 64];");
+    k.line("__shared__ __attribute__((aligned(16))) unsigned short kv_lds[" + std::to_string(KS * NBUF) + "][2][64 * 64];");
     // (the wave index through a scalar register: the LDS destinations of the direct loads and
     // the wave's row range are then scalar arithmetic)
-    k.line("const int tid = threadIdx.x, lane = tid & 63, wv = __builtin_amdgcn_readfirstlane(tid >> 6);");
+    k.line("const int tid = threadIdx.x, lane = tid & 63, wv = __builtin_amdgcn_readfirstlane(tid >> 6)" + std::string(KS > 1 ? " & 3, kg = __builtin_amdgcn_readfirstlane(tid >> 8)" : "") + ";");
     k.line("const int l16 = lane & 15, lq = lane >> 4;");
     // XCD-aware block order: blockIdx mod 8 picks the KV head group, heaviest query blocks first
     const int64_t NKV = NH / P.rep;
@@ -725,20 +770,38 @@ bool lower_flash_prefill(const sanic_program_desc* d, int si, int64_t& scratch, 
     k.line("};");
     k.line("if (klo_s < khi_s) {");
     k.indent++;
-    k.line("fetch(klo_s, 0);");
-    k.line("if (klo_s + 64 < khi_s) fetch(klo_s + 64, 1);");
+    if (KS > 1) {
+        k.line("int buf = kg * " + std::to_string(NBUF) + ";");
+        k.line("if (klo_s + 64 * kg < khi_s) fetch(klo_s + 64 * kg, buf);");
+    } else {
+        k.line("fetch(klo_s, 0);");
+        k.line("if (klo_s + 64 < khi_s) fetch(klo_s + 64, 1);");
+    }
     if (P.qexpr) emit_qexpr();
-    k.line("int buf = 0;");
-    k.line("for (int t0 = klo_s; t0 < khi_s; t0 += 64) {");
-    k.indent++;
+    if (KS > 1) {
+        // every team runs every iteration (the barriers are the workgroup's); past its last tile it
+        // neither fetches nor folds
+        k.line("for (int tb = klo_s; tb < khi_s; tb += " + step + ") {");
+        k.indent++;
+        k.line("const int t0 = tb + 64 * kg;");
+    } else {
+        k.line("int buf = 0;");
+        k.line("for (int t0 = klo_s; t0 < khi_s; t0 += 64) {");
+        k.indent++;
+    }
     // this tile's transfers have landed for every wave (only the next tile's four may still be
     // in flight; loads complete in issue order). The buffer the transfer below refills was read
     // in the previous iteration: this barrier orders every wave's reads of it before the refill,
     // so the refill must stay after the barrier. The asm carries the memory clobber that keeps
     // the compiler from moving LDS accesses across the barrier.
+    if (KS > 1) {
+        k.line("asm volatile(\"s_waitcnt vmcnt(0)\\n\\ts_barrier\" ::: \"memory\");");
+        k.line("if (t0 + " + step + " < khi_s) fetch(t0 + " + step + ", buf ^ 1);");
+    } else {
     k.line("if (t0 + 64 < khi_s) asm volatile(\"s_waitcnt vmcnt(4)\\n\\ts_barrier\" ::: \"memory\");");
     k.line("else asm volatile(\"s_waitcnt vmcnt(0)\\n\\ts_barrier\" ::: \"memory\");");
     k.line("if (t0 + 128 < khi_s) fetch(t0 + 128, buf == 0 ? 2 : buf - 1);");
+    }
     // wave-uniform tile classification (scalar branches)
     k.line("const int live = t0 < whi_s && t0 + 64 > wlo_s;");   // some row sees it
     k.line("if (live) {");
@@ -989,17 +1052,52 @@ bool lower_flash_prefill(const sanic_program_desc* d, int si, int64_t& scratch, 
         k.line("    const uint2 lo4 = *(const uint2*)(vr), hi4 = *(const uint2*)(vr2);");
         k.line("    const bf16x8 va = __builtin_bit_cast(bf16x8, (sanic_u32x4){lo4.x, lo4.y, hi4.x, hi4.y});");
     }
-    k.line("    o[dt][0] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(va, pf[0][ks], o[dt][0], 0, 0, 0);");
-    k.line("    o[dt][1] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(va, pf[1][ks], o[dt][1], 0, 0, 0);");
+    for (int qt = 0; qt < QT; qt++) {
+        const std::string q = std::to_string(qt);
+        k.line("    o[dt][" + q + "] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(va, pf[" + q + "][ks], o[dt][" + q + "], 0, 0, 0);");
+    }
     k.line("  }");
     }
     k.indent--;
     k.line("}");
-    k.line("buf = buf == 2 ? 0 : buf + 1;");
+    k.line(KS > 1 ? "buf ^= 1;" : "buf = buf == 2 ? 0 : buf + 1;");
     k.indent--;
     k.line("}");
     k.indent--;
     k.line("}");
+    if (KS > 1) {
+        // the teams' carriers meet in LDS (over the tile rings, once every wave is done with them):
+        // the first team's waves take the others' in order, by the ExpShifted combine with its −∞ guard
+        const std::string slots = std::to_string(18 * QT * 64);
+        k.line("__syncthreads();");
+        k.line("float* mg = (float*)kv_lds + lane;");
+        k.line("if (kg > 0) {");
+        k.line("  float* to = mg + ((kg - 1) * 4 + wv) * " + slots + ";");
+        k.line("  #pragma unroll");
+        k.line("  for (int qt = 0; qt < " + QTs + "; ++qt) {");
+        k.line("    #pragma unroll");
+        k.line("    for (int i = 0; i < 16; ++i) to[(qt * 18 + i) * 64] = o[i / 4][qt][i % 4];");
+        k.line("    to[(qt * 18 + 16) * 64] = m_run[qt];");
+        k.line("    to[(qt * 18 + 17) * 64] = lsum[qt][0];");
+        k.line("  }");
+        k.line("}");
+        k.line("__syncthreads();");
+        k.line("if (kg > 0) return;");
+        k.line("#pragma unroll");
+        k.line("for (int g = 0; g < " + std::to_string(KS - 1) + "; ++g) {");
+        k.line("  const float* from = mg + (g * 4 + wv) * " + slots + ";");
+        k.line("  #pragma unroll");
+        k.line("  for (int qt = 0; qt < " + QTs + "; ++qt) {");
+        k.line("    const float mo = from[(qt * 18 + 16) * 64], M = __builtin_fmaxf(m_run[qt], mo);");
+        k.line("    const float ws = m_run[qt] == -__builtin_huge_valf() ? 0.0f : __builtin_amdgcn_exp2f((m_run[qt] - M) * " + flit(LOG2E) + ");");
+        k.line("    const float wo = mo == -__builtin_huge_valf() ? 0.0f : __builtin_amdgcn_exp2f((mo - M) * " + flit(LOG2E) + ");");
+        k.line("    lsum[qt][0] = __builtin_fmaf(lsum[qt][0], ws, from[(qt * 18 + 17) * 64] * wo);");
+        k.line("    m_run[qt] = M;");
+        k.line("    #pragma unroll");
+        k.line("    for (int i = 0; i < 16; ++i) o[i / 4][qt][i % 4] = __builtin_fmaf(o[i / 4][qt][i % 4], ws, from[(qt * 18 + i) * 64] * wo);");
+        k.line("  }");
+        k.line("}");
+    }
     int64_t soff = -1;
     if (SPL > 1) {
         // partials [block][part][36][256 lanes] (o in accumulator order, m, ℓ), and one arrival
@@ -1095,8 +1193,9 @@ bool lower_flash_prefill(const sanic_program_desc* d, int si, int64_t& scratch, 
     // register cap costs a few spilled values outside the inner loop)
     // tiling variants for the measured tuner: workgroups per CU {3, 2}
     int occ = fvar == 1 ? 2 : 3;
-    src << "extern \"C\" __global__ void __launch_bounds__(256, " << occ << ") " << kname << "(Args a) {\n" << R.entry() << k.str() << "}\n";
-    out.kernel_kind = "skeleton:flash_prefill[rep " + std::to_string(P.rep) + (P.ragged ? ",any length" : "") + "]" + (SPL > 1 ? "+split2" : "");
+    if (KS > 1) occ = 4;
+    src << "extern \"C\" __global__ void __launch_bounds__(" << 256 * KS << ", " << occ << ") " << kname << "(Args a) {\n" << R.entry() << k.str() << "}\n";
+    out.kernel_kind = "skeleton:flash_prefill[rep " + std::to_string(P.rep) + (P.ragged ? ",any length" : "") + "]" + (SPL > 1 ? "+split2" : "") + (KS > 1 ? "+teams" + KSs : "");
     out.source = src.str();
     out.variants = P.ragged ? 1 : 4;
     std::vector<Arg> args = R.arg_list();
@@ -1104,7 +1203,7 @@ bool lower_flash_prefill(const sanic_program_desc* d, int si, int64_t& scratch, 
         args.push_back({Arg::SCRATCH, soff});
         args.push_back({Arg::COUNTERS, take_counters(NB)});
     }
-    out.launches.push_back({kname, "", dim3((unsigned)(NB * SPL)), dim3(256), 0, args});
+    out.launches.push_back({kname, "", dim3((unsigned)(NB * SPL)), dim3((unsigned)(256 * KS)), 0, args});
     return true;
 }
 

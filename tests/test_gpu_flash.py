@@ -212,3 +212,29 @@ def test_attention_f32_matches_generic(dev, monkeypatch, NH, NKV, NQ, T, HD, E, 
             err = max_rel_err(g[fin], w[fin])
             print(odd, err)
             assert err < 2e-5
+
+
+@pytest.mark.parametrize("NH,NKV,S,window,teams", [
+    (2, 1, 1024, 0, "+teams4"),      # whole tiles, 64-row blocks
+    (12, 4, 1024 + 64, 0, "+teams4"),   # 17 tiles over 4 teams: teams of 4 and 5
+    (1, 1, 800, 0, "+teams4"),       # a single head, 13 tiles, the last of them partial
+    (32, 8, 600, 0, "+teams2"),      # 320 blocks: 2 teams
+    (2, 1, 1024, 200, ""),           # a window of 5 tiles: one team
+])
+def test_flash_key_teams(dev, NH, NKV, S, window, teams):
+    """Small launches: teams of waves over every 2nd or 4th key tile, merged at the end, against the
+    fused f64 attention over the same RoPE'd, bf16-rounded K (and Q, where the kernel rounds it)."""
+    prog = configs.flash_prefill(NH, NKV, S, window=window)
+    vals = _inputs(NH, NKV, S, seed=520 + S)
+    got, exe = run_on_gpu(dev, prog, vals)
+    kind = exe.stage_kernel(2)
+    assert kind.startswith("skeleton:flash_prefill") and kind.endswith("]" + teams), kind
+    invf = oracle.inv_freq(500000.0, 32)
+    kr = _round_bf16_array(oracle.rope(vals["K"], 0, invf))
+    qr = oracle.rope(vals["Q"], 0, invf)
+    if "any length" not in kind:
+        qr = _round_bf16_array(qr)
+    want = oracle.attention(qr, kr, vals["V"], 1.0 / 8.0, mask=2 if window else 1, window=window)
+    err = max_rel_err(got["O"], want)
+    print(kind, err)
+    assert err < 2e-2
