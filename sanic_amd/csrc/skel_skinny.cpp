@@ -10,7 +10,9 @@
 // bytes of each weight row, 128 for 4-bit; SK rows of a [K, N] weight). A wave requests the row
 // runs and then the weights of its stages as whole 128-byte lines, builds its A fragments while
 // the weights are in flight, and turns each stage into B fragments through an LDS slot of its own;
-// no barrier until the waves' partial tiles meet in LDS, summed in wave order. A 4-bit weight goes
+// no barrier until the waves' partial tiles meet in LDS, summed in wave order. Above 32 rows also
+// as 64 × 32 "tall" tiles, where the rows' own reads would pass the weights': x then takes the
+// weights' way through LDS, and the next stage is requested once this one is there. A 4-bit weight goes
 // to the MFMA as the integer q (exact in bf16) and each group folds as s·Σ x·q ± z·Σ x, Σ x from
 // the matrix cores as well. (The weights pass through registers: with direct-to-LDS transfers in
 // flight the compiler waits for all of them before the first row run is used.)
@@ -18,6 +20,8 @@
 // The bound is the weight stream. Generic fold → here, K = 2048, N = 8192: M = 8 [N, K] weights
 // 25 → 7.6 µs (33.6 MB: 4.4 TB/s), [K, N] weights 11.5 µs (14.8 before the two halves of each
 // line met on one XCD); 4-bit, M = 16: 246 → 5.8 µs. K = 8192, N = 2048, M = 8: 14.2 µs.
+// Tall tiles, 32-row ones or GEMM tiles → here: 4-bit, M = 33, N = 8192 14.9 → 10.5 µs; K = 1968,
+// N = 1088, M = 300 23.8 → 18.8 (bound by L1 misses, 30 bytes a clock and CU, as the GEMM's tiles).
 #include <algorithm>
 #include <functional>
 #include <numeric>
@@ -71,7 +75,6 @@ bool lower_skinny(const sanic_program_desc* d, int si, LoweredStage& out) {
     const int64_t M = P.M, N = P.N, K = P.K;
     int factors = 0;
     if (!sched_is_auto(st.sched) || !exact_in_two(d, st, c.into[P.cslots[0]], P.w, factors)) return false;
-    if (M % 64 == 0 && N % 32 == 0 && K % 64 == 0) return false;      // the GEMM's own tiles
     if (N < 16) return false;
 
     // ── the weight ──
@@ -102,6 +105,9 @@ bool lower_skinny(const sanic_program_desc* d, int si, LoweredStage& out) {
         if (unit == 0) unit = 256;
         packed = true;
     }
+    // The GEMM's own tiles (groups under 64 are its slowest; it has no others for them)
+    const bool aligned = M % 64 == 0 && N % 32 == 0 && K % 64 == 0, narrow = packed && unit < 64;
+    if (aligned && !narrow) return false;
     const bool signed4 = packed && wacc.dtype == SANIC_I4;
     const int run = packed ? 32 : 8;                 // elements of a 16-byte chunk
 
@@ -144,33 +150,57 @@ bool lower_skinny(const sanic_program_desc* d, int si, LoweredStage& out) {
     if (packed && SR) return false;
 
     // ── tile ──
-    const int MT = M > 16 ? 2 : 1;
-    const int64_t NMB = (M + 16 * MT - 1) / (16 * MT);
-    int BN = kn ? 64 : 32;
-    while (BN > (kn ? 32 : 16) && (NMB * ((N + BN - 1) / BN) < 200 || N < BN)) BN /= 2;
-    if (N < BN) return false;
-    const int64_t NNB = (N + BN - 1) / BN;
-    const int NT = BN / 16;
-    // Rounds of workgroups over the 256 CUs against the GEMM's (lower_gemm's tiles), in µs at the
-    // measured cost of each (K = 2048, N = 8192): a round here 9.5 at 32 rows and 5 at 16, a
-    // quarter more for a [K, N] weight; a 64-deep K step of a GEMM tile 0.3 (64 × 32), 0.55 (128 × 32),
-    // 0.68 (128 × 64), 1.05 (128 × 128), and 5 for its operand launch. Up to 32 rows the GEMM's tile is
-    // half empty (M = 32: 13.4 here, 15.0 there); M = 48: 22.5 and 15.0; N = 1088, K = 1968: M = 200
-    // 13.8 and 33.7, M = 400 24.5 and 35.9.
+    // "Tall" tiles: 64 rows × 32 columns whose x goes through LDS as the weights do (whole lines of
+    // each row; fragment loads would take 64 bytes of 16 rows each).
+    Access xacc;
+    int tall_row = -1;
+    bool tall = M > 32 && N >= 32 && !narrow;
+    for (size_t li = 0; li < P.rows.size(); li++)
+        if (moves[li]) {
+            tall &= tall_row < 0 && sym_access(d, st.leaf[P.rows[li]], crow[li], {M, K}, xacc) && contiguous_runs(xacc, 1, 8);
+            tall_row = (int)li;
+        }
+    tall &= tall_row >= 0;
+    auto columns = [&](int64_t mb) {
+        int bn = kn ? 64 : 32;
+        while (bn > (kn ? 32 : 16) && (mb * ((N + bn - 1) / bn) < 200 || N < bn)) bn /= 2;
+        return bn;
+    };
+    // Up to 32 rows a GEMM tile is half empty (M = 32: 13.4 µs here, 15.0 there). Above, the least of
+    // three estimates in µs, rounds of workgroups over the 256 CUs at what a round measured. Per 2048 k:
+    // 32-row tiles 9.5 (4-bit 6.5, in groups of 32 10.7), tall ones 12.5 (4-bit 8.5; rows that start
+    // off a line cost them 4 more), an eighth to a quarter more for a [K, N] weight. Per 64-deep K step
+    // of the GEMM: 0.3 (64 × 32), 0.55 (128 × 32), 0.68 (128 × 64), 1.05 (128 × 128), 4-bit 0.43 and
+    // 0.52 (groups of 32, whole tiles only, 0.52 and 0.68), beside 5 for its operand launch. K = 2048,
+    // N = 8192, 4-bit: M = 50 tall 12.6, GEMM 15.1, M = 100 23.5 and 17.7. N = 1088, K = 1968: M = 200
+    // 13.6 in 32-row tiles, 18.8 tall, 22.9 GEMM; M = 400 24.6, 18.8, 25.0. N = 4000, K = 1536, M = 100:
+    // 17.4 in 32-row tiles, 13.3 tall. 4-bit groups of 32, N = 3264, K = 1408, M = 64: 10.3, GEMM 11.8.
     if (M > 32) {
-        const double here = 3.0 + (double)((NMB * NNB + 255) / 256) * ((double)K / 2048.0) * (MT > 1 ? 9.5 : 5.0) * (kn ? 1.25 : 1.0);
+        const double kd = (double)K / 2048.0;
+        auto rounds = [](int64_t blocks) { return (double)((blocks + 255) / 256); };
+        const int64_t mb2 = (M + 31) / 32, bn2 = columns(mb2), mb4 = (M + 63) / 64;
+        const double small = 3.0 + rounds(mb2 * ((N + bn2 - 1) / bn2)) * kd * (narrow ? 10.7 : packed ? 6.5 : 9.5) * (kn ? 1.25 : 1.0);
+        const double high = 3.0 + rounds(mb4 * ((N + 31) / 32)) * kd * (packed ? 8.5 : 12.5) * (kn ? 1.125 : 1.0) + (K % 64 ? 4.0 : 0.0);
         const int64_t bm = M > 64 ? 128 : 64, mb = (M + bm - 1) / bm;
         int64_t bn = 128;
         while (bn > 32 && mb * (N / bn) < 256) bn /= 2;
-        const double step = bn == 128 ? 1.05 : bn == 64 ? 0.68 : bm == 64 ? 0.3 : 0.55;
-        const double there = (split ? 5.0 : 0.0) + (double)((mb * ((N + bn - 1) / bn) + 255) / 256) * (double)((K + 63) / 64) * step;
-        if (N >= bn && there < here) return false;
+        const double step = narrow ? (bm == 64 ? 0.52 : 0.68) : bn == 128 ? 1.05 : bn == 64 ? 0.68 : bm == 64 ? (packed ? 0.43 : 0.3) : packed ? 0.52 : 0.55;
+        const double gemm = (split ? 5.0 : narrow ? 1.5 : 0.0) + rounds(mb * ((N + bn - 1) / bn)) * (double)((K + 63) / 64) * step;
+        if (N >= bn && (!narrow || aligned) && gemm < std::min(small, tall ? high : small)) return false;
+        tall &= high < small;
     }
-    const int SK = kn ? 64 : packed ? 256 : 128;                  // k of a stage
+    if (!tall) tall_row = -1;
+    const int MT = tall ? 4 : M > 16 ? 2 : 1;
+    const int64_t NMB = (M + 16 * MT - 1) / (16 * MT);
+    const int BN = tall ? 32 : columns(NMB);
+    if (N < BN) return false;
+    const int64_t NNB = (N + BN - 1) / BN;
+    const int NT = BN / 16;
+    const int SK = kn || tall ? 64 : packed ? 256 : 128;          // k of a stage
     const int64_t ST = (K + SK - 1) / SK;
     // 16 waves with one stage each where that covers K (128 registers a lane hold one stage), else
     // 8 waves (256 registers) with the next stage requested ahead of each stage's arithmetic
-    const int WMAX = ST <= 16 ? 16 : 8;
+    const int WMAX = ST <= 16 && !tall ? 16 : 8;
     const int ITER = (int)((ST + WMAX - 1) / WMAX), NW = (int)((ST + ITER - 1) / ITER);
     const int SB = kn ? SK * BN * 2 : BN * (packed ? SK / 2 : SK * 2);   // LDS bytes of a stage
     const int ND = SB / 1024;                                     // loads of a stage, 1 KB a wave each
@@ -178,8 +208,10 @@ bool lower_skinny(const sanic_program_desc* d, int si, LoweredStage& out) {
     const int RPI = 64 / LPR;                                     // rows of a load
     const bool tail = K % SK != 0;
     const int NTH = NW * 64, RBM = 16 * MT;
+    const int XB = tall ? RBM * SK * 2 : 0, NX = XB / 1024;       // x of a stage: LDS bytes, loads
     const int64_t red = (int64_t)NW * MT * NT * 1024;
-    const int64_t lds = std::max<int64_t>((int64_t)NW * SB, red);
+    const int64_t lds = std::max<int64_t>((int64_t)NW * (SB + XB), red);
+    if (tall && unit > SK) unit = SK;
     const int STEPS = SK / 32, UNITS = packed ? SK / (int)unit : 1;
 
     Code k;
@@ -213,10 +245,11 @@ bool lower_skinny(const sanic_program_desc* d, int si, LoweredStage& out) {
     std::vector<int> aoff(P.rows.size());
     int NA = 0;
     for (size_t li = 0; li < P.rows.size(); li++) {
+        if ((int)li == tall_row) continue;
         aoff[li] = NA;
         NA += STEPS * (moves[li] ? MT : 1);
     }
-    auto aix = [&](size_t li, int j, int mt) { return "ar[" + str(aoff[li] + j * (moves[li] ? MT : 1) + (moves[li] ? mt : 0)) + "]"; };
+    auto aix = [&](size_t li, int j, int mt) { return (int)li == tall_row ? "xf_" + str(j) + "_" + str(mt) : std::string(tall ? "cur[" : "ar[") + str(aoff[li] + j * (moves[li] ? MT : 1) + (moves[li] ? mt : 0)) + "]"; };
     std::vector<std::string> zname, ztype;           // held words, in order of appearance
     std::vector<std::vector<std::pair<std::string, std::string>>> sz(UNITS);
     std::vector<std::string> szdc(UNITS);
@@ -232,6 +265,7 @@ bool lower_skinny(const sanic_program_desc* d, int si, LoweredStage& out) {
         }
         for (size_t li = 0; li < P.rows.size(); li++)
             for (int mt = 0; mt < (moves[li] ? MT : 1); mt++) {
+                if ((int)li == tall_row) continue;
                 const std::string sfx = "_" + str(j) + "_" + str(mt) + "_" + str(li);
                 std::vector<int> rb, rd;
                 bool rok = true, rc = true;
@@ -242,7 +276,7 @@ bool lower_skinny(const sanic_program_desc* d, int si, LoweredStage& out) {
                 for (size_t b = 0; b < rb.size(); b++)
                     rq.line("const " + std::string(ctype_of(rd[b])) + "* __restrict__ wb" + str(b) + sfx + " = " + R.param(rb[b]) + ";");
                 rq.s << l1.str();
-                rq.line(aix(li, j, mt) + " = " + rr + ";");
+                rq.line("ar[" + str(aoff[li] + j * (moves[li] ? MT : 1) + (moves[li] ? mt : 0)) + "] = " + rr + ";");
             }
     }
     if (packed)
@@ -268,11 +302,21 @@ bool lower_skinny(const sanic_program_desc* d, int si, LoweredStage& out) {
                     rq.line("z" + str(zname.size()) + " = " + (*m)[2].str() + ";");
                     zname.push_back((*m)[2]);
                     ztype.push_back((*m)[1]);
-                    szdc[u] += "      const " + ztype.back() + " " + zname.back() + " = z" + str(zname.size() - 1) + ";\n";
+                    szdc[u] += "      const " + ztype.back() + " " + zname.back() + (tall ? " = zc" : " = z") + str(zname.size() - 1) + ";\n";
                 }
                 szdc[u] += d1.str();
                 sz[u].push_back({A_, B_});
             }
+    if (tall) {
+        // x: rows of the block (a row past the last repeats it), whole 128-byte lines
+        rq.line("#pragma unroll");
+        rq.line("for (int i = 0; i < " + str(NX) + "; ++i) {");
+        rq.line("  const int r = i * 8 + lane / 8, ch = (lane % 8) ^ (r & 7);");
+        const std::string mr = "(m0 + r)", kk = "(" + sk + "ch * 8)";
+        rq.line("  const idx_t mm = " + (M % RBM ? mr + " < " + str(M) + " ? " + mr + " : (idx_t)" + str(M - 1) : mr) + ", kk = " + (tail ? kk + " < " + str(K) + " ? " + kk + " : (idx_t)" + str(K - 8) : kk) + ";");
+        rq.line("  xr[i] = *(const sanic_u32x4_any*)(" + R.param(xacc.buffer) + " + " + xacc.addr.render({"mm", "kk"}) + ");");
+        rq.line("}");
+    }
     wq.line("#pragma unroll");
     wq.line("for (int i = 0; i < " + str(ND) + "; ++i) {");
     wq.indent++;
@@ -288,7 +332,7 @@ bool lower_skinny(const sanic_program_desc* d, int si, LoweredStage& out) {
     wq.line("}");
     std::string zargs, zdecl;
     for (size_t z = 0; z < zname.size(); z++) zargs += ", " + ztype[z] + "& z" + str(z);
-    const std::string params = "int s, sanic_u32x4 (&ar)[" + str(NA) + "], sanic_u32x4 (&wr)[" + str(ND) + "]" + zargs;
+    const std::string params = "int s, sanic_u32x4 (&ar)[" + str(std::max(NA, 1)) + "], " + (tall ? "sanic_u32x4 (&xr)[" + str(NX) + "], " : std::string()) + "sanic_u32x4 (&wr)[" + str(ND) + "]" + zargs;
     k.line("auto request = [&](" + params + ") {");
     k.s << rq.str();
     // (the row runs ahead of the weights: loads complete in issue order)
@@ -296,13 +340,12 @@ bool lower_skinny(const sanic_program_desc* d, int si, LoweredStage& out) {
     k.s << wq.str();
     k.line("  __builtin_amdgcn_sched_barrier(0);");
     k.line("};");
-    k.line("auto consume = [&](" + params + ") {");
+    k.line("auto consume = [&](" + params + (tall ? ", int next" : "") + ") {");
     k.indent++;
-    // A fragments (and the row slots), while the weights are in flight
+    // A fragments (and the row slots): while the weights are in flight, or of a tall tile a step at a time
     auto own = [&](int j) { return sk + str(j * 32) + " + lq * 8 < " + str(K); };
     const char* comp[4] = {"x", "y", "z", "w"};
-    for (int j = 0; j < STEPS; j++)
-        for (int mt = 0; mt < MT; mt++) {
+    auto fragment = [&](int j, int mt) {
             const std::string fs = "_" + str(j) + "_" + str(mt);
             auto item = [&, j, mt](int e) {
                 return [&, j, mt, e](int i) -> std::string {
@@ -331,12 +374,33 @@ bool lower_skinny(const sanic_program_desc* d, int si, LoweredStage& out) {
                 }
             R.memo.pop_back();
             k.line("}");
-        }
+    };
+    if (!tall)
+        for (int j = 0; j < STEPS; j++)
+            for (int mt = 0; mt < MT; mt++) fragment(j, mt);
     k.line("__builtin_amdgcn_sched_barrier(0);");
     // the stage through this wave's LDS slot (its own reads of the last one are done)
-    k.line("unsigned char* slot = lds + wv * " + str(SB) + ";");
+    k.line("unsigned char* slot = lds + wv * " + str(SB + XB) + ";");
+    if (tall) {
+        k.line("#pragma unroll");
+        k.line("for (int i = 0; i < " + str(NX) + "; ++i) *(sanic_u32x4*)(slot + " + str(SB) + " + i * 1024 + lane * 16) = xr[i];");
+    }
+    const std::string write = "for (int i = 0; i < " + str(ND) + "; ++i) *(sanic_u32x4*)(slot + i * 1024 + lane * 16) = wr[i];";
     k.line("#pragma unroll");
-    k.line("for (int i = 0; i < " + str(ND) + "; ++i) *(sanic_u32x4*)(slot + i * 1024 + lane * 16) = wr[i];");
+    k.line(write);
+    if (tall) {
+        // the stage is in LDS: its registers take the next one while this one is folded
+        if (NA) {
+            k.line("sanic_u32x4 cur[" + str(NA) + "];");
+            k.line("#pragma unroll");
+            k.line("for (int i = 0; i < " + str(NA) + "; ++i) cur[i] = ar[i];");
+        }
+        for (size_t z = 0; z < zname.size(); z++) k.line("const " + ztype[z] + " zc" + str(z) + " = z" + str(z) + ";");
+        std::string zs;
+        for (size_t z = 0; z < zname.size(); z++) zs += ", z" + str(z);
+        k.line("__builtin_amdgcn_sched_barrier(0);");
+        k.line("request(next, ar, xr, wr" + zs + ");");
+    }
     const int per = packed ? (int)unit / 32 : STEPS;      // steps of a fold unit
     for (int j = 0; j < STEPS; j++) {
         const int u = packed ? j / per : 0;
@@ -388,10 +452,16 @@ bool lower_skinny(const sanic_program_desc* d, int si, LoweredStage& out) {
             }
         } else {
             for (int nt = 0; nt < NT; nt++)
-                k.line("bf[" + str(nt) + "] = *(const bf16x8*)(slot + ((" + str(nt * 16) + " + l16) * " + str(LPR) + " + ((" + str(j * 4) + " + lq) ^ l16)) * 16);");
+                k.line("bf[" + str(nt) + "] = *(const bf16x8*)(slot + ((" + str(nt * 16) + " + l16) * " + str(LPR) + " + ((" + str(j * 4) + " + lq) ^ (l16 & " + str(LPR - 1) + "))) * 16);");
         }
         for (int mt = 0; mt < MT; mt++) {
             const std::string ms = str(mt), fs = "_" + str(j) + "_" + ms;
+            if (tall) {
+                // (row tiles past the last row are left out)
+                if (M % RBM && mt) k.line("if (m0 + " + str(mt * 16) + " < " + str(M) + ") {");
+                k.line("const sanic_u32x4 xf" + fs + " = *(const sanic_u32x4*)(slot + " + str(SB) + " + ((" + str(mt * 16) + " + l16) * 8 + ((" + str(j * 4) + " + lq) ^ (l16 & 7))) * 16);");
+                fragment(j, mt);
+            }
             for (int h = 0; h < (split ? 2 : 1); h++) {
                 const std::string af = std::string("__builtin_bit_cast(bf16x8, ") + (h ? "al" : "ah") + fs + ")";
                 for (int nt = 0; nt < NT; nt++) {
@@ -400,6 +470,7 @@ bool lower_skinny(const sanic_program_desc* d, int si, LoweredStage& out) {
                 }
                 if (packed) k.line("xq[" + ms + "] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(" + af + ", ones8, xq[" + ms + "], 0, 0, 0);");
             }
+            if (tall && M % RBM && mt) k.line("}");
         }
         k.indent--;
         k.line("}");
@@ -422,19 +493,29 @@ bool lower_skinny(const sanic_program_desc* d, int si, LoweredStage& out) {
     k.line("};");
     // wave wv takes stages wv, wv + NW, ...; a request past the last stage repeats that one
     auto hold = [&](const std::string& t) {
-        k.line("sanic_u32x4 ar" + t + "[" + str(NA) + "], wr" + t + "[" + str(ND) + "];");
+        k.line("sanic_u32x4 ar" + t + "[" + str(std::max(NA, 1)) + "], wr" + t + "[" + str(ND) + "];");
+        if (tall) k.line("sanic_u32x4 xr" + t + "[" + str(NX) + "];");
         for (size_t z = 0; z < zname.size(); z++) k.line(ztype[z] + " z" + t + str(z) + ";");
     };
     auto call = [&](const std::string& fn, const std::string& s, const std::string& t) {
         std::string zs;
         for (size_t z = 0; z < zname.size(); z++) zs += ", z" + t + str(z);
-        k.line(fn + "(" + s + ", ar" + t + ", wr" + t + zs + ");");
+        const std::string next = tall && fn.find("consume") != std::string::npos ? ", stage(it + 1)" : "";
+        k.line(fn + "(" + s + ", ar" + t + (tall ? ", xr" + t : std::string()) + ", wr" + t + zs + next + ");");
     };
     const std::string last = str(ST - 1);
     k.line("auto stage = [&](int it) { const int s = wv + it * " + str(NW) + "; return s < " + str(ST) + " ? s : " + last + "; };");
     hold("a");
     call("request", "stage(0)", "a");
-    if (ITER == 1) {
+    if (tall) {
+        k.line("for (int it = 0; it < " + str(ITER) + "; ++it) {");
+        k.indent++;
+        k.line("if (wv + it * " + str(NW) + " < " + str(ST) + ") {");
+        call("  consume", "stage(it)", "a");
+        k.line("}");
+        k.indent--;
+        k.line("}");
+    } else if (ITER == 1) {
         call("consume", "wv", "a");
     } else {
         hold("b");
@@ -526,7 +607,7 @@ bool lower_skinny(const sanic_program_desc* d, int si, LoweredStage& out) {
            "  lo = pk_bf16(x - __uint_as_float(h << 16), y - __uint_as_float(h & 0xFFFF0000u));\n}\n";
     src << R.args_struct({});
     src << "extern \"C\" __global__ void __launch_bounds__(" << NTH << ") " << kname << "(Args a) {\n" << R.entry() << k.str() << "}\n";
-    out.kernel_kind = "skeleton:gemm_rows[" + str(RBM) + "x" + str(BN) + (split ? ",a2" : "") + (packed ? ",grp" : "") + (kn ? ",kn" : "") + ",w" + str(NW) + "x" + str(ITER) + "]";
+    out.kernel_kind = "skeleton:gemm_rows[" + str(RBM) + "x" + str(BN) + (split ? ",a2" : "") + (packed ? unit < 64 ? ",g32" : ",grp" : "") + (kn ? ",kn" : "") + ",w" + str(NW) + "x" + str(ITER) + "]";
     out.variants = 1;
     out.source = src.str();
     out.launches.push_back({kname, "", dim3((unsigned)(NMB * NNB)), dim3((unsigned)NTH), 0, R.arg_list()});

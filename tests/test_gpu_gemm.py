@@ -123,7 +123,8 @@ def _same_as_generic(dev, monkeypatch, prog, vals, scale):
 # rows, k and columns off every tile: below one tile, one past it, K tiles odd in number and
 # overlapping, columns not a multiple of 8
 RAGGED = [(2, 64, 32), (65, 128, 96), (200, 2048, 8192), (33, 200, 77), (100, 72, 1003), (129, 1000, 333),
-          (256, 128, 8224), (127, 832, 5184), (8, 4160, 96), (20, 2200, 49), (40, 2048, 8192)]
+          (256, 128, 8224), (127, 832, 5184), (8, 4160, 96), (20, 2200, 49), (40, 2048, 8192), (300, 2000, 1088), (250, 2056, 2000),
+          (90, 1536, 2820)]
 
 
 @pytest.mark.parametrize("kmajor", [False, True])
@@ -143,7 +144,7 @@ def test_rmsnorm_gemm_any_size(dev, monkeypatch, M, K, N, kmajor):
 
 @pytest.mark.parametrize("M,K,N,G", [(2, 64, 32, 64), (16, 2048, 8192, 64), (100, 1152, 777, 64), (65, 384, 1000, 128),
                                      (33, 192, 64, 64), (17, 256, 300, 32), (31, 8320, 48, 64),
-                                     (16, 512, 16, 512)])
+                                     (16, 512, 16, 512), (100, 1920, 3270, 64), (103, 1920, 777, 32), (128, 512, 512, 32)])
 def test_int4_gemm_any_size(dev, monkeypatch, M, K, N, G):
     prog = configs.int4_matmul(M=M, K=K, N=N, G=G)
     s = _bf16_vals(331, N * K // G, 0.001, 0.02, kind="uniform").reshape(N, K // G)
