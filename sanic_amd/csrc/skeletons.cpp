@@ -277,8 +277,8 @@ struct VecW {
             int64_t step = 0;
             for (auto& t : cs.terms) {
                 if (t.var != kv) continue;
-                if (t.div == 1 && t.mod == 0) step += t.coef;
-                else if (t.div % 8 != 0 || (t.div == 1 && t.mod % 8 != 0)) { ok = false; return {}; }
+                if (t.div == 1 && t.mod % 8 == 0) step += t.coef;
+                else if (t.div % 8 != 0) { ok = false; return {}; }
             }
             std::string base = fresh("ci");
             lc.line("const float " + base + " = (float)(" + cs.render(names()) + ");");

@@ -4,6 +4,7 @@ import pytest
 
 import oracle
 from sanic_amd import configs, ir
+from sanic_amd.program import SCRATCH, Program
 from tests.util import floored_rel_err, max_rel_err, run_on_gpu
 
 pytestmark = pytest.mark.gpu
@@ -238,3 +239,26 @@ def test_flash_key_teams(dev, NH, NKV, S, window, teams):
     err = max_rel_err(got["O"], want)
     print(kind, err)
     assert err < 2e-2
+
+
+@pytest.mark.parametrize("S,H,F", [(1, 1, 8), (33, 1, 8), (128, 3, 32), (77, 2, 24)])
+def test_rotation_table_and_keys_in_one_launch(dev, monkeypatch, S, H, F):
+    """The rotation table and the keys rotated by it, formed in one launch, against the two generic
+    stages: the table bit for bit, the keys within a bf16 step and what contracting the other of the
+    two products changes in f32. Workgroups past the table's runs, partly filled ones, one run."""
+    p = Program()
+    k = p.input("K", (H, S, 2 * F), ir.BF16)
+    invf = ir.map_(ir.EXP, ir.map_(ir.MUL, ir.iota(F), ir.const(-0.4)))
+    table = p.pointwise("table", ir.rope_table(ir.iota(S), invf), ir.F32, role=SCRATCH)
+    kr = p.pointwise("Kr", ir.rope_tabled(k, table), ir.BF16, role=SCRATCH)
+    p.pointwise("Y", ir.map_(ir.MUL, kr, ir.const(1.0)), ir.F32)
+    p.pointwise("T", ir.map_(ir.MUL, table, ir.const(1.0)), ir.F32)
+    vals = {"K": np.random.default_rng(5).standard_normal((H, S, 2 * F))}
+    got, exe = run_on_gpu(dev, p, vals)
+    assert [exe.stage_kernel(i) for i in range(2)] == ["pointwise:runs8[2 stages]", "absorbed-into:0"]
+    monkeypatch.setenv("SANIC_HIP_GENERIC", "1")
+    want, exe = run_on_gpu(dev, p, vals)
+    assert exe.stage_kernel(1) == "pointwise"
+    np.testing.assert_array_equal(got["T"], want["T"])
+    a, b = np.asarray(got["Y"], np.float64), np.asarray(want["Y"], np.float64)
+    assert np.all(np.abs(a - b) <= 2.0 ** -7 * np.abs(b) + 2.0 ** -22 * np.abs(vals["K"]).max())
