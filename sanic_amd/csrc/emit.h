@@ -71,6 +71,10 @@ void emit_point_fold(Renderer& R, Code& code, const sanic_stage& st, const std::
 // `n` arrival counters of the program being lowered on this thread: their byte offset from the
 // program's first (a kernel argument Arg::COUNTERS).
 int64_t take_counters(int64_t n);
+// Bytes of the static scratch of sanic_hip_execute_static. A program whose first lowering needs more
+// is lowered again without the kernels that a form with less scratch can stand in for (lean).
+const int64_t kStaticScratchBytes = int64_t(32) << 20;
+bool lean_scratch();
 // Last-arriver handshake: the workgroups sharing counter `cnt` each add 1 once their partials
 // are stored; `flag` (a __shared__ int it declares) is true in the one that arrives last.
 // With xcd_local every workgroup sharing `cnt` runs on one XCD and exchanges data through

@@ -51,6 +51,8 @@ void set_xcd_local(bool on) { g_xcd_local.store(on, std::memory_order_relaxed); 
 bool xcd_local_enabled() { return g_xcd_local.load(std::memory_order_relaxed) && !getenv("SANIC_HIP_AGENT_MERGE"); }
 
 static thread_local int64_t t_counter_bytes = 0;
+static thread_local bool t_lean = false;
+bool lean_scratch() { return t_lean; }
 int64_t take_counters(int64_t n) {
     const int64_t at = t_counter_bytes;
     t_counter_bytes += (n * 4 + 255) / 256 * 256;
@@ -1556,8 +1558,7 @@ static bool stage_touches_q8(const sanic_program_desc* d, int s) {
     return false;
 }
 
-Lowered lower_program(const sanic_program_desc* d) {
-    validate(d);
+static Lowered lower_stages(const sanic_program_desc* d) {
     Lowered out;
     t_counter_bytes = 0;
     for (int s = 0; s < d->n_stages;) {
@@ -1624,6 +1625,24 @@ Lowered lower_program(const sanic_program_desc* d) {
     }
     out.counter_bytes = t_counter_bytes;
     return out;
+}
+
+Lowered lower_program(const sanic_program_desc* d) {
+    validate(d);
+    int64_t own = 0;
+    for (int i = 0; i < d->n_buffers; i++) {
+        const sanic_buffer_desc& b = d->buffers[i];
+        if (b.role == SANIC_BUF_SCRATCH) own += (dtype_bytes(b.dtype, vol(b.shape, b.rank)) + 255) / 256 * 256;
+    }
+    auto fits = [&](const Lowered& l) { return l.scratch_bytes + 255 + l.counter_bytes + own <= kStaticScratchBytes; };
+    Lowered out = lower_stages(d);
+    if (fits(out)) return out;
+    struct Lean {
+        Lean() { t_lean = true; }
+        ~Lean() { t_lean = false; }
+    } lean;
+    Lowered less = lower_stages(d);
+    return fits(less) ? std::move(less) : std::move(out);
 }
 
 }  // namespace sanic

@@ -41,7 +41,6 @@ struct sanic_hip_device {
 // its own copy until the process ends. In host code `scratch` names a host-side stand-in, not
 // a device address: host code uses only the per-device address hipGetSymbolAddress returns
 // (sanic_hip_device::scratch_ptr, taken in sanic_hip_open with the device current).
-static const size_t kStaticScratchBytes = size_t(32) << 20;
 static __device__ __align__(256) char scratch[kStaticScratchBytes];
 // The arrival counters of that entry point's programs, apart from the scratch so that no
 // program's data lies on them: zero at load, and every kernel leaves those it used at zero, so a
@@ -650,7 +649,7 @@ int sanic_hip_execute_static(sanic_hip_exe* exe, sanic_hip_buffer* const* bindin
         const bool own = counts > (int64_t)kStaticCounterBytes;
         char* cnt = own ? base + need : exe->dev->counters_ptr;
         if (own) need += counts;
-        if (need > (int64_t)kStaticScratchBytes)
+        if (need > kStaticScratchBytes)
             fail(SANIC_ERR_ARG, "this program needs " + std::to_string(need) + " bytes of scratch; the static scratch holds " +
                                     std::to_string(kStaticScratchBytes));
         SANIC_HIP(hipSetDevice(exe->dev->ordinal));

@@ -1296,7 +1296,7 @@ bool lower_flash_f32(const sanic_program_desc* d, int si, int64_t& scratch, Lowe
         }
     };
     const int64_t NQB = (NQ + 15) / 16, NB = NH * NQB, NBP = (NB + 7) / 8 * 8;
-    const int SPL = (int)std::max<int64_t>(1, std::min<int64_t>({8, 256 / NB, (T + 127) / 128}));
+    const int SPL = lean_scratch() ? 1 : (int)std::max<int64_t>(1, std::min<int64_t>({8, 256 / NB, (T + 127) / 128}));
     // the workgroups of a row block are NBP apart, a multiple of 8: on one XCD
     const bool xl = SPL > 1 && xcd_local_enabled();
     const std::string stx = xl ? "sanic_stx" : "sanic_st", ldx = xl ? "sanic_ldx" : "sanic_ld";

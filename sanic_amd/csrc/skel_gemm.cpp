@@ -333,7 +333,7 @@ bool lower_gemm(const sanic_program_desc* d, int si, int64_t& scratch, LoweredSt
     // so every fragment load is 1 KB contiguous (in 4-wave tiles, where two waves share rows,
     // both load them; the second from L1)
     const bool adirect = pre && deep && !getenv("SANIC_HIP_GEMM_ALDS");
-    if (rag && pre && !adirect) return false;
+    if (rag && pre && (!adirect || lean_scratch())) return false;
     if (grouped && BM == 128 && BN == 32 && gvar != 1) NTH = 512;
     // fragment-loaded A: every wave its own 16 rows of the block and all its columns, so that no A
     // fragment is loaded twice — a CU takes in ≈ 30 bytes a clock that miss L1, and A is most of
