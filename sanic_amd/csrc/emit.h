@@ -34,6 +34,9 @@ struct Renderer {
     explicit Renderer(const sanic_program_desc* dd) : d(dd) { memo.emplace_back(); }
 
     std::string param(int buffer);
+    // Another function of a kernel that passes the same Args names its buffers after r's, and r
+    // then takes the buffers that function added: an a.b<i> is one buffer in all of them.
+    void take_buffers(const Renderer& r) { bufs = r.bufs; buf_param = r.buf_param; }
     std::string fresh(const char* p);
     std::string args_struct(const std::vector<std::string>& extra) const;
     std::vector<Arg> arg_list() const;

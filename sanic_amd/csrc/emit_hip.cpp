@@ -1364,13 +1364,12 @@ LoweredStage lower_generic_fold(const sanic_program_desc* d, int si, int64_t& sc
     Code mb;
     mb.indent = 1;
     Renderer R2(d);
-    R2.bufs = R.bufs;
-    R2.buf_param = R.buf_param;
+    R2.take_buffers(R);
     mb.line("const idx_t gid = (idx_t)blockIdx.x * 256 + threadIdx.x;");
     mb.line("if (gid >= " + std::to_string(gvol) + ") return;");
     merge_point(R2, mb);
     // both kernels share one Args layout: the union of their buffers
-    for (int b : R2.bufs) R.param(b);
+    R.take_buffers(R2);
     src << R.args_struct({"float* __restrict__ scratch"});
     src << "extern \"C\" __global__ void __launch_bounds__(" << nth << ") sanic_fold_part(Args a) {\n" << R.entry() << body.str() << "}\n";
     src << "extern \"C\" __global__ void __launch_bounds__(256) sanic_fold_merge(Args a) {\n" << R2.entry() << mb.str() << "}\n";

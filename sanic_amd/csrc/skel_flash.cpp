@@ -413,18 +413,19 @@ bool lower_flash_prefill(const sanic_program_desc* d, int si, int64_t& scratch, 
         lc[j] = b == SANIC_BIND_STREAM ? "kj" : b == P.hdim ? "hh" : b == P.qdim ? "qi" : "0";
     }
     Renderer Rs(d);
+    Rs.take_buffers(R);
     Code sp, sf;
     sp.indent = sf.indent = 1;
     Rs.subst[P.dot_reduce] = "dotv";
     std::string vpart = Rs.value(sp, st.leaf[P.sleaf], lc);
     std::string entry_part = Rs.entry();
     Renderer Rf(d);
+    Rf.take_buffers(Rs);
     Rf.subst[P.dot_reduce] = "dotv";
     for (auto& w : win) Rf.subst[w.where_node] = "0.0f";
     std::string vfull = Rf.value(sf, st.leaf[P.sleaf], lc);
     std::string entry_full = Rf.entry();
-    for (int b : Rs.bufs) R.param(b);
-    for (int b : Rf.bufs) R.param(b);
+    R.take_buffers(Rf);
     double scale_c = 0.0;
     const bool scale_known = full_score_scale(d, st.leaf[P.sleaf], P.dot_reduce, win, scale_c) && scale_c > 0.0;
 
@@ -432,6 +433,7 @@ bool lower_flash_prefill(const sanic_program_desc* d, int si, int64_t& scratch, 
     Code wc;
     wc.indent = 1;
     Renderer Rw(d);
+    Rw.take_buffers(R);
     std::vector<std::string> gcw(st.rank, "0");
     if (P.hdim >= 0) gcw[P.hdim] = "hh";
     gcw[P.qdim] = "qrow";
@@ -443,10 +445,11 @@ bool lower_flash_prefill(const sanic_program_desc* d, int si, int64_t& scratch, 
         emit_window(Rw, tmp, st, win, "wlo", "whi");
         wc.s << tmp.str();
     }
-    for (int b : Rw.bufs) R.param(b);
+    R.take_buffers(Rw);
 
     // finish: project (+ epilogue) and the narrowing store of one output point
     Renderer Ro(d);
+    Ro.take_buffers(R);
     Code fo;
     fo.indent = 1;
     {
@@ -467,7 +470,7 @@ bool lower_flash_prefill(const sanic_program_desc* d, int si, int64_t& scratch, 
             lin = j == 0 ? "(idx_t)(" + gc[0] + ")" : "(" + lin + " * " + std::to_string(st.grid[j]) + " + (idx_t)(" + gc[j] + "))";
         fo.line(store_stmt(Ro.param(st.out_buffer), lin, st.out_dtype, v, false, d->buffers[st.out_buffer].scale));
     }
-    for (int b : Ro.bufs) R.param(b);
+    R.take_buffers(Ro);
     if (P.qexpr) {
         // register the expression's buffers before the argument struct is written
         Code scratch_code;
@@ -1244,7 +1247,7 @@ bool lower_flash_f32(const sanic_program_desc* d, int si, int64_t& scratch, Lowe
     const int NWV = 8;
     auto S = [](int64_t v) { return std::to_string(v); };
 
-    Renderer R(d), Rs(d), Ro(d), Rw(d);
+    Renderer R(d), Rs(d), Ro(d), Rw(d);     // the kernel, and its score, store and window functions
     auto win = honest_window(d, st);
     const sanic_node& sl = d->nodes[st.leaf[P.sleaf]];
     std::vector<std::string> lc(sl.rank);
@@ -1256,8 +1259,10 @@ bool lower_flash_f32(const sanic_program_desc* d, int si, int64_t& scratch, Lowe
     sp.indent = wc.indent = fo.indent = k.indent = 1;
     Rs.subst[P.dot_reduce] = "dotv";
     const std::string vpart = Rs.value(sp, st.leaf[P.sleaf], lc);
+    Rw.take_buffers(Rs);
     for (int j = 0; j < st.rank; j++) wc.line("const idx_t g" + S(j) + " = " + (j == P.hdim ? "hh" : j == P.qdim ? "qrow" : "0") + ";");
     emit_window(Rw, wc, st, win, "wlo", "whi");
+    Ro.take_buffers(Rw);
     std::vector<std::string> gc(st.rank, "0");
     if (P.hdim >= 0) gc[P.hdim] = "hh";
     gc[P.qdim] = "qi";
@@ -1275,8 +1280,7 @@ bool lower_flash_f32(const sanic_program_desc* d, int si, int64_t& scratch, Lowe
             lin = j == 0 ? "(idx_t)(" + gc[0] + ")" : "(" + lin + " * " + S(st.grid[j]) + " + (idx_t)(" + gc[j] + "))";
         fo.line(store_stmt(Ro.param(st.out_buffer), lin, st.out_dtype, v, false, d->buffers[st.out_buffer].scale));
     }
-    for (Renderer* r : {&Rs, &Rw, &Ro})
-        for (int b : r->bufs) R.param(b);
+    R.take_buffers(Ro);
     auto base = [&](const Access& acc, const std::vector<int64_t>& cf, int div, int64_t hcf) {
         const std::string h = div ? "(hh / " + S(div) + ") * " + S(hcf) : "hh * " + S(cf[0]);
         return R.param(acc.buffer) + " + " + S(acc.addr.c0) + " + " + h;

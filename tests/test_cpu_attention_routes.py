@@ -1,0 +1,44 @@
+"""Which kernel the attention stages lower to, and what the emitted source says (no GPU)."""
+import re
+
+import pytest
+
+from sanic_amd import ir
+from tests import attn_forms as A
+
+
+def _functions(src):
+    """name -> body of the kernel's functions"""
+    out = {}
+    for m in re.finditer(r"(?:void|bool|float)[^(;{}]* (\w+)\([^{};]*Args&? a[^{;]*\{", src):
+        out[m.group(1)] = src[m.end():src.find("\n}", m.end())]
+    return out
+
+
+@pytest.mark.parametrize("terms", [A.prefix, A.chunk, A.bias, lambda p, s: A.bias(p, s) + A.prefix(p, s)])
+@pytest.mark.parametrize("NH,NKV,NQ,T,dt", [
+    (4, 2, 128, 128, ir.BF16),      # whole tiles
+    (4, 2, 100, 300, ir.BF16),      # any length
+    (0, 0, 40, 4096, ir.BF16),      # no head dim
+    (0, 0, 200, 200, ir.F32),
+    (4, 2, 200, 200, ir.F32),
+])
+def test_every_function_of_an_attention_kernel_names_the_same_buffers(NH, NKV, NQ, T, dt, terms):
+    """A mask or an epilogue that reads a buffer: the score, window and store functions and the
+    kernel pass one argument struct, so the store goes to the output (the one float16 buffer)
+    and to nothing else."""
+    p = A.attention(NH, NKV, NQ, T, terms, dt=dt, out=ir.F16, epilogue=A.residual)
+    kind, src = p.emit(0)
+    assert kind.startswith("skeleton:flash_prefill" if dt == ir.BF16 else "skeleton:attn_f32"), kind
+    types = re.findall(r"(\S+)\* __restrict__ (b\d+);", src)
+    out = [b for t, b in types if t == "_Float16"]
+    assert len(out) == 1 and len(types) == len(p.buffers)
+    fns = _functions(src)
+    assert "finish" in fns and "window" in fns
+    for name, body in fns.items():
+        stores = set(re.findall(r"a\.(b\d+)\[[^;=]*\] = ", body))
+        assert stores == (set(out) if name == "finish" else set()), (name, stores)
+    # the mask's and the bias's float buffers are read by the score function as float
+    floats = {b for t, b in types if t == "float"}
+    score = fns["score_part"] if "score_part" in fns else fns["score"]
+    assert set(re.findall(r"a\.(b\d+)", score)) <= floats

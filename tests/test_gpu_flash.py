@@ -5,6 +5,7 @@ import pytest
 import oracle
 from sanic_amd import configs, ir
 from sanic_amd.program import SCRATCH, Program
+from tests import attn_forms as A
 from tests.util import floored_rel_err, max_rel_err, run_on_gpu
 
 pytestmark = pytest.mark.gpu
@@ -262,3 +263,41 @@ def test_rotation_table_and_keys_in_one_launch(dev, monkeypatch, S, H, F):
     np.testing.assert_array_equal(got["T"], want["T"])
     a, b = np.asarray(got["Y"], np.float64), np.asarray(want["Y"], np.float64)
     assert np.all(np.abs(a - b) <= 2.0 ** -7 * np.abs(b) + 2.0 ** -22 * np.abs(vals["K"]).max())
+
+
+def _form_values(prog, seed):
+    """Seeded inputs for every input buffer; `position` two thirds along the keys that K holds."""
+    T = prog.by_name["K"].shape[-2]
+    out = {}
+    for i, b in enumerate(b for b in prog.buffers if b.role == 0):
+        n = int(np.prod(b.shape)) if b.shape else 1
+        out[b.name] = np.array(float(2 * T // 3)) if b.name == "position" else np.asarray(
+            oracle.synth(seed + i, n, dtype=b.dtype), np.float64).reshape(b.shape)
+    return out
+
+
+@pytest.mark.parametrize("terms", [A.prefix, A.chunk, A.bias, lambda p, s: A.bias(p, s) + A.prefix(p, s)])
+@pytest.mark.parametrize("NH,NKV,NQ,T,dt", [
+    (4, 2, 128, 128, ir.BF16),      # whole tiles
+    (4, 2, 100, 300, ir.BF16),      # any length
+    (0, 0, 40, 1000, ir.BF16),      # no head dim
+    (0, 0, 200, 200, ir.F32),
+    (4, 2, 200, 200, ir.F32),
+])
+def test_masks_and_epilogues_that_read_buffers(dev, NH, NKV, NQ, T, dt, terms):
+    """Masks and biases from buffers in the scores, a stored residual in the epilogue, against the
+    f64 interpreter; the inputs come back as they were given."""
+    prog = A.attention(NH, NKV, NQ, T, terms, dt=dt, out=ir.F32, epilogue=A.residual)
+    vals = _form_values(prog, 540)
+    exe = dev.prepare(prog)
+    kind = exe.stage_kernel(0)
+    print(kind, flush=True)
+    assert kind.startswith("skeleton:flash_prefill" if dt == ir.BF16 else "skeleton:attn_f32"), kind
+    bufs = {n: dev.from_values(v, prog.by_name[n].dtype) for n, v in vals.items()}
+    held = {n: b.download() for n, b in bufs.items()}
+    got = exe.execute(bufs)["O"].read(ir.F32, int(np.prod(prog.by_name["O"].shape))).reshape(prog.by_name["O"].shape)
+    assert all(b.download() == held[n] for n, b in bufs.items())
+    err = max_rel_err(got, oracle.run_program(prog, vals)["O"])
+    print(err)
+    # whole tiles round the softmax weights to bf16 (2^-9 of Σ p|v| ≲ 3); the others hold 16 bits or more
+    assert err < (1e-2 if "any length" not in kind and dt == ir.BF16 else 1e-4)
