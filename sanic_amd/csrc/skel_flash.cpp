@@ -151,70 +151,173 @@ bool find_flash_dot(const sanic_program_desc* d, int node, const std::vector<Sym
     return true;
 }
 
-// A window edge read off the first and last row of a block must not decrease with the query row
-// in between: values that do not move with the row, coordinates, sums of such edges, differences
-// from a row-free value and products with a constant that is not negative.
-std::vector<int> kid_bind(const sanic_program_desc* d, int node, int k, const std::vector<int>& b) {
-    const sanic_node& n = d->nodes[node];
-    const sanic_node& m = d->nodes[n.in[k]];
-    std::vector<int> cb(m.rank);
-    for (int j = 0; j < m.rank; j++) cb[j] = m.shape[j] == 1 ? SANIC_BIND_BCAST : b[n.rank - m.rank + j];
-    return cb;
-}
+// How a window edge moves with the query row: `dir` 0 not at all, 1 rising, −1 falling, 2 one of
+// the two (by a factor known at run time). `convex` and `concave`: made of lines of whole slopes by
+// maxima, or by minima. A straight edge is both.
+struct EdgeForm {
+    int dir = 0;
+    bool convex = true, concave = true;
+};
 
-bool row_free(const sanic_program_desc* d, int node, const std::vector<int>& b, int qdim) {
-    const sanic_node& n = d->nodes[node];
-    if (n.kind == SANIC_NODE_COORDINATE) return b[n.dim] != qdim;
-    if (n.kind == SANIC_NODE_MAP) {
-        for (int k = 0; k < n.n_in; k++) if (!row_free(d, n.in[k], kid_bind(d, node, k, b), qdim)) return false;
-        return true;
-    }
-    for (int j = 0; j < n.rank; j++) if (n.shape[j] != 1 && b[j] == qdim) return false;
+bool join_edges(const EdgeForm& x, const EdgeForm& y, EdgeForm& out) {
+    if (x.dir && y.dir && (x.dir != y.dir || x.dir == 2)) return false;
+    out = {x.dir ? x.dir : y.dir, x.convex && y.convex, x.concave && y.concave};
     return true;
 }
 
-bool rising_edge(const sanic_program_desc* d, int node, const std::vector<int>& b, int qdim) {
+EdgeForm turned(const EdgeForm& e) { return {e.dir == 2 ? 2 : -e.dir, e.concave, e.convex}; }
+
+std::vector<Sym> kid_coords(const sanic_program_desc* d, int node, int k, const std::vector<Sym>& c) {
     const sanic_node& n = d->nodes[node];
-    if (row_free(d, node, b, qdim) || n.kind == SANIC_NODE_IOTA || n.kind == SANIC_NODE_COORDINATE) return true;
+    const sanic_node& m = d->nodes[n.in[k]];
+    std::vector<Sym> cc(m.rank);
+    for (int j = 0; j < m.rank; j++) cc[j] = m.shape[j] == 1 ? Sym() : c[n.rank - m.rank + j];
+    return cc;
+}
+
+bool sym_form(const Sym& s, int row, EdgeForm& out) {
+    out = EdgeForm();
+    for (auto& t : s.terms) {
+        if (t.var != row || !t.coef) continue;
+        if (t.mod || !join_edges(out, {t.coef > 0 ? 1 : -1, t.div == 1, t.div == 1}, out)) return false;
+    }
+    return true;
+}
+
+// The form of an edge at coordinates `c` over the grid's variables, of which `row` is the query row;
+// false for an edge that is not known to move one way.
+bool edge_form(const sanic_program_desc* d, int node, const std::vector<Sym>& c, const std::vector<int64_t>& ext, int row, EdgeForm& out) {
+    const sanic_node& n = d->nodes[node];
+    bool moves = false;
+    for (auto& s : c)
+        for (auto& t : s.terms) moves |= t.var == row;
+    out = EdgeForm();
+    if (!moves || n.kind == SANIC_NODE_CONST) return true;
+    if (n.kind == SANIC_NODE_IOTA) return sym_form(c[0], row, out);
+    if (n.kind == SANIC_NODE_COORDINATE) return sym_form(c[n.dim], row, out);
+    if (n.kind == SANIC_NODE_VIEW || n.kind == SANIC_NODE_REINDEX) {
+        std::vector<Sym> sc;
+        return sym_child_coords(d, node, c, ext, sc) && edge_form(d, n.in[0], sc, ext, row, out);
+    }
     if (n.kind != SANIC_NODE_MAP) return false;
-    auto up = [&](int k) { return rising_edge(d, n.in[k], kid_bind(d, node, k, b), qdim); };
-    if (n.op == SANIC_OP_ADD) return up(0) && up(1);
-    if (n.op == SANIC_OP_SUB) return up(0) && row_free(d, n.in[1], kid_bind(d, node, 1, b), qdim);
-    if (n.op == SANIC_OP_MUL)
-        for (int k = 0; k < 2; k++)
-            if (d->nodes[n.in[k]].kind == SANIC_NODE_CONST && d->nodes[n.in[k]].value >= 0.0) return up(1 - k);
-    return false;
+    EdgeForm e[2];
+    for (int k = 0; k < n.n_in; k++)
+        if (k > 1 || !edge_form(d, n.in[k], kid_coords(d, node, k, c), ext, row, e[k])) return false;
+    switch (n.op) {
+    case SANIC_OP_ADD: return join_edges(e[0], e[1], out);
+    case SANIC_OP_SUB: return join_edges(e[0], turned(e[1]), out);
+    case SANIC_OP_NEG: out = turned(e[0]); return true;
+    case SANIC_OP_ROUND_F32: out = e[0]; return true;
+    case SANIC_OP_MAX:
+    case SANIC_OP_MIN:
+        if (!join_edges(e[0], e[1], out)) return false;
+        (n.op == SANIC_OP_MAX ? out.concave : out.convex) &= !out.dir;
+        return true;
+    case SANIC_OP_MUL:
+    case SANIC_OP_DIV: {
+        // one side moves, the other scales it
+        const int k = e[0].dir ? 0 : 1;
+        if (e[1 - k].dir || (n.op == SANIC_OP_DIV && k)) return false;
+        out = e[k];
+        if (!out.dir) return true;
+        const sanic_node& f = d->nodes[n.in[1 - k]];
+        if (f.kind != SANIC_NODE_CONST) {
+            out = {2, false, false};
+            return true;
+        }
+        if (!std::isfinite(f.value) || (n.op == SANIC_OP_DIV && f.value == 0.0)) return false;
+        if (f.value == 0.0) out = EdgeForm();
+        if (f.value < 0.0) out = turned(out);
+        const bool whole = n.op == SANIC_OP_MUL && f.value == std::floor(f.value);
+        if (out.dir && !whole) out.convex = out.concave = false;
+        return true;
+    }
+    default: return false;
+    }
+}
+
+// The coordinates of a window edge over the grid's variables.
+std::vector<Sym> edge_coords(const WindowBound& w) {
+    std::vector<Sym> c(w.bind.size());
+    for (size_t j = 0; j < c.size(); j++)
+        if (w.bind[j] >= 0) c[j] = Sym::var(w.bind[j]);
+    return c;
+}
+
+// A block's and a wave's key range is the union of its first and last row's windows, and its fully
+// visible tiles their intersection. That holds for the rows between if each side's edges all move one
+// way, and if no window between is empty (which stands for the whole stream) where those two are
+// not: sure where one side stands still or the two move apart, and where they move together if the
+// lower edges are convex and the upper ones concave.
+bool window_between_rows(const sanic_program_desc* d, const sanic_stage& st, int qdim) {
+    const std::vector<int64_t> ext(st.grid, st.grid + st.rank);
+    EdgeForm side[2];
+    for (auto& w : honest_window(d, st)) {
+        EdgeForm e;
+        const bool low = w.kind == WindowBound::LO_CEIL;
+        if (!edge_form(d, w.node, edge_coords(w), ext, qdim, e) || !join_edges(side[low], e, side[low])) return false;
+    }
+    const EdgeForm &hi = side[0], &lo = side[1];
+    if (!hi.dir || !lo.dir) return true;
+    return hi.dir != 2 && lo.dir != 2 && (hi.dir != lo.dir || (lo.convex && hi.concave));
 }
 
 // The value of a window edge at a query row, where it is made of constants and the row alone.
-double edge_at(const sanic_program_desc* d, int node, const std::vector<int>& b, int qdim, double row, bool& known) {
+double edge_at(const sanic_program_desc* d, int node, const std::vector<Sym>& c, const std::vector<int64_t>& ext, int qdim, double row, bool& known) {
     const sanic_node& n = d->nodes[node];
+    auto at = [&](const Sym& s) {
+        double v = (double)s.c0;
+        for (auto& t : s.terms) {
+            if (t.var != qdim) known = false;
+            int64_t x = (int64_t)row / t.div;
+            v += (double)(t.coef * (t.mod ? x % t.mod : x));
+        }
+        return v;
+    };
     if (n.kind == SANIC_NODE_CONST) return n.value;
-    if (n.kind == SANIC_NODE_COORDINATE && b[n.dim] == qdim) return row;
-    if (n.kind == SANIC_NODE_IOTA && b[0] == qdim) return row;
-    if (n.kind == SANIC_NODE_MAP && n.n_in == 2 && (n.op == SANIC_OP_ADD || n.op == SANIC_OP_SUB || n.op == SANIC_OP_MUL)) {
-        const double x = edge_at(d, n.in[0], kid_bind(d, node, 0, b), qdim, row, known);
-        const double y = edge_at(d, n.in[1], kid_bind(d, node, 1, b), qdim, row, known);
-        return n.op == SANIC_OP_ADD ? x + y : n.op == SANIC_OP_SUB ? x - y : x * y;
+    if (n.kind == SANIC_NODE_COORDINATE) return at(c[n.dim]);
+    if (n.kind == SANIC_NODE_IOTA) return at(c[0]);
+    std::vector<Sym> sc;
+    if ((n.kind == SANIC_NODE_VIEW || n.kind == SANIC_NODE_REINDEX) && sym_child_coords(d, node, c, ext, sc))
+        return edge_at(d, n.in[0], sc, ext, qdim, row, known);
+    if (n.kind == SANIC_NODE_MAP && n.n_in <= 2) {
+        double v[2] = {0.0, 0.0};
+        for (int k = 0; k < n.n_in; k++) v[k] = edge_at(d, n.in[k], kid_coords(d, node, k, c), ext, qdim, row, known);
+        switch (n.op) {
+        case SANIC_OP_ADD: return v[0] + v[1];
+        case SANIC_OP_SUB: return v[0] - v[1];
+        case SANIC_OP_MUL: return v[0] * v[1];
+        case SANIC_OP_DIV: return v[0] / v[1];
+        case SANIC_OP_MAX: return std::max(v[0], v[1]);
+        case SANIC_OP_MIN: return std::min(v[0], v[1]);
+        case SANIC_OP_NEG: return -v[0];
+        default: break;
+        }
     }
     known = false;
     return 0.0;
 }
 
-// Keys that the last `rows` query rows see between them (all, where an edge is not known here).
+// The most keys that a block of `rows` query rows sees between them, over the first, the middle and
+// the last block (all, where an edge is not known here).
 int64_t longest_window(const sanic_program_desc* d, const sanic_stage& st, int qdim, int64_t nq, int64_t rows) {
-    double lo = 0.0, hi = (double)st.stream;
-    for (auto& w : honest_window(d, st)) {
-        bool known = true;
-        if (w.kind == WindowBound::LO_CEIL) {
-            const double v = edge_at(d, w.node, w.bind, qdim, (double)std::max<int64_t>(0, nq - rows), known);
-            if (known) lo = std::max(lo, v);
-        } else {
-            const double v = edge_at(d, w.node, w.bind, qdim, (double)(nq - 1), known);
-            if (known) hi = std::min(hi, v + 1.0);
+    const std::vector<int64_t> ext(st.grid, st.grid + st.rank);
+    const auto win = honest_window(d, st);
+    int64_t most = 0;
+    for (int64_t r0 : {(int64_t)0, nq / 2, std::max<int64_t>(0, nq - rows)}) {
+        const int64_t r1 = std::min(nq, r0 + rows) - 1;
+        double lo = 0.0, hi = (double)st.stream;
+        for (auto& w : win) {
+            bool known = true;
+            const auto c = edge_coords(w);
+            const double a = edge_at(d, w.node, c, ext, qdim, (double)r0, known), b = edge_at(d, w.node, c, ext, qdim, (double)r1, known);
+            if (!known) continue;
+            if (w.kind == WindowBound::LO_CEIL) lo = std::max(lo, std::min(a, b));
+            else hi = std::min(hi, std::max(a, b) + 1.0);
         }
+        most = std::max(most, hi > lo ? (int64_t)(hi - lo) : st.stream);
     }
-    return hi > lo ? (int64_t)(hi - lo) : st.stream;
+    return most;
 }
 
 // The attention structure of a stage: carrier, dims and the affine K and V (any storage dtype).
@@ -287,11 +390,7 @@ bool attention_plan(const sanic_program_desc* d, int si, FlashPlan& P) {
         vcs[j] = b == SANIC_BIND_STREAM ? Sym::var(1) : b == P.hdim ? Sym::var(0) : b == P.edim ? Sym::var(2) : Sym();
     }
     if (!sym_access(d, st.leaf[P.vleaf], vcs, {P.NH, P.T, P.E}, P.vacc)) return false;
-    // a block's and a wave's key ranges are read off their first and last rows: every edge must
-    // not decrease with the row
-    for (auto& w : honest_window(d, st))
-        if (!rising_edge(d, w.node, w.bind, P.qdim)) return false;
-    return true;
+    return window_between_rows(d, st, P.qdim);
 }
 
 bool flash_plan(const sanic_program_desc* d, int si, FlashPlan& P) {

@@ -67,3 +67,36 @@ def bias(p, s):
 
 def residual(p, fold):
     return ir.map_(ir.ADD, p.input("R", fold.shape, ir.BF16), fold)
+
+
+def _half(s):
+    return float(s.shape[-1] // 2)
+
+
+# Window edges that move one way with the query row: mask terms by name.
+EDGES = {
+    "falling": lambda p, s: [mask(ir.map_(ir.SUB, ir.const(_half(s)), row(s)), key(s), -1e30, 0.0)],
+    "falling product": lambda p, s: [mask(ir.map_(ir.ADD, ir.map_(ir.MUL, row(s), ir.const(-1.0)), ir.const(_half(s))), key(s), -1e30, 0.0)],
+    "half": lambda p, s: [mask(ir.map_(ir.DIV, row(s), ir.const(2.0)), key(s), -1e30, 0.0)],
+    "at most": lambda p, s: [mask(ir.map_(ir.MIN, row(s), ir.const(37.0)), key(s), -1e30, 0.0)],
+    "at least": lambda p, s: [mask(ir.map_(ir.MAX, row(s), ir.const(37.0)), key(s), -1e30, 0.0)],
+    "iota": lambda p, s: [mask(ir.unsqueeze(ir.iota(s.shape[-2]), 1), ir.iota(s.shape[-1]), -1e30, 0.0)],
+    "window": lambda p, s: causal(p, s) + [mask(key(s), ir.map_(ir.MAX, ir.map_(ir.SUB, row(s), ir.const(40.0)), ir.const(0.0)), -1e30, 0.0)],
+    "closing": lambda p, s: [mask(ir.map_(ir.SUB, ir.const(_half(s)), row(s)), key(s), -1e30, 0.0), mask(key(s), row(s), -1e30, 0.0)],
+    "by a factor": lambda p, s: [mask(ir.map_(ir.MUL, row(s), p.input("position", (), ir.F32)), key(s), -1e30, 0.0)],
+}
+
+
+def _per_row(p, s):
+    return ir.unsqueeze(p.input("bias", (s.shape[-2],), ir.F32), 1)
+
+
+# Edges whose value at a row between two others these do not bound.
+UNORDERED = {
+    "stored per row": lambda p, s: [mask(_per_row(p, s), key(s), -1e30, 0.0)],
+    "up and down": lambda p, s: [mask(ir.map_(ir.MIN, row(s), ir.map_(ir.SUB, ir.const(64.0), row(s))), key(s), -1e30, 0.0)],
+    "two ways": lambda p, s: causal(p, s) + EDGES["falling"](p, s),
+    # keys equal to a third of the row: no row between two multiples of 3 sees one
+    "thirds": lambda p, s: [mask(ir.map_(ir.DIV, row(s), ir.const(3.0)), key(s), -1e30, 0.0),
+                            mask(key(s), ir.map_(ir.DIV, row(s), ir.const(3.0)), -1e30, 0.0)],
+}

@@ -42,3 +42,16 @@ def test_every_function_of_an_attention_kernel_names_the_same_buffers(NH, NKV, N
     floats = {b for t, b in types if t == "float"}
     score = fns["score_part"] if "score_part" in fns else fns["score"]
     assert set(re.findall(r"a\.(b\d+)", score)) <= floats
+
+
+@pytest.mark.parametrize("name", A.EDGES)
+@pytest.mark.parametrize("NH,NKV,NQ,T,dt", [(8, 2, 512, 512, ir.BF16), (4, 2, 100, 300, ir.BF16), (0, 0, 200, 200, ir.F32)])
+def test_windows_that_move_one_way_take_the_attention_kernels(NH, NKV, NQ, T, dt, name):
+    kind = A.attention(NH, NKV, NQ, T, A.EDGES[name], dt=dt).emit(0)[0]
+    assert kind.startswith("skeleton:flash_prefill" if dt == ir.BF16 else "skeleton:attn_f32"), kind
+
+
+@pytest.mark.parametrize("name", A.UNORDERED)
+@pytest.mark.parametrize("NH,NKV,NQ,T,dt", [(8, 2, 512, 512, ir.BF16), (4, 2, 100, 300, ir.BF16), (0, 0, 200, 200, ir.F32)])
+def test_windows_not_bounded_by_their_end_rows_take_the_fold(NH, NKV, NQ, T, dt, name):
+    assert A.attention(NH, NKV, NQ, T, A.UNORDERED[name], dt=dt).emit(0)[0].startswith("fold:")

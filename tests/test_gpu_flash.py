@@ -301,3 +301,24 @@ def test_masks_and_epilogues_that_read_buffers(dev, NH, NKV, NQ, T, dt, terms):
     print(err)
     # whole tiles round the softmax weights to bf16 (2^-9 of Σ p|v| ≲ 3); the others hold 16 bits or more
     assert err < (1e-2 if "any length" not in kind and dt == ir.BF16 else 1e-4)
+
+
+@pytest.mark.parametrize("name", A.EDGES)
+@pytest.mark.parametrize("NH,NKV,NQ,T,dt", [(4, 2, 128, 192, ir.BF16), (4, 2, 100, 300, ir.BF16), (0, 0, 200, 200, ir.F32)])
+def test_windows_that_move_one_way(dev, NH, NKV, NQ, T, dt, name):
+    """Falling, halved, clamped and iota-written window edges, rows without a visible key among
+    them, against the f64 interpreter."""
+    prog = A.attention(NH, NKV, NQ, T, A.EDGES[name], dt=dt, out=ir.F32)
+    vals = _form_values(prog, 560)
+    if "position" in vals:
+        vals["position"] = np.array(-1.0 if dt == ir.F32 else 0.75)
+    exe = dev.prepare(prog)
+    kind = exe.stage_kernel(0)
+    print(kind, flush=True)
+    assert kind.startswith("skeleton:flash_prefill" if dt == ir.BF16 else "skeleton:attn_f32"), kind
+    bufs = {n: dev.from_values(v, prog.by_name[n].dtype) for n, v in vals.items()}
+    got = exe.execute(bufs)["O"].read(ir.F32, int(np.prod(prog.by_name["O"].shape))).reshape(prog.by_name["O"].shape)
+    err = max_rel_err(got, oracle.run_program(prog, vals)["O"])
+    print(err)
+    # as test_masks_and_epilogues_that_read_buffers
+    assert err < (1e-2 if "any length" not in kind and dt == ir.BF16 else 1e-4)
