@@ -459,13 +459,15 @@ bool lower_flash_prefill(const sanic_program_desc* d, int si, int64_t& scratch, 
     const sanic_carrier& c = st.carrier;
     const int64_t NH = P.NH, NQ = P.NQ, T = P.T, E = P.E, HD = P.HD;
     // Lengths off the tiles (a prompt nobody padded) and a single head were folded in f32 by the generic fold: here
-    // the softmax weights, and a query side that is an expression, go to the MFMA as hi + lo bf16
-    // pairs (16 significant bits), so they keep that precision at two MFMAs per fragment; one
-    // query tile per wave holds the second operands in the registers the second tile had (115
-    // VGPRs) and gives short prompts twice the workgroups. 32/8 heads, S = 1000, window 256, with
-    // the RoPE stages: 20.0 ms in the generic fold (it forms q·k again for each of the 64 value
-    // columns) → 20.1 µs, the same 2.2e-3 from a 64-bit evaluation.
-    const bool hilo = P.ragged;
+    // the softmax weights, and a query side that is an expression, go to the MFMA as sums of bf16 terms:
+    // two (16 significant bits) where the output is bf16, whose rounding is 128 times theirs, else three
+    // (24 bits, the fold's own). RMS error against 64 bits, fold and here, 2 heads, S = 1000: f32 output
+    // 2.5e-8 and 2.3e-8, float16 2.43e-5 and bf16 1.94e-4 in both. One query tile per wave holds the other
+    // terms in the registers the second tile had (two: 117 VGPRs) and gives short prompts twice the
+    // workgroups. 32/8 heads, S = 1000, window 256, with the RoPE stages: 20.0 ms in the generic fold (it
+    // forms q·k again for each of the 64 value columns) → 20.1 µs. Three terms, 32/8 heads, S = 1000,
+    // causal: 18.1 → 20.9 µs; 8/2 heads, S = 4000: 53 → 60.
+    const int NP = !P.ragged ? 1 : st.out_dtype == SANIC_BF16 ? 2 : 3;   // bf16 terms of a softmax weight
     const int fvar = P.ragged ? 0 : d->stages[si].sched.variant;
     // Launches that leave CUs short of waves: 64-row blocks (up to 512 of 128 rows; 32 heads, S = 2048
     // 58 → 47 µs, S = 4096, 1024 blocks, 108 against 123), and KS teams of 4 waves per block, each with
@@ -608,6 +610,11 @@ bool lower_flash_prefill(const sanic_program_desc* d, int si, int64_t& scratch, 
            "  const unsigned h = pk_bf16(x, y);\n"
            "  hi = h;\n"
            "  lo = pk_bf16(x - __uint_as_float(h << 16), y - __uint_as_float(h & 0xFFFF0000u));\n}\n";
+    if (NP == 3)
+        src << "__device__ __forceinline__ void split3_bf16(float x, float y, unsigned& hi, unsigned& mid, unsigned& lo) {\n"
+               "  const unsigned h = pk_bf16(x, y);\n"
+               "  hi = h;\n"
+               "  split_bf16(x - __uint_as_float(h << 16), y - __uint_as_float(h & 0xFFFF0000u), mid, lo);\n}\n";
     // max across the 4 lane groups of a query column (lanes l, l^16, l^32, l^48): gfx950
     // permlane swaps, no LDS round trip
     // compiler-visible maxima: the compiler forms v_max3_f32 itself and, unlike for inline asm
@@ -723,11 +730,17 @@ bool lower_flash_prefill(const sanic_program_desc* d, int si, int64_t& scratch, 
     // (variant 3 takes the rendered leaf on every edge tile: the reference form the fast path
     // is tested against bit for bit)
     const bool edge_on = raw_ok && fvar != 3;
+    // two values as the packed bf16 terms w[0] (+ w[1] (+ w[2])), component i
+    auto split = [&](const std::string& x, const std::string& y, const std::string& w, const std::string& i) {
+        if (NP == 1) return "  " + w + "[0][" + i + "] = pk_bf16(" + x + ", " + y + ");";
+        if (NP == 2) return "  { unsigned h1, l1; split_bf16(" + x + ", " + y + ", h1, l1); " + w + "[0][" + i + "] = h1; " + w + "[1][" + i + "] = l1; }";
+        return "  { unsigned h1, m1, l1; split3_bf16(" + x + ", " + y + ", h1, m1, l1); " + w + "[0][" + i + "] = h1; " + w + "[1][" + i + "] = m1; " + w + "[2][" + i + "] = l1; }";
+    };
     // Q^T as the B operand (lane = query column l16 (+16·qt), d-slots lq·8 + 0..7 (+32·ds)),
     // held in registers for the whole key loop, loaded once from global memory
     k.line("bf16x8 qf[" + QTs + "][2];");
-    const bool qlo = hilo && P.qexpr;
-    if (qlo) k.line("bf16x8 ql[" + QTs + "][2];");
+    const int NQT = P.qexpr ? NP : 1;                // bf16 terms of a query value
+    for (int h = 1; h < NQT; h++) k.line("bf16x8 q" + std::to_string(h) + "[" + QTs + "][2];");
     for (int qt = 0; qt < QT; qt++)
         k.line("const idx_t qr" + std::to_string(qt) + " = " + row_clamp("q0 + " + std::to_string(qt * 16) + " + l16") + ";");
     if (!P.qexpr) {
@@ -767,12 +780,10 @@ bool lower_flash_prefill(const sanic_program_desc* d, int si, int64_t& scratch, 
     auto emit_qexpr = [&]() {
         auto q_split = [&](int qt, int ds, const std::string* v) {
             k.line("{");
-            k.line("  sanic_u32x4 h_, l_;");
-            for (int q = 0; q < 4; q++)
-                k.line("  { unsigned h1, l1; split_bf16(" + v[2 * q] + ", " + v[2 * q + 1] + ", h1, l1); h_[" + std::to_string(q) + "] = h1; l_[" + std::to_string(q) + "] = l1; }");
+            k.line("  sanic_u32x4 w_[" + std::to_string(NP) + "];");
+            for (int q = 0; q < 4; q++) k.line(split(v[2 * q], v[2 * q + 1], "w_", std::to_string(q)));
             const std::string ix = "[" + std::to_string(qt) + "][" + std::to_string(ds) + "]";
-            k.line("  qf" + ix + " = __builtin_bit_cast(bf16x8, h_);");
-            k.line("  ql" + ix + " = __builtin_bit_cast(bf16x8, l_);");
+            for (int h = 0; h < NP; h++) k.line("  q" + (h ? std::to_string(h) : "f") + ix + " = __builtin_bit_cast(bf16x8, w_[" + std::to_string(h) + "]);");
             k.line("}");
         };
         if (q_runs) {
@@ -780,7 +791,7 @@ bool lower_flash_prefill(const sanic_program_desc* d, int si, int64_t& scratch, 
             for (int qt = 0; qt < QT; qt++)
                 for (int ds = 0; ds < 2; ds++) {
                     const auto& v = q_vals[qt][ds];
-                    if (qlo) { q_split(qt, ds, v.data()); continue; }
+                    if (NQT > 1) { q_split(qt, ds, v.data()); continue; }
                     k.line("qf[" + std::to_string(qt) + "][" + std::to_string(ds) + "] = __builtin_bit_cast(bf16x8, (sanic_u32x4){pk_bf16(" + v[0] + ", " + v[1] +
                            "), pk_bf16(" + v[2] + ", " + v[3] + "), pk_bf16(" + v[4] + ", " + v[5] + "), pk_bf16(" + v[6] + ", " + v[7] + ")});");
                 }
@@ -801,7 +812,7 @@ bool lower_flash_prefill(const sanic_program_desc* d, int si, int64_t& scratch, 
                 }
             R.memo.pop_back();
             for (int ds = 0; ds < 2; ds++) {
-                if (qlo) { q_split(qt, ds, vals[ds]); continue; }
+                if (NQT > 1) { q_split(qt, ds, vals[ds]); continue; }
                 std::string pk = "(sanic_u32x4){";
                 for (int q = 0; q < 4; q++)
                     pk += std::string(q ? ", " : "") + "pk_bf16(" + vals[ds][2 * q] + ", " + vals[ds][2 * q + 1] + ")";
@@ -917,8 +928,7 @@ bool lower_flash_prefill(const sanic_program_desc* d, int si, int64_t& scratch, 
     // MFMAs in the same order either way.
     const bool s_both = QT == 2 && SPL == 1 && fvar != 3;
     k.line("f32x4 s[4][" + QTs + "];");
-    k.line("sanic_u32x4 pw[" + QTs + "][2];");
-    if (hilo) k.line("sanic_u32x4 pl[" + QTs + "][2];");
+    k.line("sanic_u32x4 pw[" + QTs + "][2][" + std::to_string(NP) + "];");
     auto scores = [&](bool both) {
         k.line("#pragma unroll");
         k.line("for (int kt = 0; kt < 4; ++kt) {");
@@ -934,7 +944,7 @@ bool lower_flash_prefill(const sanic_program_desc* d, int si, int64_t& scratch, 
             k.line("    {");
         }
         k.line("      s[kt][qt] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(ka, qf[qt][ds], s[kt][qt], 0, 0, 0);");
-        if (qlo) k.line("      s[kt][qt] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(ka, ql[qt][ds], s[kt][qt], 0, 0, 0);");
+        for (int h = 1; h < NQT; h++) k.line("      s[kt][qt] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(ka, q" + std::to_string(h) + "[qt][ds], s[kt][qt], 0, 0, 0);");
         k.line("    }");
         k.line("  }");
         k.line("}");
@@ -1067,30 +1077,20 @@ bool lower_flash_prefill(const sanic_program_desc* d, int si, int64_t& scratch, 
     // slots 4..7 = keys 32ks + 16 + lq·4 + r (tile 2ks+1); two slots per dword, RNE in hardware
     k.line("#pragma unroll");
     k.line("for (int ks = 0; ks < 2; ++ks) {");
-    const char* comp[4] = {"x", "y", "z", "w"};
-    for (int q = 0; q < 4; q++) {
-        const std::string pp = "p[8 * ks + " + std::to_string(2 * q) + "], p[8 * ks + " + std::to_string(2 * q + 1) + "]";
-        if (hilo) k.line("  { unsigned h1, l1; split_bf16(" + pp + ", h1, l1); pw[qt][ks]." + comp[q] + " = h1; pl[qt][ks]." + comp[q] + " = l1; }");
-        else k.line("  pw[qt][ks]." + std::string(comp[q]) + " = pk_bf16(" + pp + ");");
-    }
+    for (int q = 0; q < 4; q++) k.line(split("p[8 * ks + " + std::to_string(2 * q) + "]", "p[8 * ks + " + std::to_string(2 * q + 1) + "]", "pw[qt][ks]", std::to_string(q)));
     k.line("}");
     k.indent--;
     k.line("}");
-    k.line("bf16x8 pf[" + QTs + "][2];");
-    k.line("#pragma unroll");
-    k.line("for (int qt = 0; qt < " + QTs + "; ++qt) { pf[qt][0] = __builtin_bit_cast(bf16x8, pw[qt][0]); pf[qt][1] = __builtin_bit_cast(bf16x8, pw[qt][1]); }");
-    if (hilo) {
-        k.line("bf16x8 pfl[" + QTs + "][2];");
-        k.line("#pragma unroll");
-        k.line("for (int qt = 0; qt < " + QTs + "; ++qt) { pfl[qt][0] = __builtin_bit_cast(bf16x8, pl[qt][0]); pfl[qt][1] = __builtin_bit_cast(bf16x8, pl[qt][1]); }");
-    }
+    auto weight = [&](const std::string& qt, const std::string& ks, int h) {
+        return "__builtin_bit_cast(bf16x8, pw[" + qt + "][" + ks + "][" + std::to_string(h) + "])";
+    };
     // O^T += V^T · P^T ; V^T A operand: row e = dt·16 + l16, keys in the same slot order
     k.line("#pragma unroll");
     k.line("for (int ks = 0; ks < 2; ++ks) {");
     for (int qt = 0; qt < QT; qt++)
-        for (int h = 0; h < (hilo ? 2 : 1); h++) {
+        for (int h = 0; h < NP; h++) {
             const std::string q = std::to_string(qt);
-            k.line("  lsum[" + q + "] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(ones, " + (h ? "pfl[" : "pf[") + q + "][ks], lsum[" + q + "], 0, 0, 0);");
+            k.line("  lsum[" + q + "] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(ones, " + weight(q, "ks", h) + ", lsum[" + q + "], 0, 0, 0);");
         }
     k.line("}");
     if (v_rows) {
@@ -1129,9 +1129,9 @@ bool lower_flash_prefill(const sanic_program_desc* d, int si, int64_t& scratch, 
                     const std::string ix = "[" + std::to_string(dt) + "][" + std::to_string(ks) + "]";
                     const std::string va = "__builtin_bit_cast(bf16x8, (sanic_s16x8)__builtin_shufflevector(vt" + ix + "[0], vt" + ix + "[1], 0, 1, 2, 3, 4, 5, 6, 7))";
                     for (int qt = 0; qt < QT; qt++)
-                        for (int h = 0; h < (hilo ? 2 : 1); h++) {
+                        for (int h = 0; h < NP; h++) {
                             const std::string ov = "o[" + std::to_string(dt) + "][" + std::to_string(qt) + "]";
-                            k.line(ov + " = __builtin_amdgcn_mfma_f32_16x16x32_bf16(" + va + ", " + (h ? "pfl[" : "pf[") + std::to_string(qt) + "][" + std::to_string(ks) + "], " + ov + ", 0, 0, 0);");
+                            k.line(ov + " = __builtin_amdgcn_mfma_f32_16x16x32_bf16(" + va + ", " + weight(std::to_string(qt), std::to_string(ks), h) + ", " + ov + ", 0, 0, 0);");
                         }
                 }
         };
@@ -1156,7 +1156,7 @@ bool lower_flash_prefill(const sanic_program_desc* d, int si, int64_t& scratch, 
     }
     for (int qt = 0; qt < QT; qt++) {
         const std::string q = std::to_string(qt);
-        k.line("    o[dt][" + q + "] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(va, pf[" + q + "][ks], o[dt][" + q + "], 0, 0, 0);");
+        k.line("    o[dt][" + q + "] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(va, " + weight(q, "ks", 0) + ", o[dt][" + q + "], 0, 0, 0);");
     }
     k.line("  }");
     }

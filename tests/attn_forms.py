@@ -19,16 +19,18 @@ def key(s):
     return ir.coordinate(s, s.rank - 1)
 
 
-def attention(NH, NKV, NQ, T, terms=lambda p, s: [], HD=64, dt=ir.BF16, out=ir.BF16, epilogue=None, vt=False):
+def attention(NH, NKV, NQ, T, terms=lambda p, s: [], HD=64, dt=ir.BF16, out=ir.BF16, epilogue=None, vt=False, qscale=False):
     """NH query heads over NKV key/value heads (NH = 0: no head dim), NQ rows over T keys; `terms`
     gives the nodes added to the scores, `epilogue` the node stored, from (p, fold value); `vt`: V is
-    stored [heads, HD, T]."""
+    stored [heads, HD, T]; `qscale`: the query side is q times a stored value per dim."""
     p = Program()
     lead, klead = ((NH,), (NKV,)) if NH else ((), ())
     q, k = p.input("Q", lead + (NQ, HD), dt), p.input("K", klead + (T, HD), dt)
     v = p.input("V", klead + ((HD, T) if vt else (T, HD)), dt)
     if vt:
         v = ir.transpose(v, -2, -1)
+    if qscale:
+        q = ir.map_(ir.MUL, q, p.input("scale", (HD,), ir.F32))
     if NH:
         k, v = ir.expand_heads(k, 0, NH // NKV), ir.expand_heads(v, 0, NH // NKV)
         s = ir.reduce(ir.map_(ir.MUL, ir.unsqueeze(q, 2), ir.unsqueeze(k, 1)), 3, ir.M_ADD)

@@ -322,3 +322,30 @@ def test_windows_that_move_one_way(dev, NH, NKV, NQ, T, dt, name):
     print(err)
     # as test_masks_and_epilogues_that_read_buffers
     assert err < (1e-2 if "any length" not in kind and dt == ir.BF16 else 1e-4)
+
+
+@pytest.mark.parametrize("out", [ir.F32, ir.F16, ir.BF16])
+@pytest.mark.parametrize("NH,NKV,NQ,T,terms,qscale", [
+    (4, 2, 100, 300, A.causal, False), (4, 2, 100, 300, A.EDGES["window"], True), (2, 1, 1000, 1000, A.causal, True), (0, 0, 200, 200, A.causal, True),
+])
+def test_any_length_is_no_further_from_64_bits_than_the_fold(dev, monkeypatch, NH, NKV, NQ, T, terms, qscale, out):
+    """Softmax weights and a computed query side go to the matrix cores as bf16 terms: two where the
+    output is bf16, else three (24 bits, what the f32 fold holds). Against the f64 value before the
+    output's rounding."""
+    forms = {o: A.attention(NH, NKV, NQ, T, terms, out=o, qscale=qscale) for o in (out, ir.F32)}
+    vals = _form_values(forms[out], 600)
+    want = oracle.run_program(forms[ir.F32], vals)["O"]
+    errs, kinds = [], []
+    for generic in (False, True):
+        if generic:
+            monkeypatch.setenv("SANIC_HIP_GENERIC", "1")
+        exe = dev.prepare(forms[out])
+        kinds.append(exe.stage_kernel(0))
+        bufs = {n: dev.from_values(v, forms[out].by_name[n].dtype) for n, v in vals.items()}
+        got = exe.execute(bufs)["O"].read(out, int(np.prod(want.shape))).reshape(want.shape)
+        errs.append(float(np.sqrt(np.mean((got - want) ** 2))))
+    print(kinds, errs, flush=True)
+    assert kinds[0].startswith("skeleton:flash_prefill") and kinds[1].startswith("fold:")
+    # f32: both are 24-bit sums, in different orders (within a quarter of each other); a narrower store's
+    # rounding is the error of both
+    assert errs[0] <= (1.25 if out == ir.F32 else 1.01) * errs[1]
