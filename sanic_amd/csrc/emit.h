@@ -65,6 +65,8 @@ void decode_grid(Code& code, const sanic_stage& st, const std::string& gid);
 std::vector<std::string> leaf_coords(const sanic_stage& st, const sanic_program_desc* d, int l,
                                      const std::string& s);
 std::vector<WindowBound> honest_window(const sanic_program_desc* d, const sanic_stage& st);
+// An edge of the window moves with grid dim `dim`.
+bool window_moves_with(const sanic_program_desc* d, const std::vector<WindowBound>& w, int dim);
 void emit_window(Renderer& R, Code& code, const sanic_stage& st, const std::vector<WindowBound>& w,
                  const std::string& lo, const std::string& hi);
 int64_t dtype_bytes(int dt, int64_t n);

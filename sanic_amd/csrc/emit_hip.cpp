@@ -831,25 +831,25 @@ std::vector<std::string> leaf_coords(const sanic_stage& st, const sanic_program_
 //   where(s < E, K, 0)  → visible iff s ≥ E  → lo = ceil(E)
 // where s is the stream coordinate and E does not depend on it.
 
-static bool depends_on_stream(const sanic_program_desc* d, int node, const std::vector<int>& bind_of_dims) {
-    // bind_of_dims: for the node's dims, which are the stream (value -1)
+// `node`, its dims bound to `bind_of_dims`, moves with the dim or stream bound as `which`.
+static bool depends_on(const sanic_program_desc* d, int node, const std::vector<int>& bind_of_dims, int which) {
     const sanic_node& n = d->nodes[node];
     switch (n.kind) {
     case SANIC_NODE_CONST: return false;
-    case SANIC_NODE_IOTA: return bind_of_dims[0] == SANIC_BIND_STREAM;
-    case SANIC_NODE_COORDINATE: return bind_of_dims[n.dim] == SANIC_BIND_STREAM;
+    case SANIC_NODE_IOTA: return bind_of_dims[0] == which;
+    case SANIC_NODE_COORDINATE: return bind_of_dims[n.dim] == which;
     case SANIC_NODE_MAP: {
         for (int k = 0; k < n.n_in; k++) {
             const sanic_node& m = d->nodes[n.in[k]];
             int lead = n.rank - m.rank;
             std::vector<int> b(m.rank);
             for (int j = 0; j < m.rank; j++) b[j] = m.shape[j] == 1 ? SANIC_BIND_BCAST : bind_of_dims[lead + j];
-            if (depends_on_stream(d, n.in[k], b)) return true;
+            if (depends_on(d, n.in[k], b, which)) return true;
         }
         return false;
     }
     default: {
-        for (int j = 0; j < n.rank; j++) if (bind_of_dims[j] == SANIC_BIND_STREAM) return true;
+        for (int j = 0; j < n.rank; j++) if (bind_of_dims[j] == which) return true;
         return false;
     }
     }
@@ -896,7 +896,7 @@ static void collect_window(const sanic_program_desc* d, int node, const std::vec
     std::vector<int> cb = child_bind(d, node, 0, b);
     std::vector<int> lb = child_bind(d, n.in[0], 0, cb), rb = child_bind(d, n.in[0], 1, cb);
     bool l_s = is_stream_coord(d, cond.in[0], lb), r_s = is_stream_coord(d, cond.in[1], rb);
-    bool l_dep = depends_on_stream(d, cond.in[0], lb), r_dep = depends_on_stream(d, cond.in[1], rb);
+    bool l_dep = depends_on(d, cond.in[0], lb, SANIC_BIND_STREAM), r_dep = depends_on(d, cond.in[1], rb, SANIC_BIND_STREAM);
     bool t_big = is_big_negative(d, n.in[1]), t_zero = is_zero(d, n.in[1]);
     bool f_big = is_big_negative(d, n.in[2]), f_zero = is_zero(d, n.in[2]);
     if (r_s && !l_dep && t_big && f_zero) out.push_back({WindowBound::HI_FLOOR_PLUS1, cond.in[0], lb, node});
@@ -935,6 +935,12 @@ std::vector<WindowBound> honest_window(const sanic_program_desc* d, const sanic_
     std::vector<int> b(st.bind[l], st.bind[l] + ln.rank);
     collect_window(d, st.leaf[l], b, out);
     return out;
+}
+
+bool window_moves_with(const sanic_program_desc* d, const std::vector<WindowBound>& w, int dim) {
+    for (auto& b : w)
+        if (depends_on(d, b.node, b.bind, dim)) return true;
+    return false;
 }
 
 void emit_window(Renderer& R, Code& code, const sanic_stage& st, const std::vector<WindowBound>& w,

@@ -228,6 +228,9 @@ bool attn_plan(const sanic_program_desc* d, int si, AttnPlan& P) {
     if (P.dot.depth % 8 || P.dot.depth > 256) return false;
     P.rep = repk;
     if (P.rep > 8) return false;
+    // a group's chunks are cut from its first head's window: query rows of a causal chunk, or heads
+    // with edges of their own, do not share one
+    if (P.rep > 1 && window_moves_with(d, honest_window(d, st), P.hdim)) return false;
     return true;
 }
 

@@ -102,3 +102,20 @@ UNORDERED = {
     "thirds": lambda p, s: [mask(ir.map_(ir.DIV, row(s), ir.const(3.0)), key(s), -1e30, 0.0),
                             mask(key(s), ir.map_(ir.DIV, row(s), ir.const(3.0)), -1e30, 0.0)],
 }
+
+
+def heads(NH, NKV, T, terms, HD=64):
+    """One query row per head over NKV key/value heads, V as rows."""
+    p = Program()
+    q, k, v = p.input("Q", (NH, HD), ir.BF16), p.input("K", (NKV, T, HD), ir.BF16), p.input("V", (NKV, T, HD), ir.BF16)
+    k, v = ir.expand_heads(k, 0, NH // NKV), ir.expand_heads(v, 0, NH // NKV)
+    s = ir.map_(ir.MUL, ir.reduce(ir.map_(ir.MUL, ir.unsqueeze(q, 1), k), 2, ir.M_ADD), ir.const(HD ** -0.5))
+    for t in terms(p, s):
+        s = ir.map_(ir.ADD, s, t)
+    p.fused("O", (NH, HD), T, [(s, (0, STREAM)), (v, (0, STREAM, 1))], C.online_softmax_weighted(), ir.F32)
+    return p
+
+
+def edge_per_head(p, s):
+    """Each head with a last visible key of its own."""
+    return [mask(ir.unsqueeze(p.input("edge", (s.shape[0],), ir.F32), 1), ir.iota(s.shape[1]), -1e30, 0.0)]

@@ -55,3 +55,9 @@ def test_windows_that_move_one_way_take_the_attention_kernels(NH, NKV, NQ, T, dt
 @pytest.mark.parametrize("NH,NKV,NQ,T,dt", [(8, 2, 512, 512, ir.BF16), (4, 2, 100, 300, ir.BF16), (0, 0, 200, 200, ir.F32)])
 def test_windows_not_bounded_by_their_end_rows_take_the_fold(NH, NKV, NQ, T, dt, name):
     assert A.attention(NH, NKV, NQ, T, A.UNORDERED[name], dt=dt).emit(0)[0].startswith("fold:")
+
+
+def test_heads_that_share_no_window_do_not_take_the_decode_kernel():
+    """The decode kernel cuts a group's keys by its first head's window."""
+    assert A.heads(8, 2, 1000, A.edge_per_head).emit(0)[0].startswith("fold:")
+    assert A.heads(4, 4, 1000, A.edge_per_head).emit(0)[0].startswith("skeleton:attn_decode[rep 1]")

@@ -303,25 +303,33 @@ def test_masks_and_epilogues_that_read_buffers(dev, NH, NKV, NQ, T, dt, terms):
     assert err < (1e-2 if "any length" not in kind and dt == ir.BF16 else 1e-4)
 
 
+def _against_interpreter(dev, prog, seed, bound, kind, **given):
+    vals = dict(_form_values(prog, seed), **given)
+    exe = dev.prepare(prog)
+    print(exe.stage_kernel(0), flush=True)
+    assert exe.stage_kernel(0).startswith(kind)
+    bufs = {n: dev.from_values(v, prog.by_name[n].dtype) for n, v in vals.items()}
+    got = exe.execute(bufs)["O"].read(ir.F32, int(np.prod(prog.by_name["O"].shape))).reshape(prog.by_name["O"].shape)
+    err = max_rel_err(got, oracle.run_program(prog, vals)["O"])
+    print(err)
+    assert err < bound
+
+
 @pytest.mark.parametrize("name", A.EDGES)
 @pytest.mark.parametrize("NH,NKV,NQ,T,dt", [(4, 2, 128, 192, ir.BF16), (4, 2, 100, 300, ir.BF16), (0, 0, 200, 200, ir.F32)])
 def test_windows_that_move_one_way(dev, NH, NKV, NQ, T, dt, name):
     """Falling, halved, clamped and iota-written window edges, rows without a visible key among
     them, against the f64 interpreter."""
     prog = A.attention(NH, NKV, NQ, T, A.EDGES[name], dt=dt, out=ir.F32)
-    vals = _form_values(prog, 560)
-    if "position" in vals:
-        vals["position"] = np.array(-1.0 if dt == ir.F32 else 0.75)
-    exe = dev.prepare(prog)
-    kind = exe.stage_kernel(0)
-    print(kind, flush=True)
-    assert kind.startswith("skeleton:flash_prefill" if dt == ir.BF16 else "skeleton:attn_f32"), kind
-    bufs = {n: dev.from_values(v, prog.by_name[n].dtype) for n, v in vals.items()}
-    got = exe.execute(bufs)["O"].read(ir.F32, int(np.prod(prog.by_name["O"].shape))).reshape(prog.by_name["O"].shape)
-    err = max_rel_err(got, oracle.run_program(prog, vals)["O"])
-    print(err)
+    given = {"position": np.array(-1.0 if dt == ir.F32 else 0.75)} if "position" in prog.by_name else {}
+    whole = NQ % 128 == 0 and T % 64 == 0 and dt == ir.BF16
     # as test_masks_and_epilogues_that_read_buffers
-    assert err < (1e-2 if "any length" not in kind and dt == ir.BF16 else 1e-4)
+    _against_interpreter(dev, prog, 560, 1e-2 if whole else 1e-4, "skeleton:flash_prefill" if dt == ir.BF16 else "skeleton:attn_f32", **given)
+
+
+@pytest.mark.parametrize("NH,NKV,kind", [(8, 2, "fold:"), (4, 4, "skeleton:attn_decode")])
+def test_heads_each_with_a_window(dev, NH, NKV, kind):
+    _against_interpreter(dev, A.heads(NH, NKV, 1000, A.edge_per_head), 590, 1e-5, kind, edge=np.linspace(5.0, 990.0, NH))
 
 
 @pytest.mark.parametrize("out", [ir.F32, ir.F16, ir.BF16])
