@@ -899,7 +899,9 @@ bool lower_attn_decode(const sanic_program_desc* d, int si, int64_t& scratch, Lo
     out.kernel_kind = "skeleton:attn_decode[rep " + std::to_string(REP) + "]" + (writes.empty() ? "" : "+writes" + std::to_string(writes.size())) + (sep ? "+rowwg" : "");
     // the ILP-maximising machine scheduler: C3 11.2 → 10.75 µs (the default strategy interleaves
     // the chunk's loads with its arithmetic to save registers)
-    out.source = "// sched-strategy: iterative-ilp\n" + src.str();
+    // (row-major V keeps the default one: that scheduler ends the compiler with a segmentation fault
+    // on its loops at 4 heads over 16384 positions and at 8 heads over 300)
+    out.source = (vfast ? "// sched-strategy: iterative-ilp\n" : "") + src.str();
     out.variants = nvar;
     std::vector<Arg> args = R.arg_list();
     args.push_back({Arg::SCRATCH, sbase});

@@ -61,3 +61,10 @@ def test_heads_that_share_no_window_do_not_take_the_decode_kernel():
     """The decode kernel cuts a group's keys by its first head's window."""
     assert A.heads(8, 2, 1000, A.edge_per_head).emit(0)[0].startswith("fold:")
     assert A.heads(4, 4, 1000, A.edge_per_head).emit(0)[0].startswith("skeleton:attn_decode[rep 1]")
+
+
+def test_the_decode_kernel_compiles_for_row_major_values():
+    """... which the ILP machine scheduler of the compiler does not survive (8 heads over 300 keys)."""
+    p = A.heads(8, 1, 300, A.prefix)
+    assert p.emit(0)[0].startswith("skeleton:attn_decode[rep 8]")
+    p.precompile()
