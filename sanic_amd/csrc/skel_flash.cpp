@@ -36,6 +36,9 @@ namespace sanic {
 
 namespace {
 
+// Up to this many scores (128 × 128) attention with f32 operands stays with the generic fold.
+const int64_t kFoldScores = 128 * 128;
+
 struct FlashPlan {
     int sleaf = -1, vleaf = -1, max_slot = -1;
     std::vector<int> vec_slots, scalar_slots;
@@ -415,6 +418,12 @@ bool flash_plan(const sanic_program_desc* d, int si, FlashPlan& P) {
         // They go here only where the schedule is the backend's to choose and
         // the tile rows are whole 16-byte chunks of row-major K and V
         if (!sched_is_auto(st.sched) || vc[2] != 1) return false;
+        // A row block's keys are one CU's here: a few query rows over a long cache go to the kernel
+        // below, which gives each block of 16 rows up to 8 workgroups. Here and there, µs: no head axis,
+        // 17 rows over 1024 keys 12.2 and 8.3, 16 over 4096 34.4 and 13.8, 4 over 65536 525 and 121 (the
+        // split fold 403); 32 heads of 16 rows (32 blocks of 16) 12.8 and 10.4 over 1024, of 32 (64) 12.8 and
+        // 11.7, of 64 (128) 13.8 and 14.7, over 4096 36.0 and 38.3
+        if (!P.qexpr && !lean_scratch() && P.NH * ((P.NQ + 15) / 16) <= 64 && P.T >= 1024 && P.T >= 4 * P.NQ && P.NH * P.NQ * P.T > kFoldScores) return false;
         for (int64_t v : {kc[0], kc[1], khc, P.kacc.addr.c0, vc[0], vc[1], vhc, P.vacc.addr.c0})
             if (v % 8) return false;
         if (!P.qexpr)
@@ -1336,7 +1345,7 @@ bool lower_flash_f32(const sanic_program_desc* d, int si, int64_t& scratch, Lowe
     // up to 128 × 128 scores the stage keeps the generic fold and its own choice of schedule (what a
     // program of config A's size is expected to lower to): S = 128 22.3 µs at d = 64 and 8.1 at
     // d = 32 there, 7.1 and 4.9 here
-    if (NH * NQ * T <= 128 * 128) return false;
+    if (NH * NQ * T <= kFoldScores) return false;
     std::vector<int64_t> qc, kc, vc;
     int qh, kh, vh;
     int64_t qhc, khc, vhc;

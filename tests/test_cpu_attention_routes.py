@@ -19,7 +19,7 @@ def _functions(src):
 @pytest.mark.parametrize("NH,NKV,NQ,T,dt", [
     (4, 2, 128, 128, ir.BF16),      # whole tiles
     (4, 2, 100, 300, ir.BF16),      # any length
-    (0, 0, 40, 4096, ir.BF16),      # no head dim
+    (0, 0, 40, 1000, ir.BF16),      # no head dim
     (0, 0, 200, 200, ir.F32),
     (4, 2, 200, 200, ir.F32),
 ])
@@ -68,3 +68,24 @@ def test_the_decode_kernel_compiles_for_row_major_values():
     p = A.heads(8, 1, 300, A.prefix)
     assert p.emit(0)[0].startswith("skeleton:attn_decode[rep 8]")
     p.precompile()
+
+
+@pytest.mark.parametrize("rows", [2, 4, 8])
+@pytest.mark.parametrize("T", [256, 4096, 16384])
+def test_a_few_query_rows_without_heads_take_the_decode_kernel(rows, T):
+    assert A.attention(0, 0, rows, T, A.prefix).emit(0)[0].startswith(f"skeleton:attn_decode[rep {rows}]")
+
+
+def test_query_rows_that_share_no_window_do_not_take_the_decode_kernel():
+    """The decode kernel cuts a group's keys by its first row's window."""
+    for form in (A.chunk, A.causal):
+        assert A.attention(0, 0, 8, 4096, form).emit(0)[0].startswith("skeleton:attn_f32")
+        assert A.attention(0, 0, 8, 300, form).emit(0)[0].startswith("skeleton:flash_prefill")
+
+
+@pytest.mark.parametrize("NH,NKV,NQ,T,kind", [
+    (0, 0, 4, 65536, "attn_f32"), (0, 0, 17, 1024, "attn_f32"), (2, 2, 2, 32768, "attn_f32"), (32, 8, 32, 4096, "attn_f32"),
+    (0, 0, 17, 1000, "flash_prefill"), (32, 8, 33, 4096, "flash_prefill"), (0, 0, 300, 1024, "flash_prefill"), (2, 2, 2, 1024, "flash_prefill"),
+])
+def test_a_few_rows_over_a_long_cache_take_the_kernel_that_splits_the_keys(NH, NKV, NQ, T, kind):
+    assert A.attention(NH, NKV, NQ, T, A.prefix).emit(0)[0].startswith("skeleton:" + kind)

@@ -327,6 +327,17 @@ def test_windows_that_move_one_way(dev, NH, NKV, NQ, T, dt, name):
     _against_interpreter(dev, prog, 560, 1e-2 if whole else 1e-4, "skeleton:flash_prefill" if dt == ir.BF16 else "skeleton:attn_f32", **given)
 
 
+@pytest.mark.parametrize("rows,T,terms,kind", [
+    (2, 300, A.prefix, "skeleton:attn_decode"), (8, 300, A.prefix, "skeleton:attn_decode"),
+    (5, 2049, A.prefix, "skeleton:attn_decode"), (8, 1000, A.bias, "skeleton:attn_decode"),
+    (17, 1024, A.prefix, "skeleton:attn_f32"), (9, 4096, A.causal, "skeleton:attn_f32"), (8, 2050, A.chunk, "skeleton:attn_f32"),
+    (8, 1000, A.chunk, "skeleton:flash_prefill"), (3, 300, A.causal, "skeleton:flash_prefill"),
+])
+def test_few_query_rows_without_heads(dev, rows, T, terms, kind):
+    """Rows sharing a window, and rows each with a window of its own, over short and long caches."""
+    _against_interpreter(dev, A.attention(0, 0, rows, T, terms, out=ir.F32), 580, 1e-5, kind)
+
+
 @pytest.mark.parametrize("NH,NKV,kind", [(8, 2, "fold:"), (4, 4, "skeleton:attn_decode")])
 def test_heads_each_with_a_window(dev, NH, NKV, kind):
     _against_interpreter(dev, A.heads(NH, NKV, 1000, A.edge_per_head), 590, 1e-5, kind, edge=np.linspace(5.0, 990.0, NH))
