@@ -67,7 +67,7 @@ std::string str(int64_t v) { return std::to_string(v); }
 
 }  // namespace
 
-bool lower_skinny(const sanic_program_desc* d, int si, LoweredStage& out) {
+bool lower_skinny(const sanic_program_desc* d, int si, LoweredStage& out, bool gemm_too) {
     GemmPlan P;
     if (!gemm_plan(d, si, P)) return false;
     const sanic_stage& st = d->stages[si];
@@ -186,7 +186,7 @@ bool lower_skinny(const sanic_program_desc* d, int si, LoweredStage& out) {
         while (bn > 32 && mb * (N / bn) < 256) bn /= 2;
         const double step = narrow ? (bm == 64 ? 0.52 : 0.68) : bn == 128 ? 1.05 : bn == 64 ? 0.68 : bm == 64 ? (packed ? 0.43 : 0.3) : packed ? 0.52 : 0.55;
         const double gemm = (split ? 5.0 : narrow ? 1.5 : 0.0) + rounds(mb * ((N + bn - 1) / bn)) * (double)((K + 63) / 64) * step;
-        if (N >= bn && (!narrow || aligned) && gemm < std::min(small, tall ? high : small)) return false;
+        if (gemm_too && N >= bn && (!narrow || aligned) && gemm < std::min(small, tall ? high : small)) return false;
         tall &= high < small;
     }
     if (!tall) tall_row = -1;

@@ -140,6 +140,6 @@ def test_int4_gemv_folds_each_run_as_scale_and_zero():
 
 def test_a_program_over_the_static_scratch_keeps_the_form_without_it():
     """The operand planes of a GEMM off the tiles count towards the scratch of execute_static: a call
-    whose planes would not fit (4099 x 2048 in two bf16 planes: 33.7 MB) keeps the generic fold."""
-    assert configs.rmsnorm_projection(M=4099, K=2048, N=512).emit(0)[0].startswith("fold:")
+    whose planes would not fit (4099 x 2048 in two bf16 planes: 33.7 MB) takes the kernel without them."""
+    assert configs.rmsnorm_projection(M=4099, K=2048, N=512).emit(0)[0].startswith("skeleton:gemm_rows[")
     assert configs.rmsnorm_projection(M=1999, K=2048, N=512).emit(0)[0].startswith("skeleton:gemm[")

@@ -6,6 +6,7 @@ import oracle
 from sanic_amd import configs, ir
 from sanic_amd.backend import from_bf16_bits
 from tests.test_gpu_skeletons import bf16_rel, _bf16_vals
+from tests import gemm_forms as forms
 from tests.util import run_on_gpu
 
 pytestmark = pytest.mark.gpu
@@ -121,10 +122,10 @@ def _same_as_generic(dev, monkeypatch, prog, vals, scale):
 
 
 # rows, k and columns off every tile: below one tile, one past it, K tiles odd in number and
-# overlapping, columns not a multiple of 8
+# overlapping, columns not a multiple of 8; operand planes past the static scratch
 RAGGED = [(2, 64, 32), (65, 128, 96), (200, 2048, 8192), (33, 200, 77), (100, 72, 1003), (129, 1000, 333),
           (256, 128, 8224), (127, 832, 5184), (8, 4160, 96), (20, 2200, 49), (40, 2048, 8192), (300, 2000, 1088), (250, 2056, 2000),
-          (90, 1536, 2820)]
+          (90, 1536, 2820), (4100, 2048, 136)]
 
 
 @pytest.mark.parametrize("kmajor", [False, True])
@@ -142,7 +143,7 @@ def test_rmsnorm_gemm_any_size(dev, monkeypatch, M, K, N, kmajor):
     _same_as_generic(dev, monkeypatch, prog, vals, scale=0.02 * K)
 
 
-@pytest.mark.parametrize("M,K,N,G", [(2, 64, 32, 64), (16, 2048, 8192, 64), (100, 1152, 777, 64), (65, 384, 1000, 128),
+@pytest.mark.parametrize("M,K,N,G", [(40, 1056, 8192, 1056), (2, 64, 32, 64), (16, 2048, 8192, 64), (100, 1152, 777, 64), (65, 384, 1000, 128),
                                      (33, 192, 64, 64), (17, 256, 300, 32), (31, 8320, 48, 64),
                                      (16, 512, 16, 512), (100, 1920, 3270, 64), (103, 1920, 777, 32), (128, 512, 512, 32)])
 def test_int4_gemm_any_size(dev, monkeypatch, M, K, N, G):
@@ -155,6 +156,23 @@ def test_int4_gemm_any_size(dev, monkeypatch, M, K, N, G):
     x[0, 0] = -np.inf
     s[N - 1, 0] = np.nan
     _same_as_generic(dev, monkeypatch, prog, vals, scale=0.2 * K)
+
+
+@pytest.mark.parametrize("M,K,N,order", [
+    (500, 2040, 1000, "nk"), (130, 1000, 640, "nk"), (257, 72, 96, "nk"),       # GEMM tiles whose first K tile overlaps the second
+    (8, 256, 64, "nk"), (40, 200, 300, "nk"), (200, 1968, 1088, "nk"), (20, 136, 100, "kn"), (5, 2048, 72, "kn"),   # few-row kernel, x as stored
+    (40, 2048, 8192, "nk view"), (100, 1000, 2056, "kn view"), (500, 200, 1000, "nk view"), (300, 2048, 4104, "kn view"),
+])
+def test_projection_without_a_norm(dev, monkeypatch, M, K, N, order):
+    """y = x · W with both operands as stored; a view of W keeps what the stored order takes."""
+    prog = forms.projection(M, K, N, order)
+    x = _bf16_vals(351, M * K).reshape(M, K)
+    w = _bf16_vals(352, K * N, 0.0, 0.02).reshape(prog.by_name["W"].shape)
+    kind = _same_as_generic(dev, monkeypatch, prog, {"x": x, "W": w}, scale=0.02 * K)
+    assert kind.startswith("skeleton:gemm") and (M >= 500) <= ("any size" in kind or "view" in order), kind
+    x[M - 1, K - 1] = np.inf
+    w[-1, -1] = np.nan
+    _same_as_generic(dev, monkeypatch, prog, {"x": x, "W": w}, scale=0.02 * K)
 
 
 @pytest.mark.parametrize("kmajor", [False, True])
