@@ -67,6 +67,27 @@ std::string str(int64_t v) { return std::to_string(v); }
 
 }  // namespace
 
+// A K of many stages under few output points: here and in the GEMM a workgroup walks its columns'
+// whole K, the split fold gives every point up to 64 workgroups. Estimates in µs, of a round of
+// workgroups here (stages of 1024 k over 8 waves, 512 of a [K, N] weight) and of the fold. Here and
+// there: [N, K], M = 2, N = 16, K = 65536 33 and 28, 131072 82 and 29; M = 2, N = 64, K = 131072 87 and 111;
+// M = 8, N = 16, K = 131072 115 and 110, 196608 177 and 115; M = 16, N = 16, K = 131072 154 and 222, 196608
+// 234 and 223; [K, N], M = 2, N = 32, K = 65536 66 and 56, 131072 149 and 80; M = 2, N = 64, K = 65536 134 and
+// 172, 131072 274 and 205; M = 8, N = 32, K = 196608 278 and 470.
+bool split_fold_faster(const sanic_program_desc* d, int si) {
+    GemmPlan P;
+    if (!gemm_plan(d, si, P) || !P.rslots.empty() || P.M > 16 || P.K < 32768) return false;
+    const sanic_stage& st = d->stages[si];
+    const sanic_node& wn = d->nodes[st.leaf[P.w]];
+    std::vector<Sym> cw(wn.rank);
+    for (int j = 0; j < wn.rank; j++) cw[j] = st.bind[P.w][j] == SANIC_BIND_STREAM ? Sym::var(1) : st.bind[P.w][j] == P.ndim ? Sym::var(0) : Sym();
+    Access w;
+    if (!sched_is_auto(st.sched) || !sym_access(d, st.leaf[P.w], cw, {P.N, P.K}, w)) return false;
+    const double points = (double)(P.M * P.N), m = (double)P.M, k = (double)P.K;
+    if (contiguous_runs(w, 1, 8)) return 2.0 + 0.82 * points < k / 1024.0 * (0.5 + 0.042 * m);
+    return 2.0 + 0.82 * points + 6.5e-6 * k * points < k / 512.0 * ((P.N > 32 ? 1.02 : 0.54) + 0.018 * m);
+}
+
 bool lower_skinny(const sanic_program_desc* d, int si, LoweredStage& out, bool gemm_too) {
     GemmPlan P;
     if (!gemm_plan(d, si, P)) return false;

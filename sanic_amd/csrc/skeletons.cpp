@@ -1840,13 +1840,15 @@ bool lower_gemv_kmajor(const sanic_program_desc* d, int si, int64_t& scratch, Lo
 
 bool lower_skeleton(const sanic_program_desc* d, int si, int64_t& scratch, LoweredStage& out) {
     if (lower_gemv_kmajor(d, si, scratch, out)) return true;
-    if (lower_skinny(d, si, out, true)) return true;
-    const int64_t base = scratch;
-    if (lower_gemm(d, si, scratch, out)) return true;
-    scratch = base;
-    // what the few-row kernel left to the GEMM and the GEMM does not take (off its tiles: weights that
-    // are views, one 4-bit group over a K off the tiles, operand planes past the static scratch)
-    if (lower_skinny(d, si, out, false)) return true;
+    if (!split_fold_faster(d, si)) {
+        if (lower_skinny(d, si, out, true)) return true;
+        const int64_t base = scratch;
+        if (lower_gemm(d, si, scratch, out)) return true;
+        scratch = base;
+        // what the few-row kernel left to the GEMM and the GEMM does not take (off its tiles: weights that
+        // are views, one 4-bit group over a K off the tiles, operand planes past the static scratch)
+        if (lower_skinny(d, si, out, false)) return true;
+    }
     // (up to 8 query rows without a head axis are a group of the decode kernel's, which spreads the keys
     // over the chip where flash gives a row block one workgroup: 8 rows over 256 / 4096 / 16384 keys
     // 8.1 / 9.8 / 22.5 µs, flash 7.3 / 34.7 / 127)

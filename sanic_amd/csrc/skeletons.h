@@ -81,6 +81,8 @@ bool exact_in_two(const sanic_program_desc* d, const sanic_stage& st, int e, int
 std::string expr_rest(Renderer& R, Code& code, int e, int w, const std::function<std::string(int)>& item);
 
 bool lower_gemm(const sanic_program_desc* d, int si, int64_t& scratch, LoweredStage& out);
+// The generic split fold is faster than either kernel.
+bool split_fold_faster(const sanic_program_desc* d, int si);
 // `gemm_too`: decline where the GEMM's tiles are estimated to be faster.
 bool lower_skinny(const sanic_program_desc* d, int si, LoweredStage& out, bool gemm_too);
 bool lower_flash_f32(const sanic_program_desc* d, int si, int64_t& scratch, LoweredStage& out);

@@ -23,3 +23,14 @@ def test_one_4bit_group_over_a_k_off_the_tiles_takes_a_kernel(M):
 def test_operand_planes_past_the_static_scratch_leave_a_kernel(M, K, N, kmajor):
     """Rows whose two bf16 planes pass the 32 MiB of execute_static: the kernel without planes."""
     assert configs.rmsnorm_projection(M=M, K=K, N=N, kmajor=kmajor).emit(0)[0].startswith("skeleton:gemm_rows")
+
+
+@pytest.mark.parametrize("M,K,N,order,rows", [
+    (2, 32768, 16, "nk", True), (2, 131072, 16, "nk", False), (2, 131072, 64, "nk", True), (2, 262144, 64, "nk", False),
+    (8, 65536, 16, "nk", True), (8, 196608, 16, "nk", False), (16, 131072, 16, "nk", True),
+    (2, 32768, 32, "kn", True), (2, 131072, 32, "kn", False), (2, 65536, 64, "kn", True), (2, 131072, 64, "kn", False), (8, 196608, 32, "kn", True), (2, 196608, 4096, "nk", True),
+])
+def test_a_long_k_under_few_points_keeps_the_split_fold(M, K, N, order, rows):
+    """Where one workgroup per column block would walk K longer than the fold that splits each point."""
+    kind = G.projection(M, K, N, order).emit(0)[0]
+    assert kind.startswith("skeleton:gemm_rows" if rows else "fold:split"), kind
