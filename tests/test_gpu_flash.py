@@ -190,6 +190,7 @@ F, B = ir.F32, ir.BF16
     (0, 0, 65, 300, 16, 128, False, (F, F, F)),   # more keys than rows, value tiles of 8
     (6, 2, 60, 60, 128, 16, True, (F, F, F)),     # grouped heads, d above the value size
     (16, 16, 260, 5, 48, 32, False, (B, F, B)),   # fewer keys than a tile, stored types mixed
+    (2, 1, 150, 150, 128, 128, True, (F, F, F)),  # the largest operands, whose registers are the most
 ])
 def test_attention_f32_matches_generic(dev, monkeypatch, NH, NKV, NQ, T, HD, E, causal, dtypes):
     """Both evaluations are f32 throughout: scores within HD · 2^-24 of Σ|q·k| ≤ HD of each other,
@@ -368,3 +369,33 @@ def test_any_length_is_no_further_from_64_bits_than_the_fold(dev, monkeypatch, N
     # f32: both are 24-bit sums, in different orders (within a quarter of each other); a narrower store's
     # rounding is the error of both
     assert errs[0] <= (1.25 if out == ir.F32 else 1.01) * errs[1]
+
+
+@pytest.mark.parametrize("NH,NKV,S,window", [(4, 2, 512, 0), (2, 1, 2048, 0), (4, 1, 1024, 300), (8, 2, 4096, 0)])
+def test_small_launches_are_no_further_from_64_bits_than_large_ones(dev, NH, NKV, S, window):
+    """Whole tiles in 64-row blocks, and key teams that each keep a running maximum of their own, round
+    the softmax weights to bf16 against other reference points than the 128-row form: other
+    last bits of the output, the same distance from 64 bits."""
+    def terms(p, s):
+        low = [A.mask(A.key(s), ir.map_(ir.SUB, A.row(s), ir.const(window - 1.0)), -1e30, 0.0)]
+        return A.causal(p, s) + (low if window else [])
+    prog = A.attention(NH, NKV, S, S, terms, out=ir.F32)
+    vals = _form_values(prog, 620)
+    q, k, v = (np.asarray(vals[n], np.float64) for n in "QKV")
+    i, j = np.arange(S)[:, None], np.arange(S)[None, :]
+    hidden = (j > i) | ((j < i - (window - 1)) if window else False)
+    want = np.empty_like(q)
+    for h in range(NH):
+        s = np.where(hidden, -np.inf, q[h] @ k[h // (NH // NKV)].T / 8.0)
+        e = np.exp(s - s.max(axis=1, keepdims=True))
+        want[h] = e @ v[h // (NH // NKV)] / e.sum(axis=1, keepdims=True)
+    errs, kinds, outs = [], [], []
+    for variant in (0, 1):
+        exe = dev.prepare(prog.with_variants({0: variant}))
+        kinds.append(exe.stage_kernel(0))
+        bufs = {n: dev.from_values(x, prog.by_name[n].dtype) for n, x in vals.items()}
+        outs.append(exe.execute(bufs)["O"].read(ir.F32, want.size).reshape(want.shape))
+        errs.append(float(np.sqrt(np.mean((outs[-1] - want) ** 2))))
+    apart = float(np.sqrt(np.mean((outs[0] - outs[1]) ** 2) / np.mean(want ** 2)))
+    print(kinds, errs, "rms", float(np.sqrt(np.mean(want ** 2))), "apart", apart, flush=True)
+    assert errs[0] <= 1.02 * errs[1]
