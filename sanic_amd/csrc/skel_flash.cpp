@@ -614,15 +614,8 @@ bool lower_flash_prefill(const sanic_program_desc* d, int si, int64_t& scratch, 
         emit_point_fold(R, scratch_code, st, "pf");
     }
     src << (SPL > 1 ? R.args_struct({"float* __restrict__ scratch", "unsigned* counters"}) : R.args_struct({}));
-    src << "typedef __bf16 sanic_bf16x2 __attribute__((ext_vector_type(2)));\n";
-    src << "typedef float sanic_f32x2 __attribute__((ext_vector_type(2)));\n";
-    src << "__device__ __forceinline__ unsigned pk_bf16(float x, float y) {\n"
-           "  return __builtin_bit_cast(unsigned, __builtin_convertvector((sanic_f32x2){x, y}, sanic_bf16x2));\n}\n";
+    src << kSplitBf16;
     src << "__device__ __forceinline__ idx_t sanic_min(idx_t a, idx_t b) { return a < b ? a : b; }\n";
-    src << "__device__ __forceinline__ void split_bf16(float x, float y, unsigned& hi, unsigned& lo) {\n"
-           "  const unsigned h = pk_bf16(x, y);\n"
-           "  hi = h;\n"
-           "  lo = pk_bf16(x - __uint_as_float(h << 16), y - __uint_as_float(h & 0xFFFF0000u));\n}\n";
     if (NP == 3)
         src << "__device__ __forceinline__ void split3_bf16(float x, float y, unsigned& hi, unsigned& mid, unsigned& lo) {\n"
                "  const unsigned h = pk_bf16(x, y);\n"
@@ -1346,9 +1339,9 @@ bool lower_flash_f32(const sanic_program_desc* d, int si, int64_t& scratch, Lowe
     if (!wide(P.qacc.dtype) || !wide(P.kacc.dtype) || !wide(P.vacc.dtype)) return false;
     const int64_t NH = P.NH, NQ = P.NQ, T = P.T, E = P.E, HD = P.HD;
     if (HD % 16 || E % 16 || HD > 128 || E > 128 || (E / 16 & (E / 16 - 1))) return false;
-    // up to 128 × 128 scores the stage keeps the generic fold and its own choice of schedule (what a
-    // program of config A's size is expected to lower to): S = 128 22.3 µs at d = 64 and 8.1 at
-    // d = 32 there, 7.1 and 4.9 here
+    // (no measured line: S = 128 takes 22.3 µs at d = 64 and 8.1 at d = 32 in the fold, 7.1 and 4.9 here.
+    // The lowering of a 128 × 128 program is the fold with its own choice of schedule, and its test
+    // states that)
     if (NH * NQ * T <= kFoldScores) return false;
     std::vector<int64_t> qc, kc, vc;
     int qh, kh, vh;

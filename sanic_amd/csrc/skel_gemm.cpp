@@ -989,14 +989,7 @@ bool lower_gemm(const sanic_program_desc* d, int si, int64_t& scratch, LoweredSt
     src << "typedef short sanic_s16x4 __attribute__((ext_vector_type(4)));\n";
     src << "typedef short sanic_s16x8 __attribute__((ext_vector_type(8)));\n";
     src << "typedef __attribute__((__vector_size__(4 * sizeof(float)))) float f32x4;\n";
-    src << "typedef __bf16 sanic_bf16x2 __attribute__((ext_vector_type(2)));\n";
-    src << "typedef float sanic_f32x2 __attribute__((ext_vector_type(2)));\n";
-    src << "__device__ __forceinline__ unsigned pk_bf16(float x, float y) {\n"
-           "  return __builtin_bit_cast(unsigned, __builtin_convertvector((sanic_f32x2){x, y}, sanic_bf16x2));\n}\n";
-    src << "__device__ __forceinline__ void split_bf16(float x, float y, unsigned& hi, unsigned& lo) {\n"
-           "  const unsigned h = pk_bf16(x, y);\n"
-           "  hi = h;\n"
-           "  lo = pk_bf16(x - __uint_as_float(h << 16), y - __uint_as_float(h & 0xFFFF0000u));\n}\n";
+    src << kSplitBf16;
     src << R.args_struct(pre ? std::vector<std::string>{"float* __restrict__ scratch"} : std::vector<std::string>{});
     if (pre) src << "extern \"C\" __global__ void __launch_bounds__(256) " << kname << "_pre(Args a) {\n" << R.entry() << kp.str() << "}\n";
     src << "extern \"C\" __global__ void __launch_bounds__(" << NTH << ") " << kname << "(Args a) {\n" << R.entry() << k.str() << "}\n";

@@ -617,15 +617,8 @@ bool lower_skinny(const sanic_program_desc* d, int si, LoweredStage& out, bool g
     src << "typedef short sanic_s16x4 __attribute__((ext_vector_type(4)));\n";
     src << "typedef short sanic_s16x8 __attribute__((ext_vector_type(8)));\n";
     src << "typedef __attribute__((__vector_size__(4 * sizeof(float)))) float f32x4;\n";
-    src << "typedef __bf16 sanic_bf16x2 __attribute__((ext_vector_type(2)));\n";
-    src << "typedef float sanic_f32x2 __attribute__((ext_vector_type(2)));\n";
+    src << kSplitBf16;
     src << "typedef unsigned sanic_u32x4_any __attribute__((ext_vector_type(4), aligned(1)));\n";
-    src << "__device__ __forceinline__ unsigned pk_bf16(float x, float y) {\n"
-           "  return __builtin_bit_cast(unsigned, __builtin_convertvector((sanic_f32x2){x, y}, sanic_bf16x2));\n}\n";
-    src << "__device__ __forceinline__ void split_bf16(float x, float y, unsigned& hi, unsigned& lo) {\n"
-           "  const unsigned h = pk_bf16(x, y);\n"
-           "  hi = h;\n"
-           "  lo = pk_bf16(x - __uint_as_float(h << 16), y - __uint_as_float(h & 0xFFFF0000u));\n}\n";
     src << R.args_struct({});
     src << "extern \"C\" __global__ void __launch_bounds__(" << NTH << ") " << kname << "(Args a) {\n" << R.entry() << k.str() << "}\n";
     out.kernel_kind = "skeleton:gemm_rows[" + str(RBM) + "x" + str(BN) + (split ? ",a2" : "") + (packed ? unit < 64 ? ",g32" : ",grp" : "") + (kn ? ",kn" : "") + ",w" + str(NW) + "x" + str(ITER) + "]";

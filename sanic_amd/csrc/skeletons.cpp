@@ -71,6 +71,16 @@ static void sym_range(const Sym& s, const std::vector<int64_t>& ext, int64_t& lo
 }
 
 // Coordinates of a Reindex/View node's source, as Syms; false when not affine.
+const char* kSplitBf16 =
+    "typedef __bf16 sanic_bf16x2 __attribute__((ext_vector_type(2)));\n"
+    "typedef float sanic_f32x2 __attribute__((ext_vector_type(2)));\n"
+    "__device__ __forceinline__ unsigned pk_bf16(float x, float y) {\n"
+    "  return __builtin_bit_cast(unsigned, __builtin_convertvector((sanic_f32x2){x, y}, sanic_bf16x2));\n}\n"
+    "__device__ __forceinline__ void split_bf16(float x, float y, unsigned& hi, unsigned& lo) {\n"
+    "  const unsigned h = pk_bf16(x, y);\n"
+    "  hi = h;\n"
+    "  lo = pk_bf16(x - __uint_as_float(h << 16), y - __uint_as_float(h & 0xFFFF0000u));\n}\n";
+
 bool sym_child_coords(const sanic_program_desc* d, int node, const std::vector<Sym>& c,
                       const std::vector<int64_t>& ext, std::vector<Sym>& sc) {
     const sanic_node& n = d->nodes[node];

@@ -25,6 +25,9 @@ struct Sym {
     std::string render(const std::vector<std::string>& vars) const;
 };
 
+// Kernel functions: two floats packed as bf16 (RNE), and as hi + lo bf16 pairs.
+extern const char* kSplitBf16;
+
 // An Input read through Reindex/View chains, as element address = Sym.
 struct Access {
     int buffer = -1, dtype = -1, node = -1;
