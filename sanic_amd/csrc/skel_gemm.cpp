@@ -925,7 +925,12 @@ bool lower_gemm(const sanic_program_desc* d, int si, int64_t& scratch, LoweredSt
         k.line("__syncthreads();");
     }
     // finish: project, epilogue, narrowing store per element
-    if (rag) k.line("bool odd = false;");
+    if (rag) {
+        k.line("bool odd = false;");
+        k.line("#pragma unroll");
+        k.line("for (int p = 0; p < " + std::to_string(MT * NT * 4) + "; ++p) odd |= !(__builtin_fabsf(acc[p / " + std::to_string(NT * 4) + "][p / 4 % " + std::to_string(NT) + "][p % 4]) <= 3.402823466e38f);");
+        k.line("if (!odd) {");
+    }
     k.line("#pragma unroll");
     k.line("for (int i = 0; i < " + std::to_string(MT) + "; ++i)");
     k.line("  #pragma unroll");
@@ -958,15 +963,15 @@ bool lower_gemm(const sanic_program_desc* d, int si, int64_t& scratch, LoweredSt
         R.memo.pop_back();
         k.line(store_stmt(R.param(st.out_buffer), lin, st.out_dtype, v, false, d->buffers[st.out_buffer].scale));
     };
-    if (rag) k.line("odd |= !(__builtin_fabsf(acc[i][j][r]) <= 3.402823466e38f);");
     finish();
     k.indent -= 3;
     k.line("    }");
     if (rag) {
         // Infinities and NaNs: the hi + lo split of an infinity, the repeated rows and the zeroed
         // overlap do not carry them as the fold does, so a lane with such a sum folds its points
-        // again, element by element.
-        k.line("if (odd) {");
+        // again, element by element (instead of storing them: the output may be bound to what the
+        // epilogue reads).
+        k.line("} else {");
         k.indent++;
         k.line("#pragma nounroll");
         k.line("for (int p = 0; p < " + std::to_string(MT * NT * 4) + "; ++p) {");

@@ -6,6 +6,7 @@ import oracle
 from sanic_amd import configs, ir
 from sanic_amd.backend import from_bf16_bits
 from tests.test_gpu_skeletons import bf16_rel, _bf16_vals
+from tests import attn_forms as A
 from tests import gemm_forms as forms
 from tests.util import run_on_gpu
 
@@ -173,6 +174,27 @@ def test_projection_without_a_norm(dev, monkeypatch, M, K, N, order):
     x[M - 1, K - 1] = np.inf
     w[-1, -1] = np.nan
     _same_as_generic(dev, monkeypatch, prog, {"x": x, "W": w}, scale=0.02 * K)
+
+
+@pytest.mark.parametrize("prog", [forms.projection(500, 2040, 1000, "nk", residual=True), forms.projection(20, 200, 300, "nk", residual=True),
+                                  A.attention(4, 2, 100, 300, A.causal, epilogue=A.residual), A.attention(4, 2, 200, 200, A.causal, dt=ir.F32, epilogue=A.residual)])
+def test_residual_and_output_in_one_buffer(dev, prog):
+    """y = R + f(x) bound to R itself, an infinity among the operands: every point is read and
+    stored once, so the bits are those of two buffers."""
+    out = prog.buffers[-1].name
+    vals = {b.name: _bf16_vals(360 + i, int(np.prod(b.shape))) for i, b in enumerate(prog.buffers[:-1])}
+    vals["V" if "V" in vals else "x"][10] = np.inf       # (a key that every row of its head sees)
+    exe = dev.prepare(prog)
+    print(exe.stage_kernel(0), flush=True)
+    assert exe.stage_kernel(0).startswith("skeleton:")
+    bufs = {n: dev.from_values(v, prog.by_name[n].dtype) for n, v in vals.items()}
+    bufs[out] = dev.from_values(vals["R"], ir.BF16)
+    exe.execute_static(bufs)
+    want = bufs[out].download()
+    assert not np.isfinite(from_bf16_bits(np.frombuffer(want, np.uint16))).all()
+    bufs[out] = bufs["R"]
+    exe.execute_static(bufs)
+    assert bufs["R"].download() == want
 
 
 @pytest.mark.parametrize("kmajor", [False, True])
