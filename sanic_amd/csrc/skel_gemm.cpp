@@ -929,7 +929,7 @@ bool lower_gemm(const sanic_program_desc* d, int si, int64_t& scratch, LoweredSt
         k.line("bool odd = false;");
         k.line("#pragma unroll");
         k.line("for (int p = 0; p < " + std::to_string(MT * NT * 4) + "; ++p) odd |= !(__builtin_fabsf(acc[p / " + std::to_string(NT * 4) + "][p / 4 % " + std::to_string(NT) + "][p % 4]) <= 3.402823466e38f);");
-        k.line("if (!odd) {");
+        k.line("if (!__any(odd)) {");
     }
     k.line("#pragma unroll");
     k.line("for (int i = 0; i < " + std::to_string(MT) + "; ++i)");
@@ -968,9 +968,9 @@ bool lower_gemm(const sanic_program_desc* d, int si, int64_t& scratch, LoweredSt
     k.line("    }");
     if (rag) {
         // Infinities and NaNs: the hi + lo split of an infinity, the repeated rows and the zeroed
-        // overlap do not carry them as the fold does, so a lane with such a sum folds its points
+        // overlap do not carry them as the fold does, so a wave with such a sum folds its points
         // again, element by element (instead of storing them: the output may be bound to what the
-        // epilogue reads).
+        // epilogue reads; the wave at once: a branch per lane took 0.6 µs of 23 at M = 200).
         k.line("} else {");
         k.indent++;
         k.line("#pragma nounroll");
