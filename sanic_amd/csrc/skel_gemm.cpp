@@ -214,7 +214,6 @@ bool lower_gemm(const sanic_program_desc* d, int si, int64_t& scratch, LoweredSt
         const sanic_node& n = d->nodes[st.leaf[leaf]];
         return n.kind == SANIC_NODE_INPUT && n.dtype == SANIC_BF16;
     };
-    bool splitB = !raw_bf16_input(P.w);
     bool splitA = true;
     {
         const sanic_expr& e = d->exprs[c.into[P.cslots[0]]];
@@ -262,7 +261,10 @@ bool lower_gemm(const sanic_program_desc* d, int si, int64_t& scratch, LoweredSt
         Code l1, d1;
         render_weight_run(d, st.leaf[P.w], cwt, {K, N}, l1, d1, "kk", "n0", "_p", tb, td, tok, tc, tr, false);
         bkn = tok && tc;
+        if (bkn) raw = tr;
     }
+    // (a weight whose runs are stored bf16 as they are, also through a view, goes as loaded)
+    bool splitB = raw.empty();
     // Grouped dequantization (packed 4-bit weights): the weight leaf is q·s ± z with q a packed
     // 4-bit run and s, z constant over every 64-wide K tile (a quantization group of 64 or a
     // multiple of it). Per tile, Σ_k x·w = s·Σ_k x·q ± z·Σ_k x, so the MFMA's B operand is q

@@ -13,6 +13,15 @@ def test_a_weight_that_is_a_view_takes_a_kernel_at_every_row_count(M, K, N, orde
     assert G.projection(M, K, N, order).emit(0)[0].startswith("skeleton:gemm")
 
 
+@pytest.mark.parametrize("order", ["nk view", "kn view"])
+@pytest.mark.parametrize("M,K,N", [(64, 64, 32), (128, 512, 128), (500, 200, 1000)])
+def test_the_gemm_over_a_weight_that_is_a_view_compiles(M, K, N, order):
+    """... its runs are stored bf16: one product, no lo part."""
+    p = G.projection(M, K, N, order)
+    assert p.emit(0)[0].startswith("skeleton:gemm[") and ",b2" not in p.emit(0)[0]
+    p.precompile()
+
+
 @pytest.mark.parametrize("M", [32, 40, 100, 200, 300])
 def test_one_4bit_group_over_a_k_off_the_tiles_takes_a_kernel(M):
     assert configs.int4_matmul(M=M, K=1056, G=1056, N=8192).emit(0)[0].startswith("skeleton:gemm_rows")
