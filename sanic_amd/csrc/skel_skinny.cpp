@@ -17,11 +17,14 @@
 // the matrix cores as well. (The weights pass through registers: with direct-to-LDS transfers in
 // flight the compiler waits for all of them before the first row run is used.)
 //
-// The bound is the weight stream. Generic fold → here, K = 2048, N = 8192: M = 8 [N, K] weights
-// 25 → 7.6 µs (33.6 MB: 4.4 TB/s), [K, N] weights 11.5 µs (14.8 before the two halves of each
-// line met on one XCD); 4-bit, M = 16: 246 → 5.8 µs. K = 8192, N = 2048, M = 8: 14.2 µs.
-// Tall tiles, 32-row ones or GEMM tiles → here: 4-bit, M = 33, N = 8192 14.9 → 10.5 µs; K = 1968,
-// N = 1088, M = 300 23.8 → 18.8 (bound by L1 misses, 30 bytes a clock and CU, as the GEMM's tiles).
+// The bound is the weight stream, above 32 rows the arithmetic between its stages. Generic fold → here, K = 2048,
+// N = 8192, launches on one weight (33.6 MB, which the Infinity Cache holds; 4-bit 9.5 MB): M = 8 [N, K]
+// weights 25 → 7.6 µs, [K, N] weights 11.5 µs (14.8 before the two halves of each line met on one XCD);
+// 4-bit, M = 16: 246 → 5.8 µs. On three weights in turn 8.8 µs (3.8 TB/s) and 8.1. K = 8192, N = 2048,
+// M = 8: 14.2 µs. Tall tiles, 32-row ones or GEMM tiles → here: 4-bit, M = 33, N = 8192 14.9 → 10.5 µs;
+// K = 1968, N = 1088, M = 300 23.8 → 18.8: 170 workgroups, whose CUs issue vector instructions about
+// half of the time (every column block forms the hi + lo pairs of its x·g) and take 14 bytes a
+// clock that miss L1 (the GEMM's tiles 28).
 #include <algorithm>
 #include <functional>
 #include <numeric>
@@ -196,6 +199,8 @@ bool lower_skinny(const sanic_program_desc* d, int si, LoweredStage& out, bool g
     // N = 8192, 4-bit: M = 50 tall 12.6, GEMM 15.1, M = 100 23.5 and 17.7. N = 1088, K = 1968: M = 200
     // 13.6 in 32-row tiles, 18.8 tall, 22.9 GEMM; M = 400 24.6, 18.8, 25.0. N = 4000, K = 1536, M = 100:
     // 17.4 in 32-row tiles, 13.3 tall. 4-bit groups of 32, N = 3264, K = 1408, M = 64: 10.3, GEMM 11.8.
+    // They hold at K = 8192, N = 2048, with the norm (32-row, tall, GEMM): M = 40 26.8 / 31.3 / 35.4, M = 100
+    // 38.9 / 41.5 / 56.6, M = 200 72.8 / 45.5 / 58.7, M = 300 106 / 75.5 / 62.3; the least is taken in each.
     if (M > 32) {
         const double kd = (double)K / 2048.0;
         auto rounds = [](int64_t blocks) { return (double)((blocks + 255) / 256); };
